@@ -346,8 +346,11 @@ void molot_hip_set_merge(int in_launch);
  * itself.  Both give the same bits.  A Q8 cache at d = 256 always takes the
  * pieces (its matrix-core kernel has no per-tile split); without them it
  * runs on the vector-ALU kernel, each query row a sequence of its own (the
- * path of d = 512, of head dims that are not multiples of 8 and of Q8 caches
- * at head dims other than 64, 128 and 256), which agrees to fp32 rounding. */
+ * path of head dims that are not multiples of 8 and of Q8 caches at head dims
+ * other than 64, 128 and 256), which agrees to fp32 rounding.  So do head dims
+ * above 256, which otherwise (every cache type, whatever this switch says)
+ * take fp16 pieces in the same workspace: two of an fp32 row, one of a bf16 or
+ * Q8 row. */
 void molot_hip_set_prefill_presplit(int on);
 
 /* Order in which the waves of a workgroup take their chunk's row blocks.

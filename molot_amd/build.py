@@ -18,6 +18,7 @@ import os
 import shutil
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 PKG = os.path.join(ROOT, "molot_amd")
@@ -54,10 +55,22 @@ def _run(cmd: list[str]) -> None:
     subprocess.run(cmd, check=True)
 
 
+# the library's kernel sources, compiled side by side
+LIB_SOURCES = ("attn_decode.hip", "prefill_wide.hip")
+
+
+def _compile(name: str) -> str:
+    obj = os.path.join(CSRC, "_build", name.replace(".hip", ".o"))
+    _run([_hipcc(), *HIP_FLAGS, "-c", f"-I{INCLUDE}", os.path.join(CSRC, name), "-o", obj])
+    return obj
+
+
 def build_library() -> str:
+    os.makedirs(os.path.join(CSRC, "_build"), exist_ok=True)
+    with ThreadPoolExecutor(len(LIB_SOURCES)) as ex:
+        objs = list(ex.map(_compile, LIB_SOURCES))
     tmp = LIB + ".tmp"
-    _run([_hipcc(), *HIP_FLAGS, "-shared", f"-I{INCLUDE}", os.path.join(CSRC, "attn_decode.hip"),
-          "-o", tmp])
+    _run([_hipcc(), *HIP_FLAGS, "-shared", *objs, "-o", tmp])
     os.replace(tmp, LIB)
     return LIB
 

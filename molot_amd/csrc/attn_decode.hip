@@ -31,313 +31,12 @@
 #include <utility>
 #include <vector>
 
+#include "device_util.hpp"
 #include "molot_amd/attn_hip.h"
+#include "prefill.hpp"
+#include "prefill_wide.hpp"
 
 namespace {
-
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
-
-// ---------------------------------------------------------------------------
-// KV element traits: one 16-byte vector = VW elements.
-template <typename T>
-struct KVT;
-
-template <>
-struct KVT<float> {
-  static constexpr int VW = 4;
-  using vec = f32x4;
-  __device__ static __forceinline__ void unpack(const vec& v, float* x) {
-    x[0] = v[0];
-    x[1] = v[1];
-    x[2] = v[2];
-    x[3] = v[3];
-  }
-};
-
-struct bf16_t {
-  uint16_t bits;
-};
-
-template <>
-struct KVT<bf16_t> {
-  static constexpr int VW = 8;
-  using vec = u32x4;
-  __device__ static __forceinline__ void unpack(const vec& v, float* x) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      x[2 * i] = __uint_as_float(v[i] << 16);
-      x[2 * i + 1] = __uint_as_float(v[i] & 0xFFFF0000u);
-    }
-  }
-};
-
-// Q8 codes (the row scale is applied by the kernel that reads them).
-struct q8_t {
-  int8_t code;
-};
-
-template <>
-struct KVT<q8_t> {
-  static constexpr int VW = 16;
-  using vec = u32x4;
-  __device__ static __forceinline__ void unpack(const vec& v, float* x) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      x[4 * i] = (float)(int8_t)(v[i] & 0xFF);
-      x[4 * i + 1] = (float)(int8_t)((v[i] >> 8) & 0xFF);
-      x[4 * i + 2] = (float)(int8_t)((v[i] >> 16) & 0xFF);
-      x[4 * i + 3] = (float)((int32_t)v[i] >> 24);
-    }
-  }
-};
-
-// K/V rows are read exactly once per step: non-temporal 16-byte loads (the
-// streaming hint measurably raises the sustained HBM read rate on gfx950).
-// Q8 rows excepted: the KV heads of a token share 128-byte lines (head rows
-// of d bytes at t*R + h*d, the token's scales after them), so a line one
-// head's workgroup fetched has to stay in the L2 for its neighbour's.
-template <typename T>
-__device__ __forceinline__ typename KVT<T>::vec load16(const T* p) {
-  if constexpr (std::is_same<T, q8_t>::value)
-    return *reinterpret_cast<const typename KVT<T>::vec*>(p);
-  else
-    return __builtin_nontemporal_load(reinterpret_cast<const typename KVT<T>::vec*>(p));
-}
-
-// A 16-byte vector of row elements [e, e + VW) of a head row of dh
-// elements (dh even, possibly not a multiple of VW), read as VW/2 pieces of
-// two elements (Q8: VW/4 pieces of four codes, dh a multiple of 4).  Pieces
-// at or past dh read the row's first piece instead: they stay inside the
-// row, their K products meet q's zero padding and their V products land in
-// output elements that are never stored.
-template <typename T>
-__device__ __forceinline__ typename KVT<T>::vec load_pad(const T* row, int e, int dh) {
-  using V = typename KVT<T>::vec;
-  constexpr int PB = 2 * (int)sizeof(T);  // bytes per two-element piece
-  V v;
-  const char* r = reinterpret_cast<const char*>(row);
-  if constexpr (std::is_same<T, q8_t>::value) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int ee = e + 4 * i < dh ? e + 4 * i : 0;
-      v[i] = *reinterpret_cast<const uint32_t*>(r + ee);  // plain: heads share lines
-    }
-  } else if constexpr (PB == 8) {
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int ee = e + 2 * i < dh ? e + 2 * i : 0;
-      const f32x2 x = __builtin_nontemporal_load(reinterpret_cast<const f32x2*>(r + ee * 4));
-      v[2 * i] = x[0];
-      v[2 * i + 1] = x[1];
-    }
-  } else {
-    static_assert(PB == 4, "fp32 or bf16 rows");
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int ee = e + 2 * i < dh ? e + 2 * i : 0;
-      v[i] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(r + ee * 2));
-    }
-  }
-  return v;
-}
-
-// Round-to-nearest-even fp32 -> bf16 (include/molot/quant.h:192-198).
-__device__ __forceinline__ uint16_t f32_to_bf16(float f) {
-  uint32_t u = __float_as_uint(f);
-  u += 0x7FFFu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
-}
-
-// ---------------------------------------------------------------------------
-// Q8 rows (the Q8_0 row quantizer of include/molot/quant.h:34-50, applied
-// per KV head row): s = absmax/127 (1 when that is not > 0), codes
-// clamp(nearbyint(x/s), -127, 127); a row dequantizes as code * s.  The
-// divisions are IEEE-correct (hipcc's default for fp32 / ), so the codes and
-// scales are the reference quantizer's bit for bit on the same fp32 input.
-__device__ __forceinline__ float q8_scale(float amax) {
-  const float s = amax / 127.0f;
-  return s > 0.f ? s : 1.0f;
-}
-__device__ __forceinline__ int q8_code(float x, float s) {
-  const int v = (int)__builtin_rintf(x / s);
-  return v > 127 ? 127 : (v < -127 ? -127 : v);
-}
-
-// ---------------------------------------------------------------------------
-// Cross-lane sums.  Lanes are grouped in aligned groups of N; every lane of
-// a group receives the group's sum.  Groups up to 16 use DPP within a row
-// (quad_perm xor1, quad_perm xor2, row_half_mirror, row_mirror: after the
-// quad steps every lane holds its quad's sum, and each mirror pairs a lane
-// with one in the other half of its 8/16-lane block).
-template <int CTRL>
-__device__ __forceinline__ float dpp_f(float x) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, false));
-}
-
-// x of lanes l and l ^ 16 (xor16), or l and l ^ 32 (xor32), as the pair
-// (lower lane's, upper lane's) in every lane: v_permlane16_swap and
-// v_permlane32_swap exchange 16- or 32-lane rows of two registers, so with
-// both operands x they leave the lower row's x in the first and the upper
-// row's in the second, in both rows (checked lane by lane on the GPU).
-// Reducing the pair gives every lane the same operands in the same order,
-// where a shuffle would take two LDS round trips.
-__device__ __forceinline__ float max_xor16(float x) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false,
-                                                  false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float max_xor32(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false,
-                                                  false);
-  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
-}
-__device__ __forceinline__ float sum_xor16(float x) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false,
-                                                  false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-__device__ __forceinline__ float sum_xor32(float x) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false,
-                                                  false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
-// x combined with lane l ^ OFF's x (a sum in the shuffle's operand order)
-template <int OFF>
-__device__ __forceinline__ float sum_xor(float x) {
-  if constexpr (OFF == 16) return sum_xor16(x);
-  else if constexpr (OFF == 32) return sum_xor32(x);
-  else return x + __shfl_xor(x, OFF);
-}
-template <int OFF>
-__device__ __forceinline__ float max_xor(float x) {
-  if constexpr (OFF == 16) return max_xor16(x);
-  else if constexpr (OFF == 32) return max_xor32(x);
-  else return fmaxf(x, __shfl_xor(x, OFF));
-}
-
-template <int N>
-__device__ __forceinline__ float group_max(float v) {
-  if constexpr (N >= 2) v = fmaxf(v, dpp_f<0xB1>(v));
-  if constexpr (N >= 4) v = fmaxf(v, dpp_f<0x4E>(v));
-  if constexpr (N >= 8) v = fmaxf(v, dpp_f<0x141>(v));
-  if constexpr (N >= 16) v = fmaxf(v, dpp_f<0x140>(v));
-  if constexpr (N >= 32) v = max_xor16(v);
-  if constexpr (N >= 64) v = max_xor32(v);
-  return v;
-}
-
-template <int N>
-__device__ __forceinline__ float group_sum(float v) {
-  if constexpr (N >= 2) v += dpp_f<0xB1>(v);   // quad_perm [1,0,3,2]
-  if constexpr (N >= 4) v += dpp_f<0x4E>(v);   // quad_perm [2,3,0,1]
-  if constexpr (N >= 8) v += dpp_f<0x141>(v);  // row_half_mirror
-  if constexpr (N >= 16) v += dpp_f<0x140>(v); // row_mirror
-  if constexpr (N >= 32) v = sum_xor16(v);
-  if constexpr (N >= 64) v = sum_xor32(v);
-  return v;
-}
-
-// Wave-wide max / sum with DPP only (no LDS round trips): the quad and
-// mirror steps reduce each row of 16 lanes, row_bcast:15 and row_bcast:31
-// carry the partial results up to lane 63, which readlane broadcasts.
-template <bool MAX>
-__device__ __forceinline__ float wave_reduce(float v) {
-  auto op = [](float x, float y) { return MAX ? fmaxf(x, y) : x + y; };
-  v = op(v, dpp_f<0xB1>(v));   // quad_perm [1,0,3,2]
-  v = op(v, dpp_f<0x4E>(v));   // quad_perm [2,3,0,1]
-  v = op(v, dpp_f<0x141>(v));  // row_half_mirror
-  v = op(v, dpp_f<0x140>(v));  // row_mirror
-  // row_bcast:15 into rows 1 and 3, row_bcast:31 into rows 2 and 3; rows
-  // outside the mask keep their value (old = v)
-  v = op(v, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(MAX ? -INFINITY : 0.f),
-                                                       __float_as_int(v), 0x142, 0xA, 0xF,
-                                                       false)));
-  v = op(v, __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(MAX ? -INFINITY : 0.f),
-                                                       __float_as_int(v), 0x143, 0xC, 0xF,
-                                                       false)));
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
-}
-
-// exp used by the split-K merges (full-accuracy device expf).
-__device__ __forceinline__ float softmax_exp(float x) { return expf(x); }
-
-// The decode kernels' softmax runs in base 2: a score is q.k * scale*log2(e)
-// (the matrix-core kernel pre-scales q, the vector-ALU kernel each score), so
-// p = 2^(s - m) is one v_exp_f32 (relative error ~|s - m| * 2^-24, within
-// the reference's own exp, exp_avx512_ps at 1.5e-6).  The maxima leave the
-// kernels in natural units (m * ln 2) for the split-K merges.
-constexpr float kLog2e = 1.4426950408889634f;
-constexpr float kLn2 = 0.6931471805599453f;
-__device__ __forceinline__ float exp2_hw(float x) { return __builtin_amdgcn_exp2f(x); }
-// A running max moves only when a score exceeds it by more than kLazyMax
-// (p <= 2^8 otherwise): o and l always share the max they were formed with,
-// so the result is exact either way, and most blocks skip the rescale.
-constexpr float kLazyMax = 8.f;
-
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ uint32_t bf16_pair_exact(float a, float b) {
-  const bf16x2_t p = {(__bf16)a, (__bf16)b};
-  return __builtin_bit_cast(uint32_t, p);
-}
-
-// split3 of two values at once: each piece of the pair is one
-// v_cvt_pk_bf16_f32 (round to nearest even, as split3), element a in the
-// low half.  The same pieces as split3 on each value.
-__device__ __forceinline__ uint32_t bf16_pair(float a, float b) { return bf16_pair_exact(a, b); }
-__device__ __forceinline__ void split3x2(float a, float b, uint32_t& hi, uint32_t& mid,
-                                         uint32_t& lo) {
-  // The residuals are taken of a and b as rounded to fp32: a product that
-  // formed them (a Q8 code times its scale, q times the score scale) must
-  // not fuse into the first subtraction, or the pieces would split the
-  // unrounded product and differ between the kernels that form a and b
-  // differently.
-#pragma clang fp contract(off)
-  hi = bf16_pair(a, b);
-  float ra = a - __uint_as_float(hi << 16), rb = b - __uint_as_float(hi & 0xFFFF0000u);
-  mid = bf16_pair(ra, rb);
-  ra -= __uint_as_float(mid << 16);
-  rb -= __uint_as_float(mid & 0xFFFF0000u);
-  lo = bf16_pair(ra, rb);
-}
-
-// Two fp16 pieces of a row scaled by a power of two: with the row's largest
-// |x| in [2^(ex-1), 2^ex) (frexpf of it), y = x * 2^(14-ex) has |y| < 2^14,
-// hi = fp16(y), lo = fp16(y - hi), each rounded to nearest even.  hi + lo
-// holds y to 2^-22 of |y| while |y| >= 2^-3 (lo a normal fp16), and to
-// 2^-25 absolute below (2^-38 of the row's largest |y|); the scaling is
-// exact.  y's unit is 2^(ex-14) (f16_row_unit), the factor that takes a
-// dot product of such pieces back.  Non-finite values make NaN pieces.
-__device__ __forceinline__ int f16_row_shift(float amax) {
-  int ex = 0;
-  (void)frexpf(amax, &ex);
-  return 14 - ex;
-}
-__device__ __forceinline__ float f16_row_unit(int shift) { return ldexpf(1.f, -shift); }
-__device__ __forceinline__ uint32_t f16_pair(float a, float b) {
-  const _Float16 ha = (_Float16)a, hb = (_Float16)b;
-  return (uint32_t)__builtin_bit_cast(uint16_t, ha) |
-         ((uint32_t)__builtin_bit_cast(uint16_t, hb) << 16);
-}
-__device__ __forceinline__ void split2h(float a, float b, int shift, uint32_t& hi, uint32_t& lo) {
-#pragma clang fp contract(off)
-  const float ya = ldexpf(a, shift), yb = ldexpf(b, shift);
-  hi = f16_pair(ya, yb);
-  const float ra = ya - (float)__builtin_bit_cast(_Float16, (uint16_t)(hi & 0xFFFFu));
-  const float rb = yb - (float)__builtin_bit_cast(_Float16, (uint16_t)(hi >> 16));
-  lo = f16_pair(ra, rb);
-}
-// V rows (the prefill's PV operand): the same split, with the unit kept a
-// normal float (shift <= 120: 2^-120 and up; rows below 2^-106 keep fewer
-// bits, as fp32 denormals would) and 0 for a row of zeros, which then
-// weighs nothing and never sets a tile's largest unit.
-__device__ __forceinline__ int f16_vrow_shift(float amax) { return min(f16_row_shift(amax), 120); }
-__device__ __forceinline__ float f16_vrow_unit(float amax, int shift) {
-  return amax > 0.f ? f16_row_unit(shift) : 0.f;
-}
 
 // ---------------------------------------------------------------------------
 // RoPE + append.
@@ -969,25 +668,6 @@ struct Lds {
   }
 };
 
-
-// Workgroup barrier that orders LDS accesses only.  __syncthreads() also
-// waits for every outstanding global load and store of the thread
-// (s_waitcnt vmcnt(0)), which would stall the prologue on the K/V blocks
-// already in flight.  No global data crosses workgroups inside a launch
-// (the combine is a separate kernel).
-// s_waitcnt vmcnt(N) alone (expcnt and lgkmcnt at their maxima; gfx9
-// encoding: vmcnt bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8).
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-  static_assert(N >= 0 && N < 64, "vmcnt range");
-  __builtin_amdgcn_s_waitcnt((N & 15) | (((N >> 4) & 3) << 14) | (7 << 4) | (15 << 8));
-}
-
-__device__ __forceinline__ void lds_barrier() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
-  __builtin_amdgcn_s_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-}
 
 // RMS norms of the step's fresh vectors (forward.h:554, 562-563):
 // y = (x * 1/sqrt(mean(x^2) + eps)) * w (rmsnorm, include/molot/norm.h:9-28).
@@ -2243,8 +1923,6 @@ __device__ __forceinline__ f32x4 mfma_bf16(bf16x8_t a, bf16x8_t b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
-typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
-
 __device__ __forceinline__ f32x4 mfma_f16(f16x8_t a, f16x8_t b, f32x4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
@@ -2828,30 +2506,6 @@ __global__ __launch_bounds__(kMfmaThreads, 2) void attn_mfma_kernel(AttnArgs a) 
 // normalised before PV; here the hardware base-2 exp of scores pre-scaled by
 // log2(e), fp32 running sums with a lazy max rescale, and one division at
 // the end (fp32 rounding differences).
-struct PfArgs {
-  const float* q;  // [M][nq][D]
-  const void* k;   // token-major cache [N][nkv*D], or pages [block][nkv][page][D]
-  const void* v;
-  float* o;        // [M][nq][D]
-  const int32_t* block_table;  // paged: the sequence's row of block ids
-  int nq, nkv, M, N, pos0, window, nqb;  // nqb: blocks of 16 * (waves) query rows per KV head
-  int dh;  // head dim as stored (< D: the launch runs padded to D, through the pieces)
-  int page_shift;
-  float scale;
-  // the attended keys [T0, T0 + R) of every KV head split into 16-bit pieces
-  // once for the launch (pf_split_kernel): [K, V][nkv][3 pieces][R][D]; NULL:
-  // the kernel splits each staged tile itself
-  const uint16_t* pieces;
-  int T0, R;
-  int Rsplit;  // pf_split_kernel splits rows [T0, T0 + Rsplit); the appending step wrote the rest
-  // split-K over the key tiles (nsplit > 1): split s of a query block takes
-  // its share of the tiles and writes unnormalised o and (max, sum) per query
-  // row, slot m*nq + head, to part_o [slot][nsplit][D] and part_ml
-  // [slot][nsplit][2]; combine_kernel merges them into O
-  int nsplit;
-  float* part_o;
-  float* part_ml;
-};
 
 // Cache offset (elements of T; Q8: bytes) of row t of KV head h, and for Q8
 // the byte offset of its scale (soff).  Token-major: [N][nkv*D] (Q8 rows of
@@ -2934,31 +2588,6 @@ __global__ __launch_bounds__(256) void pf_split_kernel(PfArgs a, uint16_t* out) 
 #pragma unroll
   for (int p = 0; p < 2; ++p)
     *reinterpret_cast<u32x4*>(row(p) + 8 * j) = u32x4{pc[p][0], pc[p][1], pc[p][2], pc[p][3]};
-}
-
-// One 16-byte global -> LDS copy per lane (global_load_lds_dwordx4, scalar
-// base + lane offset): lane l's 16 bytes land at LDS address lds + 16*l.
-// Written as inline assembly, so the compiler does not see an LDS store in
-// flight: with the builtin it put an s_waitcnt vmcnt(0) before the next LDS
-// reads it could not tell apart from the copy's destination (the transposed
-// V reads of the other tile buffer), which waited for the next tile's copies
-// halfway through every tile.  The kernel orders the copies itself
-// (wait_vmcnt, then a barrier, before a buffer is read).  m0 takes the LDS
-// address as an input operand (the compiler writes it); one wait state
-// between that write and the copy.
-__device__ __forceinline__ void dma16(const void* base, uint32_t off, uint32_t lds) {
-  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
-               :
-               : "v"(off), "s"(base), "{m0}"(lds)
-               : "memory");
-}
-// The same with 4 bytes a lane (global_load_lds_dword): lane l's 4 bytes
-// land at LDS address lds + 4*l.
-__device__ __forceinline__ void dma4(const void* base, uint32_t off, uint32_t lds) {
-  asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1"
-               :
-               : "v"(off), "s"(base), "{m0}"(lds)
-               : "memory");
 }
 
 // Waves per prefill workgroup (16 query rows each): 8, so that 128 rows
@@ -4611,7 +4240,6 @@ struct Norms {
 
 bool norms_ok(const Norms& nm) { return nm.eps >= 0.f && nm.eps < INFINITY; }
 
-using PfFn = void (*)(PfArgs);
 std::atomic<int> g_presplit{1};  // molot_hip_set_prefill_presplit
 
 template <int D, typename T, bool PAGED>
@@ -4638,7 +4266,6 @@ PfFn pf_kernel_pre(int d, int pw) {
                  : prefill_mfma16_kernel<256, float, false, 4, true>;
 }
 
-using SplitFn = void (*)(PfArgs, uint16_t*);
 SplitFn pf_split(int d, int kv_dtype, bool paged) {
   if (kv_dtype == MOLOT_KV_Q8) {
     if (d == 64) return paged ? pf_split_kernel<64, q8_t, true> : pf_split_kernel<64, q8_t, false>;
@@ -5171,9 +4798,9 @@ static int prefill_pieces(int nkv, int N, int d, int pos0, int window, int kv_dt
   return 0;
 }
 
-// The prefill at a head dim the matrix-core prefill cannot tile (d = 512:
-// its three q pieces alone would take 192 registers a lane and a 32-key tile
-// of K and V pieces 192 KB of LDS; an even d that is not a multiple of 8):
+// The prefill at a head dim the matrix-core prefill does not tile (an even d
+// that is not a multiple of 8; a padded Q8 cache), and above 256 where the
+// prompt is too small for prefill_wide or its workspace cannot be had:
 // the vector-ALU decode kernel with each query row as a sequence of its own
 // (AttnArgs::pf) over the one cache, contiguous or through the prompt's
 // block-table row.  Each query row streams its attended rows; neighbouring
@@ -5210,6 +4837,170 @@ static int prefill_rows(const float* Qm, const void* K, const void* V, float* Om
                    : run_attn<false, false>(a, d, kv_dtype, span, M, stream);
 }
 
+// Launches a prefill attention kernel of `wgs` workgroups and, where its key
+// tiles are split, the merge of the splits' partials after it.
+static int launch_prefill(PfFn pk, int64_t wgs, int threads, const PfArgs& a, int D,
+                          void* stream) {
+  const dim3 grid((unsigned)wgs);
+  const int nsplit = a.nsplit;
+  int st = 0;
+  CombArgs cb{};  // split-K: (token, q head) rows as slots of one head each
+  cb.part_o = a.part_o;
+  cb.part_ml = a.part_ml;
+  cb.o = a.o;
+  cb.nq = a.nq;
+  cb.nkv = a.nq;
+  cb.gh = 1;
+  cb.nsub = 1;
+  cb.d = D;
+  cb.dh = a.dh;
+  cb.nchunks = nsplit;
+  cb.chunk = 1;
+  cb.pairs = comb_pairs(nsplit);
+  // at most 8 splits: the row merge, one wave per 64V outputs of a slot
+  // (2048 tokens x 8 q heads at d = 256 over 2 splits: 9.2 us, against 22.2
+  // with a wave per 64 outputs and 82 us on combine_kernel's 4 workgroups a
+  // slot); more splits: combine_kernel
+  const bool cwave = nsplit <= 8;
+  const int cv = D % 256 == 0 ? 4 : (D % 128 == 0 ? 2 : 1);
+  const int64_t cunits = (int64_t)a.M * a.nq * (D / (64 * cv));
+  using RowsFn = void (*)(CombArgs, int64_t);
+  const RowsFn rk = nsplit <= 4 ? (cv == 4 ? combine_rows_kernel<4, 4>
+                                  : cv == 2 ? combine_rows_kernel<4, 2> : combine_rows_kernel<4, 1>)
+                                : (cv == 4 ? combine_rows_kernel<8, 4>
+                                  : cv == 2 ? combine_rows_kernel<8, 2> : combine_rows_kernel<8, 1>);
+  const dim3 cgrid = cwave ? dim3((unsigned)((cunits + 3) / 4))
+                           : dim3((unsigned)((int64_t)a.M * a.nq), (unsigned)(D / cb.pairs));
+  const dim3 cblock = cwave ? dim3((unsigned)kCombWaveThreads) : dim3(kCombThreads);
+  const size_t clds = cwave ? 0 : sizeof(float) * (size_t)comb_lds_floats(nsplit);
+  std::lock_guard<std::mutex> plk(g_prof_mu);
+  if (prof_active(stream)) {
+    ProfRec pr{prof_event(), prof_event(), nullptr, nullptr, nsplit > 1};
+    hipExtLaunchKernelGGL(pk, grid, dim3(threads), 0, (hipStream_t)stream, pr.a0, pr.a1, 0, a);
+    st = (int)hipGetLastError();
+    if (!st && nsplit > 1) {
+      pr.c0 = prof_event();
+      pr.c1 = prof_event();
+      if (cwave)
+        hipExtLaunchKernelGGL(rk, cgrid, cblock, 0, (hipStream_t)stream, pr.c0, pr.c1, 0, cb,
+                              cunits);
+      else
+        hipExtLaunchKernelGGL(combine_kernel, cgrid, cblock, clds, (hipStream_t)stream, pr.c0,
+                              pr.c1, 0, cb);
+      st = (int)hipGetLastError();
+    }
+    g_prof.push_back(pr);
+    return st;
+  }
+  hipLaunchKernelGGL(pk, grid, dim3(threads), 0, (hipStream_t)stream, a);
+  st = (int)hipGetLastError();
+  if (st || nsplit == 1) return st;
+  if (cwave)
+    hipLaunchKernelGGL(rk, cgrid, cblock, 0, (hipStream_t)stream, cb, cunits);
+  else
+    hipLaunchKernelGGL(combine_kernel, cgrid, cblock, clds, (hipStream_t)stream, cb);
+  return (int)hipGetLastError();
+}
+
+// Key splits of a prefill_wide_kernel launch of nqb * nkv query blocks (one
+// workgroup a CU): the count with the least estimated time.  A split's cost
+// is its tiles' plus its start and end; the launch's the longest split's, or
+// the CUs' share of all of them with half of the shortest for the uneven last
+// round; and more than one split pays the merge of their partials.
+static int wide_splits(int64_t nqb, int nkv, int M, int N, int G, int qb, int D, int pos0,
+                       int window, int nq) {
+  auto tiles_of = [&](int64_t b) {  // query block b's tiles (32 keys)
+    const int64_t m0 = b * qb / G, m1 = std::min<int64_t>(((b + 1) * qb - 1) / G, M - 1);
+    const int64_t lo = window > 0 ? std::max<int64_t>(0, pos0 + m0 - window + 1) : 0;
+    const int64_t hi = std::min<int64_t>(pos0 + m1 + 1, N);
+    return hi > lo ? (double)((hi - lo + kWideTile - 1) / kWideTile) : 0.0;
+  };
+  const double first = tiles_of(0), last = tiles_of(nqb - 1), mid = tiles_of(nqb / 2);
+  const double longest = std::max({first, mid, last}), shortest = std::min({first, mid, last});
+  const double total = (first + 4 * mid + last) / 6 * (double)(nqb * nkv);
+  const double kStart = 3.0;                 // a split's start and end, in tiles
+  const double kTileUs = 1.8 * D / 512;
+  const int cus = num_cus();
+  double best = 0;
+  int ns_best = 1;
+  for (int ns = 1; ns <= 64 && ns <= std::max(1.0, longest / 4); ++ns) {
+    const double wgs = (double)(nqb * nkv) * ns;
+    double est = longest / ns + kStart;
+    if (wgs > cus)
+      est = std::max(est, (total + wgs * kStart) / cus + 0.5 * (shortest / ns + kStart));
+    est *= kTileUs;
+    if (ns > 1) est += 4.0 + 8.0 * M * nq * (double)D * ns / 4e6;
+    if (ns == 1 || est < best) {
+      best = est;
+      ns_best = ns;
+    }
+  }
+  return ns_best;
+}
+
+// The prefill at head dims above 256 on the matrix cores
+// (prefill_wide_kernel, padded to D = 512): the attended keys' pieces first,
+// then the attention over them.  MOLOT_ENOWS: a capture that would have to
+// grow the workspace, or keys past its cap (the caller takes prefill_rows).
+static int prefill_wide(const float* Qm, const void* K, const void* V, float* Om, int nq, int nkv,
+                        int M, int N, int d, float scale, int pos0, int window, int kv_dtype,
+                        const int32_t* block_row, int page, void* stream) {
+  const int D = 512, np = wide_pieces(kv_dtype == MOLOT_KV_F32), qb = wide_rows(D);
+  PfArgs a{};
+  a.q = Qm;
+  a.k = K;
+  a.v = V;
+  a.o = Om;
+  a.nq = nq;
+  a.nkv = nkv;
+  a.M = M;
+  a.N = N;
+  a.dh = d;
+  a.pos0 = pos0;
+  a.window = window;
+  a.scale = scale;
+  if (block_row) {
+    if (page <= 0 || (page & (page - 1)) || !q8_pages_ok(nkv, page, kv_dtype))
+      return MOLOT_EINVAL;
+    a.block_table = block_row;
+    while ((1 << a.page_shift) < page) ++a.page_shift;
+  }
+  a.T0 = window > 0 && pos0 - window + 1 > 0 ? std::min(pos0 - window + 1, N) : 0;
+  a.R = N - a.T0;
+  if (a.R == 0) return zero_out(Om, (int64_t)M * nq * d, (hipStream_t)stream);  // no key attended
+  const size_t need = wide_bytes(nkv, D, np, a.R);
+  if (need > kMaxPiecesBytes) return MOLOT_ENOWS;
+  void* pieces = nullptr;
+  int st = pieces_workspace(stream, need, &pieces);
+  if (st) return st;
+  a.pieces = reinterpret_cast<const uint16_t*>(pieces);
+  const int G = nq / nkv;
+  const int64_t nqb = ((int64_t)M * G + qb - 1) / qb;
+  a.nqb = (int)nqb;
+  a.nsplit = wide_splits(nqb, nkv, M, N, G, qb, D, pos0, window, nq);
+  if (a.nsplit > 1) {
+    unsigned long long* ctr = nullptr;
+    void* ws = nullptr;
+    st = workspace(stream, sizeof(float) * (size_t)M * nq * a.nsplit * (D + 2), &ctr, &ws);
+    if (st && st != MOLOT_ENOWS) return st;
+    if (st) {
+      a.nsplit = 1;  // under capture the workspace cannot grow
+    } else {
+      a.part_o = reinterpret_cast<float*>(ws);
+      a.part_ml = a.part_o + (size_t)M * nq * a.nsplit * D;
+    }
+  }
+  if (nqb * nkv * a.nsplit > (int64_t)0x7FFFFFFF) return MOLOT_ENOTSUP;
+  const int64_t units = wide_padded_rows(a.R) * (D / 8);
+  hipLaunchKernelGGL(prefill_wide_split(D, kv_dtype, block_row != nullptr),
+                     dim3((unsigned)((units + 255) / 256), nkv, 2), dim3(256), 0,
+                     (hipStream_t)stream, a, reinterpret_cast<uint16_t*>(pieces));
+  st = (int)hipGetLastError();
+  if (st) return st;
+  return launch_prefill(prefill_wide_fn(D, kv_dtype), nqb * nkv * a.nsplit, 64 * kWideWaves, a, D,
+                        stream);
+}
+
 // split_rows: rows of [T0, N) pf_split_kernel still has to split (the
 // appending step wrote the pieces of the others; -1: all of them)
 static int attn_prefill_impl(const float* Qm, const void* K, const void* V, float* Om, int nq,
@@ -5225,7 +5016,8 @@ static int attn_prefill_impl(const float* Qm, const void* K, const void* V, floa
   // at d.  A Q8 cache at d = 256 runs only through the pieces (the kernel
   // that splits staged Q8 tiles itself is built for 64 and 128).  Head dims
   // above 256 and even ones that are not multiples of 8 run as prefill rows
-  // (prefill_rows).
+  // (prefill_rows), those above 256 on the matrix cores (prefill_wide) where
+  // there is enough work.
   const bool padded = !supported_d(d);
   // Q8 caches at padded dims too (the matrix-core prefill reads whole
   // 16-code chunks of the built dims only)
@@ -5237,6 +5029,19 @@ static int attn_prefill_impl(const float* Qm, const void* K, const void* V, floa
   if (N == 0) return zero_out(Om, (int64_t)M * nq * d, (hipStream_t)stream);
   if (!K || !V || !aligned16(K) || !aligned16(V) || !aligned16(Qm) || !aligned16(Om))
     return MOLOT_EINVAL;
+  // Above 256 on the matrix cores from kWideWork (query head, key) pairs on.
+  // Both sides, 8q/2kv/d512, us a step over fp32 / bf16 / Q8 caches:
+  // (rows, cached) = (64, 500) prefill rows 40 / 40 / 37, matrix cores 44 /
+  // 38 / 38; (8, 4000) 43 / 38 / 37 against 47 / 38 / 41; (24, 4000) 123 /
+  // 117 / 96 against 53 / 44 / 46; (8, 16384) 118 / 94 / 77 against 92 / 64
+  // / 61; (2, 16384) 63 / 41 / 36 against 89 / 60 / 58.
+  constexpr int64_t kWideWork = 400000;
+  const int64_t span = window > 0 && window < N ? window : N;
+  if (d > 256 && M <= 65535 && (int64_t)M * nq * span >= kWideWork) {
+    st = prefill_wide(Qm, K, V, Om, nq, nkv, M, N, d, scale, pos0, window, kv_dtype, block_row,
+                      page, stream);
+    if (st != MOLOT_ENOWS) return st;
+  }
   if (rows_path)
     return prefill_rows(Qm, K, V, Om, nq, nkv, M, N, d, scale, pos0, window, kv_dtype, block_row,
                         page, stream);
@@ -5331,63 +5136,7 @@ static int attn_prefill_impl(const float* Qm, const void* K, const void* V, floa
       pk = pf_kernel_pre(D, pw);
     }
   }
-  const dim3 grid((unsigned)(nqb * nkv * nsplit));
-  CombArgs cb{};  // split-K: (token, q head) rows as slots of one head each
-  cb.part_o = a.part_o;
-  cb.part_ml = a.part_ml;
-  cb.o = Om;
-  cb.nq = nq;
-  cb.nkv = nq;
-  cb.gh = 1;
-  cb.nsub = 1;
-  cb.d = D;
-  cb.dh = d;
-  cb.nchunks = nsplit;
-  cb.chunk = 1;
-  cb.pairs = comb_pairs(nsplit);
-  // at most 8 splits: the row merge, one wave per 64V outputs of a slot
-  // (2048 tokens x 8 q heads at d = 256 over 2 splits: 9.2 us, against 22.2
-  // with a wave per 64 outputs and 82 us on combine_kernel's 4 workgroups a
-  // slot); more splits: combine_kernel
-  const bool cwave = nsplit <= 8;
-  const int cv = D % 256 == 0 ? 4 : (D % 128 == 0 ? 2 : 1);
-  const int64_t cunits = (int64_t)M * nq * (D / (64 * cv));
-  using RowsFn = void (*)(CombArgs, int64_t);
-  const RowsFn rk = nsplit <= 4 ? (cv == 4 ? combine_rows_kernel<4, 4>
-                                  : cv == 2 ? combine_rows_kernel<4, 2> : combine_rows_kernel<4, 1>)
-                                : (cv == 4 ? combine_rows_kernel<8, 4>
-                                  : cv == 2 ? combine_rows_kernel<8, 2> : combine_rows_kernel<8, 1>);
-  const dim3 cgrid = cwave ? dim3((unsigned)((cunits + 3) / 4))
-                           : dim3((unsigned)((int64_t)M * nq), (unsigned)(D / cb.pairs));
-  const dim3 cblock = cwave ? dim3((unsigned)kCombWaveThreads) : dim3(kCombThreads);
-  const size_t clds = cwave ? 0 : sizeof(float) * (size_t)comb_lds_floats(nsplit);
-  std::lock_guard<std::mutex> plk(g_prof_mu);
-  if (prof_active(stream)) {
-    ProfRec pr{prof_event(), prof_event(), nullptr, nullptr, nsplit > 1};
-    hipExtLaunchKernelGGL(pk, grid, dim3(pf_threads), 0, (hipStream_t)stream, pr.a0, pr.a1, 0, a);
-    st = (int)hipGetLastError();
-    if (!st && nsplit > 1) {
-      pr.c0 = prof_event();
-      pr.c1 = prof_event();
-      if (cwave)
-        hipExtLaunchKernelGGL(rk, cgrid, cblock, 0, (hipStream_t)stream, pr.c0, pr.c1, 0, cb,
-                              cunits);
-      else
-        hipExtLaunchKernelGGL(combine_kernel, cgrid, cblock, clds, (hipStream_t)stream, pr.c0,
-                              pr.c1, 0, cb);
-      st = (int)hipGetLastError();
-    }
-    g_prof.push_back(pr);
-    return st;
-  }
-  hipLaunchKernelGGL(pk, grid, dim3(pf_threads), 0, (hipStream_t)stream, a);
-  st = (int)hipGetLastError();
-  if (st || nsplit == 1) return st;
-  if (cwave)
-    hipLaunchKernelGGL(rk, cgrid, cblock, 0, (hipStream_t)stream, cb, cunits);
-  else
-    hipLaunchKernelGGL(combine_kernel, cgrid, cblock, clds, (hipStream_t)stream, cb);
-  return (int)hipGetLastError();
+  return launch_prefill(pk, nqb * nkv * nsplit, pf_threads, a, D, stream);
 }
 
 int molot_hip_attn_prefill_gqa(const float* Qm, const void* K, const void* V, float* Om, int nq,

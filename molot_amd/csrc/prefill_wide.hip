@@ -1,0 +1,653 @@
+// Causal prefill attention (include/molot/gemm.h:409-446) for wide head dims
+// on the matrix cores: 32 query rows a wave, the head dim sliced over waves.
+//
+// Query rows of one KV head are r = m*G + g (token m at pos0 + m, q head g of
+// the group), as in prefill_mfma16_kernel.  A workgroup of 8 waves owns
+// 32 * RG of them: wave (rg, sl) takes row group rg and the SL = 128
+// elements sl*128 .. of the head dim, for the scores and for the output.
+//   D = 512: 2 row groups x 4 slices, 64 rows;
+//   D = 256: 4 row groups x 2 slices, 128 rows.
+// Per tile of 32 keys:
+//   1. every wave forms its slice's share of S^T = K . Q^T on
+//      v_mfma_f32_32x32x16_f16 (A = K from LDS, B = its q pieces in
+//      registers) and leaves it in LDS;
+//   2. wave sl owns 32/NSL of the row group's rows: it adds the slices'
+//      shares, runs the online softmax over whole rows (lanes of a row side
+//      by side, DPP reductions) and leaves P's pieces in LDS, and the factor
+//      the rows' o must take when the running max or P's unit moved;
+//   3. every wave adds its slice of O^T += V^T . P^T (A = V^T by transposed
+//      LDS reads).
+// Why this split: a wave's registers hold 32 rows x 128 elements of q pieces
+// (64) and of o (64), so two waves a SIMD fit at every D, and each staged K
+// or V operand of 1 KB serves 32 rows: 16 rows a wave (prefill_mfma16_kernel)
+// would ask 170 bytes a cycle of an LDS that reads 128 at the full matrix
+// rate, 32 rows ask 85.
+//
+// Products: q and p enter as two fp16 pieces of a row scaled by a power of
+// two (split2h), K and V as NP such pieces: NP = 2 for fp32 values (three
+// products a term, 2^-22 of it dropped), NP = 1 for bf16 and Q8 rows, whose
+// values (8 bits; codes of 7) one piece holds exactly down to 2^-28 of the
+// row's largest (two products).  A Q8 row's fp32 scale goes into its unit.
+//
+// What bounds it (D = 512, fp32, 8q/2kv, a fresh 1999-token prompt; cycles a
+// tile, stamped): the three phases' latencies, 7400 against the 3072 its 192
+// products of 32 cycles a SIMD take.  Scores 3000 and PV 2300 (each 1536 of
+// products, then the barrier, the first LDS reads and the stores of the
+// shares), the softmax with the next K copies 1950.  The copies go out between
+// products and softmax steps: in a row they held each wave ~500 cycles.
+// The step: 1468 us with each query row streamed by the vector-ALU kernel
+// (prefill_rows), 230 us here, of which this kernel ~140.
+#include <hip/hip_runtime.h>
+
+#include "device_util.hpp"
+#include "molot_amd/attn_hip.h"
+#include "prefill.hpp"
+#include "prefill_wide.hpp"
+
+namespace {
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));  // dword-aligned
+typedef short i16x4_t __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ f32x16 mfma32_f16(f16x8_t a, f16x8_t b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+
+// Swizzles of the staged rows (16-byte units; unit ch of row r at ch ^ f(r)).
+// K: a 16-byte read takes one unit of 16 consecutive rows.  V: a transposed
+// read takes 64 bytes of 4 consecutive rows.  Both then cover 256 bytes.
+__device__ __forceinline__ int wk_f(int r) { return r & 15; }
+__device__ __forceinline__ int wv_f(int r) { return (r & 3) << 2; }
+
+// Offset (elements; Q8 bytes) of row t of KV head h in a cache of head dim
+// a.dh, and of a Q8 row's scale.
+template <typename T, bool PAGED>
+__device__ __forceinline__ int64_t wide_row_off(const PfArgs& a, int h, int t, int64_t& soff) {
+  constexpr bool Q8 = std::is_same<T, q8_t>::value;
+  const int dh = a.dh;
+  if constexpr (PAGED) {
+    const int pg = 1 << a.page_shift;
+    const int64_t blk = a.block_table[t >> a.page_shift];
+    const int sl = t & (pg - 1);
+    if constexpr (Q8) {
+      const int64_t bb = (int64_t)a.nkv * pg * (dh + 4);
+      soff = blk * bb + (int64_t)a.nkv * pg * dh + 4 * ((int64_t)h * pg + sl);
+      return blk * bb + ((int64_t)h * pg + sl) * dh;
+    }
+    return ((blk * a.nkv + h) * pg + sl) * (int64_t)dh;
+  } else {
+    if constexpr (Q8) {
+      const int64_t rb = (int64_t)a.nkv * dh + ((4 * a.nkv + 15) & ~15);
+      soff = (int64_t)t * rb + (int64_t)a.nkv * dh + 4 * h;
+      return (int64_t)t * rb + (int64_t)h * dh;
+    }
+    return ((int64_t)t * a.nkv + h) * (int64_t)dh;
+  }
+}
+
+// The attended keys [T0, T0 + R) of every KV head as fp16 pieces, in the
+// layout of prefill_wide.hpp; the kWideTail rows after them are zeros, so
+// that the last tile reads finite values.  Thread: 8 elements of a row, a
+// row's D/8 units in consecutive lanes; grid (units / 256, nkv, K or V).
+template <int D, typename T, bool PAGED>
+__global__ __launch_bounds__(256) void wide_split_kernel(PfArgs a, uint16_t* out) {
+  constexpr bool Q8 = std::is_same<T, q8_t>::value;
+  constexpr int NP = wide_pieces_v<T>;
+  constexpr int UPR = D / 8;
+  const int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t Rp = wide_padded_rows(a.R);
+  if (u >= Rp * UPR) return;
+  const int h = blockIdx.y, kv = blockIdx.z;
+  const int64_t r = u / UPR;
+  const int j = (int)(u - r * UPR);
+  float x[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) x[e] = 0.f;
+  float s = 1.f;
+  if (r < a.R) {
+    int64_t soff = 0;
+    const int64_t off = wide_row_off<T, PAGED>(a, h, a.T0 + (int)r, soff);
+    const char* base = reinterpret_cast<const char*>(kv ? a.v : a.k);
+    const int e0 = 8 * j, n = min(8, a.dh - e0);  // elements of the row in this unit
+    if constexpr (Q8) {  // dh a multiple of 4: whole 4-code words
+      s = *reinterpret_cast<const float*>(base + soff);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        if (4 * i < n) {
+          const uint32_t c = *reinterpret_cast<const uint32_t*>(base + off + e0 + 4 * i);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[4 * i + e] = (float)(int8_t)((c >> (8 * e)) & 0xFF);
+        }
+      }
+    } else if constexpr (sizeof(T) == 2) {
+      const uint16_t* p = reinterpret_cast<const uint16_t*>(base) + off + e0;
+      if (n == 8 && (a.dh & 7) == 0) {
+        const u32x4 v = *reinterpret_cast<const u32x4*>(p);
+        KVT<bf16_t>::unpack(v, x);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (2 * i < n) {
+            const uint32_t v = *reinterpret_cast<const uint32_t*>(p + 2 * i);
+            x[2 * i] = __uint_as_float(v << 16);
+            x[2 * i + 1] = __uint_as_float(v & 0xFFFF0000u);
+          }
+      }
+    } else {
+      const float* p = reinterpret_cast<const float*>(base) + off + e0;
+      if (n == 8 && (a.dh & 3) == 0) {
+        const f32x4 x0 = *reinterpret_cast<const f32x4*>(p);
+        const f32x4 x1 = *reinterpret_cast<const f32x4*>(p + 4);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          x[e] = x0[e];
+          x[4 + e] = x1[e];
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (2 * i < n) {
+            const f32x2 v = *reinterpret_cast<const f32x2*>(p + 2 * i);
+            x[2 * i] = v[0];
+            x[2 * i + 1] = v[1];
+          }
+      }
+    }
+  }
+  float xm = 0.f;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) xm = fmaxf(xm, fabsf(x[e]));
+  xm = group_max<UPR>(xm);
+  const int shift = kv ? f16_vrow_shift(xm) : f16_row_shift(xm);
+  uint32_t pc[2][4];
+#pragma unroll
+  for (int e = 0; e < 8; e += 2) split2h(x[e], x[e + 1], shift, pc[0][e / 2], pc[1][e / 2]);
+  uint16_t* head = out + ((int64_t)kv * a.nkv + h) * wide_head_elems(D, NP, Rp);
+#pragma unroll
+  for (int p = 0; p < NP; ++p)
+    *reinterpret_cast<u32x4*>(head + (p * Rp + r) * D + 8 * j) =
+        u32x4{pc[p][0], pc[p][1], pc[p][2], pc[p][3]};
+  if (j == 0)
+    reinterpret_cast<float*>(head + NP * Rp * D)[r] =
+        (kv ? f16_vrow_unit(xm, shift) : f16_row_unit(shift)) * s;
+}
+
+template <int D, int NP>
+__global__ __launch_bounds__(512) void prefill_wide_kernel(PfArgs a) {
+  constexpr int KT = kWideTile;
+  constexpr int NSL = D / 128;       // slices of the head dim
+  constexpr int RG = 8 / NSL;        // row groups of 32
+  constexpr int QB = 32 * RG;        // query rows a workgroup
+  constexpr int RPO = 32 / NSL;      // rows of its group a wave owns in the softmax
+  constexpr int LPR = 64 / RPO;      // lanes of an owned row
+  constexpr int KPL = KT / LPR;      // keys a lane of it holds (4 or 8)
+  constexpr int RB = 2 * D;          // bytes of a staged row of one piece
+  constexpr int TB = NP * KT * RB;   // bytes of a staged tile (K or V)
+  constexpr int SXB = 8 * 4096;      // score shares, then P (8 owner regions)
+  constexpr bool DB = 4 * TB + SXB <= 160 * 1024;  // two buffers of K and of V
+  constexpr int NB = DB ? 2 : 1;
+  constexpr int NL = TB / 1024 / 8;  // 1 KB copies a wave issues per K or V tile
+  static_assert(KPL == 4 || KPL == 8, "4 or 8 keys a lane");
+  static_assert(2 * NB * TB + SXB <= 160 * 1024, "LDS");
+  __shared__ __attribute__((aligned(16))) char kbuf[NB][TB];
+  __shared__ __attribute__((aligned(16))) char vbuf[NB][TB];
+  __shared__ __attribute__((aligned(16))) char sx[SXB];
+
+  const int G = a.nq / a.nkv;
+  const int h = blockIdx.x % a.nkv;
+  const int rest = (int)(blockIdx.x / a.nkv);
+  const int sp = rest % a.nsplit;              // key split
+  const int qb = a.nqb - 1 - rest / a.nsplit;  // latest rows (most keys) first
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rg = w / NSL, sl = w % NSL;
+  const int c32 = lane & 31, hh = lane >> 5;
+  const int rows = a.M * G;
+  const int r0 = qb * QB;
+  const int rl = min(r0 + QB, rows) - 1;
+  auto t0_of = [&](int m) {
+    const int pos = a.pos0 + m;
+    int t0 = (a.window > 0 && pos - a.window + 1 > 0) ? pos - a.window + 1 : 0;
+    return t0 > a.N ? a.N : t0;
+  };
+  auto nn_of = [&](int m) { return a.pos0 + m + 1 < a.N ? a.pos0 + m + 1 : a.N; };
+  const int kt_lo = t0_of(r0 / G);
+  const int kt_hi = nn_of(rl / G);
+  const int ntile_all = kt_hi > kt_lo ? (kt_hi - kt_lo + KT - 1) / KT : 0;
+  const int tb0 = (int)((int64_t)sp * ntile_all / a.nsplit);
+  const int ntile = (int)((int64_t)(sp + 1) * ntile_all / a.nsplit) - tb0;
+  const int kt_s = kt_lo + tb0 * KT;
+
+  const int64_t Rp = wide_padded_rows(a.R);
+  const uint16_t* khead = a.pieces + (int64_t)h * wide_head_elems(D, NP, Rp);
+  const uint16_t* vhead = khead + (int64_t)a.nkv * wide_head_elems(D, NP, Rp);
+
+  // K or V of the tile at key tk into LDS: 1 KB blocks of 1024/RB rows, wave
+  // w blocks w, w + 8, ...; lane l's 16 bytes land at block + 16*l, so it
+  // loads the unit the swizzle keeps there
+  auto copy1 = [&](int t, int tk, char* buf, const uint16_t* head, bool isv) {
+    constexpr int UPR = D / 8, RPB = 64 / UPR, BPP = KT / RPB;
+    const int r_in = lane / UPR, jpos = lane % UPR;
+    const int bi = w + 8 * t;  // wave-uniform
+    const int pc = bi / BPP, rb = (bi % BPP) * RPB;
+    const int ch = jpos ^ (isv ? wv_f(rb + r_in) : wk_f(rb + r_in));
+    dma16(head + (pc * Rp + (tk - a.T0) + rb) * D, (uint32_t)(r_in * RB + 16 * ch),
+          (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)(buf + bi * 1024));
+  };
+  auto stage = [&](int tk, char* buf, const uint16_t* head, bool isv) {
+#pragma unroll
+    for (int t = 0; t < NL; ++t) copy1(t, tk, buf, head, isv);
+  };
+
+  if (ntile > 0) {
+    stage(kt_s, kbuf[0], khead, false);
+    if constexpr (DB) stage(kt_s, vbuf[0], vhead, true);
+  }
+
+  // q pieces of this wave's rows and slice (B operand: lane l row c32,
+  // elements 16s + 8*hh .. +7 of the slice), scaled by scale*log2(e) and,
+  // with the row's largest |q| over all slices, by a power of two
+  f16x8_t qh[8], ql[8];
+  {
+    const int row = r0 + 32 * rg + c32;
+    const bool rv = row < rows;
+    const int m = rv ? row / G : 0, g = rv ? row - m * G : 0;
+    const float* qr = a.q + ((int64_t)m * a.nq + h * G + g) * a.dh;
+    const float qsc = a.scale * kLog2e;
+    float x[8][8];
+    const bool v4 = (a.dh & 3) == 0;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const int e0 = 128 * sl + 16 * s + 8 * hh;
+      if (v4) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          f32x4 y = {0.f, 0.f, 0.f, 0.f};
+          if (rv && e0 + 4 * i < a.dh) y = *reinterpret_cast<const f32x4*>(qr + e0 + 4 * i);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) x[s][4 * i + e] = y[e] * qsc;
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          f32x2 y = {0.f, 0.f};
+          if (rv && e0 + 2 * i < a.dh) y = *reinterpret_cast<const f32x2*>(qr + e0 + 2 * i);
+          x[s][2 * i] = y[0] * qsc;
+          x[s][2 * i + 1] = y[1] * qsc;
+        }
+      }
+    }
+    float qm = 0.f;
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) qm = fmaxf(qm, fabsf(x[s][e]));
+    qm = max_xor32(qm);
+    float* qmx = reinterpret_cast<float*>(sx);  // [rg][slice][32 rows]
+    if (hh == 0) qmx[(rg * NSL + sl) * 32 + c32] = qm;
+    lds_barrier();
+#pragma unroll
+    for (int s = 0; s < NSL; ++s) qm = fmaxf(qm, qmx[(rg * NSL + s) * 32 + c32]);
+    const int qshift = f16_row_shift(qm);
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      uint32_t h4[4], l4[4];
+#pragma unroll
+      for (int e = 0; e < 8; e += 2) split2h(x[s][e], x[s][e + 1], qshift, h4[e / 2], l4[e / 2]);
+      qh[s] = __builtin_bit_cast(f16x8_t, u32x4{h4[0], h4[1], h4[2], h4[3]});
+      ql[s] = __builtin_bit_cast(f16x8_t, u32x4{l4[0], l4[1], l4[2], l4[3]});
+    }
+  }
+  // the softmax's row of this lane: row orr of the wave's RPO, keys
+  // KPL*oc .. +KPL-1 of a tile
+  const int orr = lane / LPR, oc = lane % LPR;
+  int rt0, rnn;
+  float qunit;
+  bool orv;
+  {
+    const int row = r0 + 32 * rg + RPO * sl + orr;
+    orv = row < rows;
+    const int m = orv ? row / G : 0;
+    rt0 = orv ? t0_of(m) : 0;
+    rnn = orv ? nn_of(m) : 0;
+    const float* qmx = reinterpret_cast<const float*>(sx);
+    float qm = 0.f;
+#pragma unroll
+    for (int s = 0; s < NSL; ++s) qm = fmaxf(qm, qmx[(rg * NSL + s) * 32 + RPO * sl + orr]);
+    qunit = f16_row_unit(f16_row_shift(qm));
+  }
+
+  f32x16 o[4];
+#pragma unroll
+  for (int b = 0; b < 4; ++b)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) o[b][i] = 0.f;
+  float m_run = -INFINITY, l_run = 0.f;
+  constexpr int kNoShift = 1 << 20;  // no key yet (o = 0)
+  constexpr int kRoom = 3;
+  int wsh = kNoShift;
+
+  // Owner region of rows RPO*ow .. of row group g: 4 KB of sx.  First the
+  // score shares [slice][RPO rows][32 keys] floats, a row's 16-byte units
+  // (key quads) swizzled so that a store of 8 rows and a read of 16 lanes
+  // hit distinct units; then, read by its owner alone, overwritten with P:
+  // [piece][key octet][row] 16 bytes, and the rows' (alpha, dsh).
+  auto region = [&](int ow) { return sx + (rg * NSL + ow) * 4096; };
+  auto swz = [](int rr) {
+    return NSL == 4 ? rr & 7 : ((rr >> 1) & 1) | ((rr & 1) << 1) | (rr & 4);
+  };
+  const int my_ow = c32 / RPO, my_rr = c32 % RPO;  // this lane's MFMA column
+  char* s_st = region(my_ow) + sl * (RPO * 128) + my_rr * 128;
+  const int s_sw = 16 * (hh ^ swz(my_rr));
+  const char* s_ld = region(sl) + orr * 128;
+  const int o_sw = 16 * swz(orr);
+  const char* p_ld = region(my_ow) + (NSL == 4 ? (my_ow & 1) * 128 : 0) + my_rr * 16;
+  char* p_st = region(sl) + (NSL == 4 ? (sl & 1) * 128 : 0) + orr * 16;
+
+  const float* kun = reinterpret_cast<const float*>(khead + NP * Rp * D) - a.T0 + KPL * oc;
+  const float* vun = reinterpret_cast<const float*>(vhead + NP * Rp * D) - a.T0 + KPL * oc;
+  float ku[KPL], vu[KPL];
+  auto load_units = [&](int tk) {
+#pragma unroll
+    for (int q = 0; q < KPL; q += 4) {
+      const f32x4_u x = *reinterpret_cast<const f32x4_u*>(kun + tk + q);
+      const f32x4_u y = *reinterpret_cast<const f32x4_u*>(vun + tk + q);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        ku[q + e] = x[e];
+        vu[q + e] = y[e];
+      }
+    }
+  };
+  float nku[KPL], nvu[KPL];
+  if (ntile > 0) load_units(kt_s);
+  wait_vmcnt<0>();
+  __syncthreads();
+
+  for (int it = 0; it < ntile; ++it) {
+    const int tk = kt_s + it * KT;
+    const bool more = it + 1 < ntile;
+    const char* kb = kbuf[DB ? (it & 1) : 0];
+    const char* vb = vbuf[DB ? (it & 1) : 0];
+    {  // 1. this slice's share of the scores
+      f32x16 s2[2];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) s2[0][i] = s2[1][i] = 0.f;
+      const char* kr = kb + c32 * RB + 256 * sl;
+      const int kx = 16 * (hh ^ wk_f(c32));
+#pragma unroll
+      for (int s0 = 0; s0 < 8; s0 += 2) {
+        f16x8_t kc[2][NP];
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int p = 0; p < NP; ++p)
+            kc[j][p] = *reinterpret_cast<const f16x8_t*>(kr + p * KT * RB + (kx ^ (32 * (s0 + j))));
+        if constexpr (NP == 2) {
+#pragma unroll
+          for (int j = 0; j < 2; ++j) s2[j] = mfma32_f16(kc[j][1], qh[s0 + j], s2[j]);
+        }
+        // a quarter of V's copies (one buffer: this tile's, free since the
+        // last barrier; two: the next tile's K and V) between the products:
+        // issued together they hold a wave until the load path took them
+        if constexpr (DB) {
+          if (more) {
+#pragma unroll
+            for (int t = s0 / 2; t < NL; t += 4) {
+              copy1(t, tk + KT, kbuf[(it + 1) & 1], khead, false);
+              copy1(t, tk + KT, vbuf[(it + 1) & 1], vhead, true);
+            }
+          }
+        } else {
+#pragma unroll
+          for (int t = s0 / 2; t < NL; t += 4) copy1(t, tk, vbuf[0], vhead, true);
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) s2[j] = mfma32_f16(kc[j][0], ql[s0 + j], s2[j]);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) s2[j] = mfma32_f16(kc[j][0], qh[s0 + j], s2[j]);
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        f32x4 y;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = s2[0][4 * i + e] + s2[1][4 * i + e];
+        *reinterpret_cast<f32x4*>(s_st + (s_sw ^ (32 * i))) = y;
+      }
+    }
+    lds_barrier();  // A: the shares are in LDS, K's buffer is free
+    if (more) {
+      // the next tile's units (waited for where the copies are, below)
+#pragma unroll
+      for (int q = 0; q < KPL; q += 4) {
+        const f32x4_u x = *reinterpret_cast<const f32x4_u*>(kun + tk + KT + q);
+        const f32x4_u y = *reinterpret_cast<const f32x4_u*>(vun + tk + KT + q);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          nku[q + e] = x[e];
+          nvu[q + e] = y[e];
+        }
+      }
+    }
+    // K's copies of the next tile between the softmax's steps
+    auto next_k = [&](int t) {
+      if constexpr (!DB) {
+        if (more) {
+#pragma unroll
+          for (int i = 0; i < NL / 4; ++i) copy1(t * (NL / 4) + i, tk + KT, kbuf[0], khead, false);
+        }
+      }
+    };
+    {  // 2. softmax of the owned rows
+      float sv[KPL];
+#pragma unroll
+      for (int q = 0; q < KPL; q += 4) {
+        const int un = 16 * ((KPL / 4) * oc + q / 4);
+        f32x4 t = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < NSL; ++s) {
+          const f32x4 y = *reinterpret_cast<const f32x4*>(s_ld + s * (RPO * 128) + (un ^ o_sw));
+          t = s ? t + y : y;
+        }
+        if (q == 0) next_k(0);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) sv[q + e] = t[e] * ku[q + e];
+      }
+      const int k0 = tk + KPL * oc;
+      const bool full = __builtin_amdgcn_ballot_w64(!(orv && tk >= rt0 && tk + KT <= rnn)) == 0;
+      if (!full) {
+#pragma unroll
+        for (int e = 0; e < KPL; ++e)
+          sv[e] = (k0 + e >= rt0 && k0 + e < rnn) ? sv[e] : -INFINITY;
+      }
+      float tmax = sv[0];
+#pragma unroll
+      for (int e = 1; e < KPL; ++e) tmax = fmaxf(tmax, sv[e]);
+      next_k(1);
+      tmax = group_max<LPR>(tmax) * qunit;
+      // lazy rescale: the running max moves only when a score passes it by
+      // more than kLazyMax
+      const bool grow = tmax > m_run + kLazyMax;
+      const float mn = grow ? fmaxf(m_run, tmax) : m_run;
+      const float alpha = m_run == -INFINITY ? 1.f : exp2_hw(m_run - mn);
+      const int gsh = (grow && m_run != -INFINITY) ? (int)fminf(floorf(mn - m_run), 1000.f) : 0;
+      m_run = mn;
+      float p[KPL], ps = 0.f;
+#pragma unroll
+      for (int e = 0; e < KPL; ++e) {
+        p[e] = (!full && sv[e] == -INFINITY) ? 0.f : exp2_hw(fmaf(sv[e], qunit, -m_run));
+        ps += p[e];
+      }
+      {
+#pragma clang fp contract(off)
+        l_run = l_run * alpha + ps;
+      }
+      // y = p * u_key * 2^wsh below 2^14 (u_key the key's V row unit); wsh
+      // follows the row's largest p * u_key, and o down when the max moves.
+      // A larger term takes wsh kRoom bits lower than it needs, so that the
+      // next records of 32 rows do not each rescale o.
+      float zt = 0.f;
+#pragma unroll
+      for (int e = 0; e < KPL; ++e) {
+        p[e] *= vu[e];
+        zt = fmaxf(zt, p[e]);
+      }
+      next_k(2);
+      zt = group_max<LPR>(zt);
+      next_k(3);
+      const int grown = min(wsh + gsh, kNoShift);
+      const int most = zt > 0.f ? f16_row_shift(zt) : kNoShift;
+      const int ns = most < grown ? most - kRoom : grown;
+      const float fac = ldexpf(alpha, ns - wsh);  // of o (a power of two times alpha)
+      wsh = ns;
+      uint32_t yh[KPL / 2], yl[KPL / 2];
+#pragma unroll
+      for (int e = 0; e < KPL; e += 2) split2h(p[e], p[e + 1], ns, yh[e / 2], yl[e / 2]);
+      if constexpr (KPL == 4) {
+        char* d = p_st + (oc >> 1) * 256 + (oc & 1) * 8;
+        *reinterpret_cast<u32x2*>(d) = u32x2{yh[0], yh[1]};
+        *reinterpret_cast<u32x2*>(d + 1024) = u32x2{yl[0], yl[1]};
+      } else {
+        char* d = p_st + oc * 256;
+        *reinterpret_cast<u32x4*>(d) = u32x4{yh[0], yh[1], yh[KPL / 2 - 2], yh[KPL / 2 - 1]};
+        *reinterpret_cast<u32x4*>(d + 1024) = u32x4{yl[0], yl[1], yl[KPL / 2 - 2], yl[KPL / 2 - 1]};
+      }
+      if (oc == 0)
+        *reinterpret_cast<f32x4*>(region(sl) + 2048 + 16 * orr) = f32x4{fac, 0.f, 0.f, 0.f};
+    }
+    if constexpr (!DB) {  // V of this tile is in LDS; K of the next may be in flight
+      if (more)
+        wait_vmcnt<NL>();
+      else
+        wait_vmcnt<0>();
+    }
+    lds_barrier();  // B: P is in LDS
+    {  // 3. O^T += V^T . P^T of this slice
+      const float fac = (*reinterpret_cast<const f32x4*>(region(my_ow) + 2048 + 16 * my_rr))[0];
+      f16x8_t yh[2], yl[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        yh[j] = *reinterpret_cast<const f16x8_t*>(p_ld + (2 * j + hh) * 256);
+        yl[j] = *reinterpret_cast<const f16x8_t*>(p_ld + 1024 + (2 * j + hh) * 256);
+      }
+      if (__builtin_amdgcn_ballot_w64(fac != 1.f) != 0) {
+#pragma unroll
+        for (int b = 0; b < 4; ++b)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) o[b][i] *= fac;
+      }
+      // transposed reads: 16-lane group (2*h + x) reads keys 16j + 8h + 4u ..
+      // +3 (lane/4 of it) of the block's 16 columns 16x .. +15
+      const int l16 = lane & 15;
+      const char* vr = vb + (8 * hh + (l16 >> 2)) * RB + 256 * sl + 32 * ((lane >> 4) & 1) +
+                       16 * ((l16 & 3) >> 1) + 8 * (l16 & 1);
+      const int vx = 64 * (l16 >> 2);  // the rows' swizzle (64-byte steps)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+#pragma unroll
+        for (int b0 = 0; b0 < 4; b0 += 2) {
+          f16x8_t av[2][NP];
+#pragma unroll
+          for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int p = 0; p < NP; ++p) {
+              i16x4_t t2[2];
+#pragma unroll
+              for (int u = 0; u < 2; ++u)
+                t2[u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                    (__attribute__((address_space(3))) i16x4_t*)(
+                        vr + p * KT * RB + (16 * j + 4 * u) * RB + ((64 * (b0 + b)) ^ vx)));
+              av[b][p] = __builtin_bit_cast(
+                  f16x8_t, __builtin_shufflevector(t2[0], t2[1], 0, 1, 2, 3, 4, 5, 6, 7));
+            }
+          if constexpr (NP == 2) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b) o[b0 + b] = mfma32_f16(av[b][1], yh[j], o[b0 + b]);
+          }
+#pragma unroll
+          for (int b = 0; b < 2; ++b) o[b0 + b] = mfma32_f16(av[b][0], yl[j], o[b0 + b]);
+#pragma unroll
+          for (int b = 0; b < 2; ++b) o[b0 + b] = mfma32_f16(av[b][0], yh[j], o[b0 + b]);
+        }
+      }
+    }
+    if (more) {
+#pragma unroll
+      for (int e = 0; e < KPL; ++e) {
+        ku[e] = nku[e];
+        vu[e] = nvu[e];
+        asm volatile("" : "+v"(ku[e]), "+v"(vu[e]));  // the units' wait falls here
+      }
+    }
+    wait_vmcnt<0>();  // the next tile's copies (one buffer: K's) are in LDS
+    lds_barrier();    // C: V, P and the shares may be overwritten
+  }
+
+  // the rows' (l, m, wsh) from their owners to the waves that hold their o
+  l_run = group_sum<LPR>(l_run);
+  if (oc == 0)
+    *reinterpret_cast<f32x4*>(region(sl) + 16 * orr) = f32x4{l_run, m_run, (float)wsh, 0.f};
+  lds_barrier();
+  const f32x4 st = *reinterpret_cast<const f32x4*>(region(my_ow) + 16 * my_rr);
+  const int row = r0 + 32 * rg + c32;
+  if (row >= rows) return;
+  const int m = row / G, g = row - m * G;
+  const int64_t slot = (int64_t)m * a.nq + h * G + g;
+  const int sh = -(int)st[2];
+  if (a.nsplit > 1) {
+    const int64_t ps = slot * a.nsplit + sp;
+    float* po = a.part_o + ps * D + 128 * sl + 4 * hh;
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        f32x4 y;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = ldexpf(o[b][4 * i + e], sh);
+        *reinterpret_cast<f32x4*>(po + 32 * b + 8 * i) = y;
+      }
+    if (sl == 0 && hh == 0) {
+      a.part_ml[2 * ps] = st[1] == -INFINITY ? -INFINITY : st[1] * kLn2;
+      a.part_ml[2 * ps + 1] = st[0];
+    }
+  } else {
+    const float inv = st[0] > 0.f ? 1.f / st[0] : 0.f;  // no key: O = 0 (gemm.h:438)
+    float* po = a.o + slot * a.dh;
+    const bool v4 = (a.dh & 3) == 0;
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int e0 = 128 * sl + 32 * b + 8 * i + 4 * hh;
+        f32x4 y;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) y[e] = ldexpf(o[b][4 * i + e], sh) * inv;
+        if (v4) {
+          if (e0 < a.dh) *reinterpret_cast<f32x4*>(po + e0) = y;
+        } else {
+          if (e0 < a.dh) *reinterpret_cast<f32x2*>(po + e0) = f32x2{y[0], y[1]};
+          if (e0 + 2 < a.dh) *reinterpret_cast<f32x2*>(po + e0 + 2) = f32x2{y[2], y[3]};
+        }
+      }
+  }
+}
+
+template <int D, typename T>
+SplitFn split_of(bool paged) {
+  return paged ? wide_split_kernel<D, T, true> : wide_split_kernel<D, T, false>;
+}
+
+}  // namespace
+
+SplitFn prefill_wide_split(int D, int kv_dtype, bool paged) {
+  if (D != 512) return nullptr;
+  if (kv_dtype == MOLOT_KV_Q8) return split_of<512, q8_t>(paged);
+  if (kv_dtype == MOLOT_KV_BF16) return split_of<512, bf16_t>(paged);
+  return split_of<512, float>(paged);
+}
+
+PfFn prefill_wide_fn(int D, int kv_dtype) {
+  if (D != 512) return nullptr;
+  return kv_dtype == MOLOT_KV_F32 ? prefill_wide_kernel<512, 2> : prefill_wide_kernel<512, 1>;
+}
