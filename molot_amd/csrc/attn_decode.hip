@@ -435,11 +435,15 @@ __global__ __launch_bounds__(kRopeTokThreads) void rope_append_tok_kernel(RopeAr
   }
 }
 
-// rope_append_tok_kernel for M tokens of head dim d (<= 2048).
+// rope_append_tok_kernel for M tokens of head dim d (<= 2048), in the
+// narrowest instance: each pair group past d/2 costs registers and issue
+// slots (1999 tokens of 8q/2kv/d512: 63 us in the 16-group instance, 29 in
+// the 4-group one).
 int launch_rope_tok(const RopeArgs& r, int M, void* stream) {
   const int half = r.d / 2;
   auto k = half <= 64 ? rope_append_tok_kernel<1>
            : half <= 128 ? rope_append_tok_kernel<2>
+           : half <= 256 ? rope_append_tok_kernel<4>
                          : rope_append_tok_kernel<kRopeMaxPairs / 64>;
   hipLaunchKernelGGL(k, dim3(M), dim3(kRopeTokThreads), 0, (hipStream_t)stream, r);
   return (int)hipGetLastError();
