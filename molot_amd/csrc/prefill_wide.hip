@@ -42,49 +42,10 @@
 #include "device_util.hpp"
 #include "molot_amd/attn_hip.h"
 #include "prefill.hpp"
+#include "prefill_tile.hpp"
 #include "prefill_wide.hpp"
 
 namespace {
-
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));  // dword-aligned
-typedef short i16x4_t __attribute__((ext_vector_type(4)));
-
-__device__ __forceinline__ f32x16 mfma32_f16(f16x8_t a, f16x8_t b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-}
-
-// Swizzles of the staged rows (16-byte units; unit ch of row r at ch ^ f(r)).
-// K: a 16-byte read takes one unit of 16 consecutive rows.  V: a transposed
-// read takes 64 bytes of 4 consecutive rows.  Both then cover 256 bytes.
-__device__ __forceinline__ int wk_f(int r) { return r & 15; }
-__device__ __forceinline__ int wv_f(int r) { return (r & 3) << 2; }
-
-// Offset (elements; Q8 bytes) of row t of KV head h in a cache of head dim
-// a.dh, and of a Q8 row's scale.
-template <typename T, bool PAGED>
-__device__ __forceinline__ int64_t wide_row_off(const PfArgs& a, int h, int t, int64_t& soff) {
-  constexpr bool Q8 = std::is_same<T, q8_t>::value;
-  const int dh = a.dh;
-  if constexpr (PAGED) {
-    const int pg = 1 << a.page_shift;
-    const int64_t blk = a.block_table[t >> a.page_shift];
-    const int sl = t & (pg - 1);
-    if constexpr (Q8) {
-      const int64_t bb = (int64_t)a.nkv * pg * (dh + 4);
-      soff = blk * bb + (int64_t)a.nkv * pg * dh + 4 * ((int64_t)h * pg + sl);
-      return blk * bb + ((int64_t)h * pg + sl) * dh;
-    }
-    return ((blk * a.nkv + h) * pg + sl) * (int64_t)dh;
-  } else {
-    if constexpr (Q8) {
-      const int64_t rb = (int64_t)a.nkv * dh + ((4 * a.nkv + 15) & ~15);
-      soff = (int64_t)t * rb + (int64_t)a.nkv * dh + 4 * h;
-      return (int64_t)t * rb + (int64_t)h * dh;
-    }
-    return ((int64_t)t * a.nkv + h) * (int64_t)dh;
-  }
-}
 
 // The attended keys [T0, T0 + R) of every KV head as fp16 pieces, in the
 // layout of prefill_wide.hpp; the kWideTail rows after them are zeros, so
@@ -92,7 +53,6 @@ __device__ __forceinline__ int64_t wide_row_off(const PfArgs& a, int h, int t, i
 // row's D/8 units in consecutive lanes; grid (units / 256, nkv, K or V).
 template <int D, typename T, bool PAGED>
 __global__ __launch_bounds__(256) void wide_split_kernel(PfArgs a, uint16_t* out) {
-  constexpr bool Q8 = std::is_same<T, q8_t>::value;
   constexpr int NP = wide_pieces_v<T>;
   constexpr int UPR = D / 8;
   const int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -101,60 +61,9 @@ __global__ __launch_bounds__(256) void wide_split_kernel(PfArgs a, uint16_t* out
   const int h = blockIdx.y, kv = blockIdx.z;
   const int64_t r = u / UPR;
   const int j = (int)(u - r * UPR);
-  float x[8];
-#pragma unroll
-  for (int e = 0; e < 8; ++e) x[e] = 0.f;
+  float x[8] = {};
   float s = 1.f;
-  if (r < a.R) {
-    int64_t soff = 0;
-    const int64_t off = wide_row_off<T, PAGED>(a, h, a.T0 + (int)r, soff);
-    const char* base = reinterpret_cast<const char*>(kv ? a.v : a.k);
-    const int e0 = 8 * j, n = min(8, a.dh - e0);  // elements of the row in this unit
-    if constexpr (Q8) {  // dh a multiple of 4: whole 4-code words
-      s = *reinterpret_cast<const float*>(base + soff);
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        if (4 * i < n) {
-          const uint32_t c = *reinterpret_cast<const uint32_t*>(base + off + e0 + 4 * i);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) x[4 * i + e] = (float)(int8_t)((c >> (8 * e)) & 0xFF);
-        }
-      }
-    } else if constexpr (sizeof(T) == 2) {
-      const uint16_t* p = reinterpret_cast<const uint16_t*>(base) + off + e0;
-      if (n == 8 && (a.dh & 7) == 0) {
-        const u32x4 v = *reinterpret_cast<const u32x4*>(p);
-        KVT<bf16_t>::unpack(v, x);
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (2 * i < n) {
-            const uint32_t v = *reinterpret_cast<const uint32_t*>(p + 2 * i);
-            x[2 * i] = __uint_as_float(v << 16);
-            x[2 * i + 1] = __uint_as_float(v & 0xFFFF0000u);
-          }
-      }
-    } else {
-      const float* p = reinterpret_cast<const float*>(base) + off + e0;
-      if (n == 8 && (a.dh & 3) == 0) {
-        const f32x4 x0 = *reinterpret_cast<const f32x4*>(p);
-        const f32x4 x1 = *reinterpret_cast<const f32x4*>(p + 4);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          x[e] = x0[e];
-          x[4 + e] = x1[e];
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          if (2 * i < n) {
-            const f32x2 v = *reinterpret_cast<const f32x2*>(p + 2 * i);
-            x[2 * i] = v[0];
-            x[2 * i + 1] = v[1];
-          }
-      }
-    }
-  }
+  if (r < a.R) s = wide_load8<T, PAGED>(a, kv, h, a.T0 + (int)r, j, x);
   float xm = 0.f;
 #pragma unroll
   for (int e = 0; e < 8; ++e) xm = fmaxf(xm, fabsf(x[e]));
@@ -231,7 +140,7 @@ __global__ __launch_bounds__(512) void prefill_wide_kernel(PfArgs a) {
     const int r_in = lane / UPR, jpos = lane % UPR;
     const int bi = w + 8 * t;  // wave-uniform
     const int pc = bi / BPP, rb = (bi % BPP) * RPB;
-    const int ch = jpos ^ (isv ? wv_f(rb + r_in) : wk_f(rb + r_in));
+    const int ch = jpos ^ (isv ? wv_f<D>(rb + r_in) : wk_f<D>(rb + r_in));
     dma16(head + (pc * Rp + (tk - a.T0) + rb) * D, (uint32_t)(r_in * RB + 16 * ch),
           (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)(buf + bi * 1024));
   };
@@ -304,13 +213,12 @@ __global__ __launch_bounds__(512) void prefill_wide_kernel(PfArgs a) {
   const int orr = lane / LPR, oc = lane % LPR;
   int rt0, rnn;
   float qunit;
-  bool orv;
   {
     const int row = r0 + 32 * rg + RPO * sl + orr;
-    orv = row < rows;
+    const bool orv = row < rows;
     const int m = orv ? row / G : 0;
-    rt0 = orv ? t0_of(m) : 0;
-    rnn = orv ? nn_of(m) : 0;
+    rt0 = orv ? t0_of(m) : 0;  // a row past the last: any keys (not stored)
+    rnn = orv ? nn_of(m) : 0x7FFFFFFF;
     const float* qmx = reinterpret_cast<const float*>(sx);
     float qm = 0.f;
 #pragma unroll
@@ -323,10 +231,7 @@ __global__ __launch_bounds__(512) void prefill_wide_kernel(PfArgs a) {
   for (int b = 0; b < 4; ++b)
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[b][i] = 0.f;
-  float m_run = -INFINITY, l_run = 0.f;
-  constexpr int kNoShift = 1 << 20;  // no key yet (o = 0)
-  constexpr int kRoom = 3;
-  int wsh = kNoShift;
+  RowState rs;  // of the owned row
 
   // Owner region of rows RPO*ow .. of row group g: 4 KB of sx.  First the
   // score shares [slice][RPO rows][32 keys] floats, a row's 16-byte units
@@ -375,7 +280,7 @@ __global__ __launch_bounds__(512) void prefill_wide_kernel(PfArgs a) {
 #pragma unroll
       for (int i = 0; i < 16; ++i) s2[0][i] = s2[1][i] = 0.f;
       const char* kr = kb + c32 * RB + 256 * sl;
-      const int kx = 16 * (hh ^ wk_f(c32));
+      const int kx = 16 * (hh ^ wk_f<D>(c32));
 #pragma unroll
       for (int s0 = 0; s0 < 8; s0 += 2) {
         f16x8_t kc[2][NP];
@@ -452,58 +357,17 @@ __global__ __launch_bounds__(512) void prefill_wide_kernel(PfArgs a) {
         }
         if (q == 0) next_k(0);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) sv[q + e] = t[e] * ku[q + e];
+        for (int e = 0; e < 4; ++e) sv[q + e] = t[e];
       }
       const int k0 = tk + KPL * oc;
-      const bool full = __builtin_amdgcn_ballot_w64(!(orv && tk >= rt0 && tk + KT <= rnn)) == 0;
-      if (!full) {
-#pragma unroll
-        for (int e = 0; e < KPL; ++e)
-          sv[e] = (k0 + e >= rt0 && k0 + e < rnn) ? sv[e] : -INFINITY;
-      }
-      float tmax = sv[0];
-#pragma unroll
-      for (int e = 1; e < KPL; ++e) tmax = fmaxf(tmax, sv[e]);
+      const bool full = __builtin_amdgcn_ballot_w64(tk < rt0 || tk + KT > rnn) == 0;
       next_k(1);
-      tmax = group_max<LPR>(tmax) * qunit;
-      // lazy rescale: the running max moves only when a score passes it by
-      // more than kLazyMax
-      const bool grow = tmax > m_run + kLazyMax;
-      const float mn = grow ? fmaxf(m_run, tmax) : m_run;
-      const float alpha = m_run == -INFINITY ? 1.f : exp2_hw(m_run - mn);
-      const int gsh = (grow && m_run != -INFINITY) ? (int)fminf(floorf(mn - m_run), 1000.f) : 0;
-      m_run = mn;
-      float p[KPL], ps = 0.f;
-#pragma unroll
-      for (int e = 0; e < KPL; ++e) {
-        p[e] = (!full && sv[e] == -INFINITY) ? 0.f : exp2_hw(fmaf(sv[e], qunit, -m_run));
-        ps += p[e];
-      }
-      {
-#pragma clang fp contract(off)
-        l_run = l_run * alpha + ps;
-      }
-      // y = p * u_key * 2^wsh below 2^14 (u_key the key's V row unit); wsh
-      // follows the row's largest p * u_key, and o down when the max moves.
-      // A larger term takes wsh kRoom bits lower than it needs, so that the
-      // next records of 32 rows do not each rescale o.
-      float zt = 0.f;
-#pragma unroll
-      for (int e = 0; e < KPL; ++e) {
-        p[e] *= vu[e];
-        zt = fmaxf(zt, p[e]);
-      }
-      next_k(2);
-      zt = group_max<LPR>(zt);
-      next_k(3);
-      const int grown = min(wsh + gsh, kNoShift);
-      const int most = zt > 0.f ? f16_row_shift(zt) : kNoShift;
-      const int ns = most < grown ? most - kRoom : grown;
-      const float fac = ldexpf(alpha, ns - wsh);  // of o (a power of two times alpha)
-      wsh = ns;
       uint32_t yh[KPL / 2], yl[KPL / 2];
-#pragma unroll
-      for (int e = 0; e < KPL; e += 2) split2h(p[e], p[e + 1], ns, yh[e / 2], yl[e / 2]);
+      const float fac = softmax_tile<KPL>(
+          sv, ku, vu, qunit, rs, full, [](float x) { return group_max<LPR>(x); },
+          [&](int e) { return k0 + e < rt0 || k0 + e >= rnn; }, yh, yl);
+      next_k(2);
+      next_k(3);
       if constexpr (KPL == 4) {
         char* d = p_st + (oc >> 1) * 256 + (oc & 1) * 8;
         *reinterpret_cast<u32x2*>(d) = u32x2{yh[0], yh[1]};
@@ -585,9 +449,9 @@ __global__ __launch_bounds__(512) void prefill_wide_kernel(PfArgs a) {
   }
 
   // the rows' (l, m, wsh) from their owners to the waves that hold their o
-  l_run = group_sum<LPR>(l_run);
+  rs.l = group_sum<LPR>(rs.l);
   if (oc == 0)
-    *reinterpret_cast<f32x4*>(region(sl) + 16 * orr) = f32x4{l_run, m_run, (float)wsh, 0.f};
+    *reinterpret_cast<f32x4*>(region(sl) + 16 * orr) = f32x4{rs.l, rs.m, (float)rs.wsh, 0.f};
   lds_barrier();
   const f32x4 st = *reinterpret_cast<const f32x4*>(region(my_ow) + 16 * my_rr);
   const int row = r0 + 32 * rg + c32;
@@ -608,7 +472,7 @@ __global__ __launch_bounds__(512) void prefill_wide_kernel(PfArgs a) {
         *reinterpret_cast<f32x4*>(po + 32 * b + 8 * i) = y;
       }
     if (sl == 0 && hh == 0) {
-      a.part_ml[2 * ps] = st[1] == -INFINITY ? -INFINITY : st[1] * kLn2;
+      a.part_ml[2 * ps] = st[0] > 0.f ? st[1] * kLn2 : -INFINITY;
       a.part_ml[2 * ps + 1] = st[0];
     }
   } else {
