@@ -56,7 +56,7 @@ def _run(cmd: list[str]) -> None:
 
 
 # the library's kernel sources, compiled side by side
-LIB_SOURCES = ("attn_decode.hip", "prefill_wide.hip")
+LIB_SOURCES = ("attn_decode.hip", "prefill_wide.hip", "prefill_narrow.hip")
 
 
 def _compile(name: str) -> str:

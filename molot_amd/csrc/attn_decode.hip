@@ -63,6 +63,9 @@ struct RopeArgs {
   // [K, V][nkv][3][pc_R][d], when that row lies in [0, pc_R) (NULL: none)
   uint16_t* pieces;
   int pc_T0, pc_R;
+  // pieces per value in the layout of prefill_wide.hpp (0: the three-slot
+  // layout of pf_split_kernel)
+  int pc_np;
 };
 
 // Sum over the workgroup (at most 16 waves); every thread gets the total.
@@ -210,7 +213,10 @@ __global__ void rope_append_kernel(RopeArgs a) {
 // 2048 tokens of 32q/8kv/d128: 81920 single-wave workgroups became 2048.
 constexpr int kRopeTokThreads = 256;
 constexpr int kRopeMaxPairs = 1024;  // d <= 2048
-template <int KMAX>  // pair groups of 64 a head holds at most (d <= 128 KMAX)
+// KMAX: pair groups of 64 a head holds at most (d <= 128 KMAX); P32: the
+// rows' pieces in the layout of prefill_wide.hpp, pc_np of them, else in the
+// three slots of pf_split_kernel.
+template <int KMAX, bool P32>
 __global__ __launch_bounds__(kRopeTokThreads) void rope_append_tok_kernel(RopeArgs a) {
   __shared__ float cs_s[kRopeMaxPairs], sn_s[kRopeMaxPairs];
   __shared__ float sh[16];
@@ -391,10 +397,18 @@ __global__ __launch_bounds__(kRopeTokThreads) void rope_append_tok_kernel(RopeAr
     // V as two fp16 pieces of the row scaled by a power of two (split2h,
     // the row's unit at float pr of the head's third piece)
     const int pr = slot - a.pc_T0;
-    if (a.pieces && a.kv_dtype != MOLOT_KV_BF16 && pr >= 0 && pr < a.pc_R) {
-      const int64_t pstride = (int64_t)a.pc_R * a.d;  // one piece of one head
+    if (a.pieces && (P32 || a.kv_dtype != MOLOT_KV_BF16) && pr >= 0 && pr < a.pc_R) {
+      const int np = P32 ? a.pc_np : 0;
+      const int64_t Rp = np ? wide_padded_rows(a.pc_R) : a.pc_R;
+      const int64_t pstride = Rp * a.d;  // one piece of one head
+      const int64_t hstride = np ? wide_head_elems(a.d, np, Rp) : 3 * pstride;
+      // the value a piece holds: as cached (three-slot layout: Q8 code *
+      // scale; else its code, the scale goes into the unit)
       auto cached = [&](float x, float sc) {
-        return a.kv_dtype == MOLOT_KV_Q8 ? (float)q8_code(x, sc) * sc : x;
+        if (a.kv_dtype == MOLOT_KV_Q8) return np ? (float)q8_code(x, sc) : (float)q8_code(x, sc) * sc;
+        if (P32 && a.kv_dtype == MOLOT_KV_BF16)
+          return __uint_as_float((uint32_t)f32_to_bf16(x) << 16);
+        return x;
       };
       float kpm = 0.f, vpm = 0.f;  // the rows' largest |k| and |v| as cached
 #pragma unroll
@@ -408,12 +422,13 @@ __global__ __launch_bounds__(kRopeTokThreads) void rope_append_tok_kernel(RopeAr
       const int kshift = f16_row_shift(group_max<64>(kpm));
       vpm = group_max<64>(vpm);
       const int vshift = f16_vrow_shift(vpm);
-      uint16_t* ok = a.pieces + (int64_t)kh * 3 * pstride + (int64_t)pr * a.d;
-      uint16_t* ov = ok + (int64_t)a.nkv * 3 * pstride;
-      if (lane == 0) {  // the units of a head's rows side by side in its third piece
-        reinterpret_cast<float*>(ok - (int64_t)pr * a.d + 2 * pstride)[pr] = f16_row_unit(kshift);
-        reinterpret_cast<float*>(ov - (int64_t)pr * a.d + 2 * pstride)[pr] =
-            f16_vrow_unit(vpm, vshift);
+      uint16_t* ok = a.pieces + (int64_t)kh * hstride + (int64_t)pr * a.d;
+      uint16_t* ov = ok + (int64_t)a.nkv * hstride;
+      if (lane == 0) {  // the units of a head's rows side by side after its pieces
+        const int64_t uo = (np ? np : 2) * pstride - (int64_t)pr * a.d;
+        const bool q8u = np && a.kv_dtype == MOLOT_KV_Q8;
+        reinterpret_cast<float*>(ok + uo)[pr] = f16_row_unit(kshift) * (q8u ? ks : 1.f);
+        reinterpret_cast<float*>(ov + uo)[pr] = f16_vrow_unit(vpm, vshift) * (q8u ? vs : 1.f);
       }
 #pragma unroll
       for (int k = 0; k < KMAX; ++k) {
@@ -425,11 +440,27 @@ __global__ __launch_bounds__(kRopeTokThreads) void rope_append_tok_kernel(RopeAr
         split2h(cached(v0[k], vs), cached(v1[k], vs), vshift, pv[0], pv[1]);
 #pragma unroll
         for (int pc = 0; pc < 2; ++pc) {
+          if (pc == 1 && np == 1) break;
           ok[pc * pstride + j] = (uint16_t)(pk[pc] & 0xFFFF);
           ok[pc * pstride + j + half] = (uint16_t)(pk[pc] >> 16);
           ov[pc * pstride + j] = (uint16_t)(pv[pc] & 0xFFFF);
           ov[pc * pstride + j + half] = (uint16_t)(pv[pc] >> 16);
         }
+      }
+    }
+  }
+  // the rows of zeros after the pieces, dealt to the tokens' workgroups
+  if constexpr (P32) {
+    const int64_t Rp = wide_padded_rows(a.pc_R), hs = wide_head_elems(a.d, a.pc_np, Rp);
+    const int upr = a.d / 8;  // 16-byte units a row
+    const int n = 2 * a.nkv * a.pc_np * upr;
+    for (int64_t r = a.pc_R + b; r < Rp; r += gridDim.x) {
+      for (int i = tid; i < n; i += kRopeTokThreads) {
+        const int j = i % upr, p = i / upr % a.pc_np, hd = i / upr / a.pc_np;
+        *reinterpret_cast<u32x4*>(a.pieces + hd * hs + (p * Rp + r) * a.d + 8 * j) =
+            u32x4{0u, 0u, 0u, 0u};
+        if (j == 0 && p == 0)
+          reinterpret_cast<float*>(a.pieces + hd * hs + a.pc_np * Rp * a.d)[r] = 0.f;
       }
     }
   }
@@ -441,10 +472,11 @@ __global__ __launch_bounds__(kRopeTokThreads) void rope_append_tok_kernel(RopeAr
 // the 4-group one).
 int launch_rope_tok(const RopeArgs& r, int M, void* stream) {
   const int half = r.d / 2;
-  auto k = half <= 64 ? rope_append_tok_kernel<1>
-           : half <= 128 ? rope_append_tok_kernel<2>
-           : half <= 256 ? rope_append_tok_kernel<4>
-                         : rope_append_tok_kernel<kRopeMaxPairs / 64>;
+  auto k = half <= 64 ? (r.pieces && r.pc_np ? rope_append_tok_kernel<1, true>
+                                             : rope_append_tok_kernel<1, false>)
+           : half <= 128 ? rope_append_tok_kernel<2, false>
+           : half <= 256 ? rope_append_tok_kernel<4, false>
+                         : rope_append_tok_kernel<kRopeMaxPairs / 64, false>;
   hipLaunchKernelGGL(k, dim3(M), dim3(kRopeTokThreads), 0, (hipStream_t)stream, r);
   return (int)hipGetLastError();
 }
@@ -4260,7 +4292,7 @@ PfFn pf_kernel_d(int d, int pw) {
   return nullptr;  // Q8 prefill: d = 64, 128
 }
 
-// The prefill kernel over pre-split pieces (any cache type but bf16).
+// prefill_mfma16_kernel over pre-split pieces (any cache type but bf16).
 PfFn pf_kernel_pre(int d, int pw) {
   if (d == 64) return pw == 8 ? prefill_mfma16_kernel<64, float, false, 8, true>
                               : prefill_mfma16_kernel<64, float, false, 4, true>;
@@ -4270,15 +4302,11 @@ PfFn pf_kernel_pre(int d, int pw) {
                  : prefill_mfma16_kernel<256, float, false, 4, true>;
 }
 
-SplitFn pf_split(int d, int kv_dtype, bool paged) {
-  if (kv_dtype == MOLOT_KV_Q8) {
-    if (d == 64) return paged ? pf_split_kernel<64, q8_t, true> : pf_split_kernel<64, q8_t, false>;
-    if (d == 128)
-      return paged ? pf_split_kernel<128, q8_t, true> : pf_split_kernel<128, q8_t, false>;
+// The split of cached rows for it (d = 256: below, a step's rows leave their
+// pieces themselves or no pieces are made).
+SplitFn pf_split(int kv_dtype, bool paged) {
+  if (kv_dtype == MOLOT_KV_Q8)
     return paged ? pf_split_kernel<256, q8_t, true> : pf_split_kernel<256, q8_t, false>;
-  }
-  if (d == 64) return paged ? pf_split_kernel<64, float, true> : pf_split_kernel<64, float, false>;
-  if (d == 128) return paged ? pf_split_kernel<128, float, true> : pf_split_kernel<128, float, false>;
   return paged ? pf_split_kernel<256, float, true> : pf_split_kernel<256, float, false>;
 }
 
@@ -4804,7 +4832,7 @@ static int prefill_pieces(int nkv, int N, int d, int pos0, int window, int kv_dt
 
 // The prefill at a head dim the matrix-core prefill does not tile (an even d
 // that is not a multiple of 8; a padded Q8 cache), and above 256 where the
-// prompt is too small for prefill_wide or its workspace cannot be had:
+// prompt is too small for prefill_on_pieces or its workspace cannot be had:
 // the vector-ALU decode kernel with each query row as a sequence of its own
 // (AttnArgs::pf) over the one cache, contiguous or through the prompt's
 // block-table row.  Each query row streams its attended rows; neighbouring
@@ -4906,13 +4934,14 @@ static int launch_prefill(PfFn pk, int64_t wgs, int threads, const PfArgs& a, in
   return (int)hipGetLastError();
 }
 
-// Key splits of a prefill_wide_kernel launch of nqb * nkv query blocks (one
-// workgroup a CU): the count with the least estimated time.  A split's cost
-// is its tiles' plus its start and end; the launch's the longest split's, or
-// the CUs' share of all of them with half of the shortest for the uneven last
-// round; and more than one split pays the merge of their partials.
-static int wide_splits(int64_t nqb, int nkv, int M, int N, int G, int qb, int D, int pos0,
-                       int window, int nq) {
+// Key splits of a launch of nqb * nkv query blocks of qb rows on the 32-row
+// kernels (one workgroup a CU): the count with the least estimated time.  A
+// split's cost is its tiles' plus its start and end; the launch's the longest
+// split's, or the CUs' share of all of them with half of the shortest for the
+// uneven last round; and more than one split pays the merge of their
+// partials.
+static int pieces_splits(int64_t nqb, int nkv, int M, int N, int G, int qb, int D, bool f32,
+                         int pos0, int window, int nq) {
   auto tiles_of = [&](int64_t b) {  // query block b's tiles (32 keys)
     const int64_t m0 = b * qb / G, m1 = std::min<int64_t>(((b + 1) * qb - 1) / G, M - 1);
     const int64_t lo = window > 0 ? std::max<int64_t>(0, pos0 + m0 - window + 1) : 0;
@@ -4922,8 +4951,10 @@ static int wide_splits(int64_t nqb, int nkv, int M, int N, int G, int qb, int D,
   const double first = tiles_of(0), last = tiles_of(nqb - 1), mid = tiles_of(nqb / 2);
   const double longest = std::max({first, mid, last}), shortest = std::min({first, mid, last});
   const double total = (first + 4 * mid + last) / 6 * (double)(nqb * nkv);
-  const double kStart = 3.0;                 // a split's start and end, in tiles
-  const double kTileUs = 1.8 * D / 512;
+  // measured, us: a tile (D = 128 two in 2.3 over fp32, 1.75 over one piece;
+  // D = 512 3.2) and a split's start and end
+  const double kTileUs = (D <= 128 ? 1.15 * D / 128 : 3.2 * D / 512) * (f32 ? 1.0 : 0.75);
+  const double kStart = 6.0 / kTileUs;
   const int cus = num_cus();
   double best = 0;
   int ns_best = 1;
@@ -4942,14 +4973,52 @@ static int wide_splits(int64_t nqb, int nkv, int M, int N, int G, int qb, int D,
   return ns_best;
 }
 
-// The prefill at head dims above 256 on the matrix cores
-// (prefill_wide_kernel, padded to D = 512): the attended keys' pieces first,
-// then the attention over them.  MOLOT_ENOWS: a capture that would have to
-// grow the workspace, or keys past its cap (the caller takes prefill_rows).
-static int prefill_wide(const float* Qm, const void* K, const void* V, float* Om, int nq, int nkv,
-                        int M, int N, int d, float scale, int pos0, int window, int kv_dtype,
-                        const int32_t* block_row, int page, void* stream) {
-  const int D = 512, np = wide_pieces(kv_dtype == MOLOT_KV_F32), qb = wide_rows(D);
+// The head dim a prefill of head dim d is padded to.
+static int prefill_D(int d) { return d <= 64 ? 64 : d <= 128 ? 128 : d <= 256 ? 256 : 512; }
+
+// Whether a prefill runs on the 32-row kernels over fp16 pieces
+// (prefill_on_pieces): those stage and start more, so they take prompts with
+// enough work.  Not at 129 to 256: prefill_wide_kernel built for D = 256 took
+// 103 / 117 / 118 us a step (2048 tokens, 8q/4kv/d256, window 1024; fp32 / bf16
+// / Q8) against 102 / 90 / 105 on prefill_mfma16_kernel.
+// Above 256 the other path is prefill_rows.  Both sides, 8q/2kv/d512, us a
+// step over fp32 / bf16 / Q8 caches: (rows, cached) = (64, 500) prefill rows
+// 40 / 40 / 37, matrix cores 44 / 38 / 38; (8, 4000) 43 / 38 / 37 against 47 /
+// 38 / 41; (24, 4000) 123 / 117 / 96 against 53 / 44 / 46; (8, 16384) 118 / 94
+// / 77 against 92 / 64 / 61; (2, 16384) 63 / 41 / 36 against 89 / 60 / 58.
+// Up to 128 it is prefill_mfma16_kernel.  32q/8kv/d128, fp32 / bf16 / Q8:
+// (77, 4000) 80 / 64 / 78 against 75 / 64 / 65; (200, 2000) 76 / - / 77
+// against 70 / - / 62; (512, 0) 39 / 35 / 40 against 38 / 36 / 37; (200, 500)
+// 44 / 35 / 45 against 48 / 45 / 46; (512, 16384) 497 / 414 / 485 against 432
+// / 299 / 294.
+static bool prefill_takes_pieces(int d, int M, int N, int nq, int window) {
+  constexpr int64_t kWideWork = 400000, kPairFlops = 1200000000;
+  const int64_t span = window > 0 && window < N ? window : N;
+  const int64_t pairs = (int64_t)M * nq * span;
+  if (M > 65535 || (d > 128 && d <= 256)) return false;
+  return d > 256 ? pairs >= kWideWork : pairs * prefill_D(d) >= kPairFlops;
+}
+
+// Their workspace for the attended keys [T0, N).
+static int pieces32_workspace(int nkv, int N, int d, int pos0, int window, int kv_dtype,
+                              void* stream, void** ws, int* T0, int* R) {
+  *T0 = window > 0 && pos0 - window + 1 > 0 ? std::min(pos0 - window + 1, N) : 0;
+  *R = N - *T0;
+  const size_t need = wide_bytes(nkv, prefill_D(d), wide_pieces(kv_dtype == MOLOT_KV_F32), *R);
+  if (need > kMaxPiecesBytes) return MOLOT_ENOWS;
+  return pieces_workspace(stream, need, ws);
+}
+
+// The prefill on the 32-row kernels (prefill_narrow.hip, prefill_wide.hip):
+// the attended keys' pieces first (split_rows of them; the appending step
+// wrote the others), then the attention over them.  MOLOT_ENOWS: a capture
+// that would have to grow the workspace, or keys past its cap (the caller
+// takes the other path).
+static int prefill_on_pieces(const float* Qm, const void* K, const void* V, float* Om, int nq,
+                             int nkv, int M, int N, int d, float scale, int pos0, int window,
+                             int kv_dtype, const int32_t* block_row, int page, void* stream,
+                             int split_rows) {
+  const int D = prefill_D(d), qb = wide_rows(D);
   PfArgs a{};
   a.q = Qm;
   a.k = K;
@@ -4969,19 +5038,15 @@ static int prefill_wide(const float* Qm, const void* K, const void* V, float* Om
     a.block_table = block_row;
     while ((1 << a.page_shift) < page) ++a.page_shift;
   }
-  a.T0 = window > 0 && pos0 - window + 1 > 0 ? std::min(pos0 - window + 1, N) : 0;
-  a.R = N - a.T0;
-  if (a.R == 0) return zero_out(Om, (int64_t)M * nq * d, (hipStream_t)stream);  // no key attended
-  const size_t need = wide_bytes(nkv, D, np, a.R);
-  if (need > kMaxPiecesBytes) return MOLOT_ENOWS;
   void* pieces = nullptr;
-  int st = pieces_workspace(stream, need, &pieces);
+  int st = pieces32_workspace(nkv, N, d, pos0, window, kv_dtype, stream, &pieces, &a.T0, &a.R);
   if (st) return st;
+  if (a.R == 0) return zero_out(Om, (int64_t)M * nq * d, (hipStream_t)stream);  // no key attended
   a.pieces = reinterpret_cast<const uint16_t*>(pieces);
   const int G = nq / nkv;
   const int64_t nqb = ((int64_t)M * G + qb - 1) / qb;
   a.nqb = (int)nqb;
-  a.nsplit = wide_splits(nqb, nkv, M, N, G, qb, D, pos0, window, nq);
+  a.nsplit = pieces_splits(nqb, nkv, M, N, G, qb, D, kv_dtype == MOLOT_KV_F32, pos0, window, nq);
   if (a.nsplit > 1) {
     unsigned long long* ctr = nullptr;
     void* ws = nullptr;
@@ -4995,14 +5060,17 @@ static int prefill_wide(const float* Qm, const void* K, const void* V, float* Om
     }
   }
   if (nqb * nkv * a.nsplit > (int64_t)0x7FFFFFFF) return MOLOT_ENOTSUP;
-  const int64_t units = wide_padded_rows(a.R) * (D / 8);
-  hipLaunchKernelGGL(prefill_wide_split(D, kv_dtype, block_row != nullptr),
-                     dim3((unsigned)((units + 255) / 256), nkv, 2), dim3(256), 0,
-                     (hipStream_t)stream, a, reinterpret_cast<uint16_t*>(pieces));
-  st = (int)hipGetLastError();
-  if (st) return st;
-  return launch_prefill(prefill_wide_fn(D, kv_dtype), nqb * nkv * a.nsplit, 64 * kWideWaves, a, D,
-                        stream);
+  a.Rsplit = split_rows < 0 ? a.R : std::min(split_rows, a.R);
+  if (a.Rsplit > 0) {
+    const int64_t units = (a.Rsplit == a.R ? wide_padded_rows(a.R) : a.Rsplit) * (D / 8);
+    hipLaunchKernelGGL(prefill_wide_split(D, kv_dtype, block_row != nullptr),
+                       dim3((unsigned)((units + 255) / 256), nkv, 2), dim3(256), 0,
+                       (hipStream_t)stream, a, reinterpret_cast<uint16_t*>(pieces));
+    st = (int)hipGetLastError();
+    if (st) return st;
+  }
+  return launch_prefill(D <= 128 ? prefill_narrow_fn(D, kv_dtype) : prefill_wide_fn(D, kv_dtype),
+                        nqb * nkv * a.nsplit, 64 * kWideWaves, a, D, stream);
 }
 
 // split_rows: rows of [T0, N) pf_split_kernel still has to split (the
@@ -5020,8 +5088,8 @@ static int attn_prefill_impl(const float* Qm, const void* K, const void* V, floa
   // at d.  A Q8 cache at d = 256 runs only through the pieces (the kernel
   // that splits staged Q8 tiles itself is built for 64 and 128).  Head dims
   // above 256 and even ones that are not multiples of 8 run as prefill rows
-  // (prefill_rows), those above 256 on the matrix cores (prefill_wide) where
-  // there is enough work.
+  // (prefill_rows).  Prompts with enough work, at any head dim, take the
+  // 32-row kernels instead (prefill_on_pieces).
   const bool padded = !supported_d(d);
   // Q8 caches at padded dims too (the matrix-core prefill reads whole
   // 16-code chunks of the built dims only)
@@ -5033,18 +5101,11 @@ static int attn_prefill_impl(const float* Qm, const void* K, const void* V, floa
   if (N == 0) return zero_out(Om, (int64_t)M * nq * d, (hipStream_t)stream);
   if (!K || !V || !aligned16(K) || !aligned16(V) || !aligned16(Qm) || !aligned16(Om))
     return MOLOT_EINVAL;
-  // Above 256 on the matrix cores from kWideWork (query head, key) pairs on.
-  // Both sides, 8q/2kv/d512, us a step over fp32 / bf16 / Q8 caches:
-  // (rows, cached) = (64, 500) prefill rows 40 / 40 / 37, matrix cores 44 /
-  // 38 / 38; (8, 4000) 43 / 38 / 37 against 47 / 38 / 41; (24, 4000) 123 /
-  // 117 / 96 against 53 / 44 / 46; (8, 16384) 118 / 94 / 77 against 92 / 64
-  // / 61; (2, 16384) 63 / 41 / 36 against 89 / 60 / 58.
-  constexpr int64_t kWideWork = 400000;
-  const int64_t span = window > 0 && window < N ? window : N;
-  if (d > 256 && M <= 65535 && (int64_t)M * nq * span >= kWideWork) {
-    st = prefill_wide(Qm, K, V, Om, nq, nkv, M, N, d, scale, pos0, window, kv_dtype, block_row,
-                      page, stream);
+  if (prefill_takes_pieces(d, M, N, nq, window)) {
+    st = prefill_on_pieces(Qm, K, V, Om, nq, nkv, M, N, d, scale, pos0, window, kv_dtype, block_row,
+                           page, stream, split_rows);
     if (st != MOLOT_ENOWS) return st;
+    split_rows = -1;
   }
   if (rows_path)
     return prefill_rows(Qm, K, V, Om, nq, nkv, M, N, d, scale, pos0, window, kv_dtype, block_row,
@@ -5079,7 +5140,6 @@ static int attn_prefill_impl(const float* Qm, const void* K, const void* V, floa
     pw = 4;  // no split: twice the workgroups on 4 waves
     nqb = nqb_of(4);
   }
-  const int pf_threads = 64 * pw;
   if (nqb * nkv * nsplit > (int64_t)0x7FFFFFFF) return MOLOT_ENOTSUP;
   PfArgs a{};
   a.q = Qm;
@@ -5106,12 +5166,14 @@ static int attn_prefill_impl(const float* Qm, const void* K, const void* V, floa
   }
   PfFn pk = pieces_only ? nullptr : pf_kernel(D, kv_dtype, block_row != nullptr, pw);
   if (!pk && !pieces_only) return MOLOT_ENOTSUP;
-  // fp32 and Q8 caches: split the attended keys into 16-bit pieces once
-  // (pf_split_kernel), and let the attention kernel copy them into LDS.
-  // Every query attends keys in [t0(query 0), N).  Not under stream capture
-  // when the workspace would have to grow, nor past kMaxPiecesBytes: the
-  // kernel then splits each staged tile itself.
-  {
+  // fp32 and Q8 caches: the attended keys as 16-bit pieces, which the
+  // attention kernel copies into LDS, where a fresh prompt's step wrote them
+  // (split_rows = 0), and at d = 256, split here.  Not under stream capture
+  // when the workspace would have to grow, nor past kMaxPiecesBytes, nor at
+  // d <= 128 after cached rows (a prompt too small for prefill_on_pieces:
+  // 16 rows after 2000 of 32q/8kv/d128 fp32 take 36 us with the split, 29
+  // without): the kernel then splits each staged tile itself.
+  if (D == 256 || split_rows == 0) {
     void* ws = nullptr;
     int T0 = 0;
     int64_t R = 0;
@@ -5131,7 +5193,7 @@ static int attn_prefill_impl(const float* Qm, const void* K, const void* V, floa
       a.Rsplit = split_rows < 0 ? (int)R : (int)std::min<int64_t>(split_rows, R);
       if (a.Rsplit > 0) {
         const int64_t units = (int64_t)a.Rsplit * (D / 8);
-        hipLaunchKernelGGL(pf_split(D, kv_dtype, block_row != nullptr),
+        hipLaunchKernelGGL(pf_split(kv_dtype, block_row != nullptr),
                            dim3((unsigned)((units + 255) / 256), nkv, 2), dim3(256), 0,
                            (hipStream_t)stream, a, reinterpret_cast<uint16_t*>(ws));
         st = (int)hipGetLastError();
@@ -5140,6 +5202,7 @@ static int attn_prefill_impl(const float* Qm, const void* K, const void* V, floa
       pk = pf_kernel_pre(D, pw);
     }
   }
+  const int pf_threads = 64 * pw;
   return launch_prefill(pk, nqb * nkv * nsplit, pf_threads, a, D, stream);
 }
 
@@ -5206,18 +5269,31 @@ static int prefill_step_impl(float* q, const float* k_new, const float* v_new, v
   // fp32 252 -> 249 us, 8q/4kv/d256 window 1024 164.7 -> 161.6 us)
   void* pws = nullptr;
   int T0 = 0;
-  int64_t R = 0;
   int split_rows = -1;
-  if (supported_d(d)) {
+  if (prefill_takes_pieces(d, M, slot0 + M, nq, window)) {
+    // at d = 512 the split of all rows is as fast (8q/2kv, 1999 tokens: 29 + 7
+    // us against 49 for a RoPE/append that leaves the pieces)
+    if (d == 64 || d == 128) {
+      int R = 0;
+      st = pieces32_workspace(nkv, slot0 + M, d, pos0, window, kv_dtype, stream, &pws, &T0, &R);
+      if (st && st != MOLOT_ENOWS) return st;
+      if (!st) {
+        r.pc_R = R;
+        r.pc_np = wide_pieces(kv_dtype == MOLOT_KV_F32);
+      }
+    }
+  } else if (supported_d(d)) {
+    int64_t R = 0;
     st = prefill_pieces(nkv, slot0 + M, d, pos0, window, kv_dtype, stream, &pws, &T0, &R,
                         pieces_only);
     if (st) return st;
-    if (pws) {
-      r.pieces = reinterpret_cast<uint16_t*>(pws);
-      r.pc_T0 = T0;
-      r.pc_R = (int)R;
-      split_rows = std::max(0, slot0 - T0);
-    }
+    r.pc_R = (int)R;
+    if (d <= 128 && slot0 > T0) pws = nullptr;  // cached rows attended: split per tile
+  }
+  if (pws) {
+    r.pieces = reinterpret_cast<uint16_t*>(pws);
+    r.pc_T0 = T0;
+    split_rows = std::max(0, slot0 - T0);
   }
   st = launch_rope_tok(r, M, stream);
   if (st) return st;

@@ -346,18 +346,28 @@ typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 // V reads of the other tile buffer), which waited for the next tile's copies
 // halfway through every tile.  The kernel orders the copies itself
 // (wait_vmcnt, then a barrier, before a buffer is read).  m0 takes the LDS
-// address as an input operand (the compiler writes it); one wait state
-// between that write and the copy.
+// address as an input operand (the compiler writes it).  Five wait states
+// (s_nop 4) go before the copy: one after the write of m0, five where a
+// vector instruction (v_readfirstlane) wrote the scalar base, a hazard that
+// the compiler does not resolve inside inline assembly.
 __device__ __forceinline__ void dma16(const void* base, uint32_t off, uint32_t lds) {
-  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, %1"
+  asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %0, %1"
                :
                : "v"(off), "s"(base), "{m0}"(lds)
                : "memory");
 }
-// The same with 4 bytes a lane (global_load_lds_dword): lane l's 4 bytes
+// A wave-uniform address, in scalar registers whatever formed it.
+template <typename P>
+__device__ __forceinline__ const P* uniform_ptr(const P* p) {
+  const uint64_t u = (uint64_t)p;
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)u);
+  const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(u >> 32));
+  return (const P*)((uint64_t)hi << 32 | lo);
+}
+// dma16 with 4 bytes a lane (global_load_lds_dword): lane l's 4 bytes
 // land at LDS address lds + 4*l.
 __device__ __forceinline__ void dma4(const void* base, uint32_t off, uint32_t lds) {
-  asm volatile("s_nop 0\n\tglobal_load_lds_dword %0, %1"
+  asm volatile("s_nop 4\n\tglobal_load_lds_dword %0, %1"
                :
                : "v"(off), "s"(base), "{m0}"(lds)
                : "memory");

@@ -5,8 +5,7 @@
 // the group), as in prefill_mfma16_kernel.  A workgroup of 8 waves owns
 // 32 * RG of them: wave (rg, sl) takes row group rg and the SL = 128
 // elements sl*128 .. of the head dim, for the scores and for the output.
-//   D = 512: 2 row groups x 4 slices, 64 rows;
-//   D = 256: 4 row groups x 2 slices, 128 rows.
+// (D = 512: 2 row groups x 4 slices, 64 rows).
 // Per tile of 32 keys:
 //   1. every wave forms its slice's share of S^T = K . Q^T on
 //      v_mfma_f32_32x32x16_f16 (A = K from LDS, B = its q pieces in
@@ -57,7 +56,8 @@ __global__ __launch_bounds__(256) void wide_split_kernel(PfArgs a, uint16_t* out
   constexpr int UPR = D / 8;
   const int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x;
   const int64_t Rp = wide_padded_rows(a.R);
-  if (u >= Rp * UPR) return;
+  // rows [0, Rsplit), and with the last of them the tail
+  if (u >= (a.Rsplit == a.R ? Rp : (int64_t)a.Rsplit) * UPR) return;
   const int h = blockIdx.y, kv = blockIdx.z;
   const int64_t r = u / UPR;
   const int j = (int)(u - r * UPR);
@@ -505,10 +505,15 @@ SplitFn split_of(bool paged) {
 }  // namespace
 
 SplitFn prefill_wide_split(int D, int kv_dtype, bool paged) {
-  if (D != 512) return nullptr;
-  if (kv_dtype == MOLOT_KV_Q8) return split_of<512, q8_t>(paged);
-  if (kv_dtype == MOLOT_KV_BF16) return split_of<512, bf16_t>(paged);
-  return split_of<512, float>(paged);
+  auto of = [&](auto d) -> SplitFn {
+    constexpr int N = decltype(d)::value;
+    if (kv_dtype == MOLOT_KV_Q8) return split_of<N, q8_t>(paged);
+    if (kv_dtype == MOLOT_KV_BF16) return split_of<N, bf16_t>(paged);
+    return split_of<N, float>(paged);
+  };
+  if (D == 64) return of(std::integral_constant<int, 64>{});
+  if (D == 128) return of(std::integral_constant<int, 128>{});
+  return of(std::integral_constant<int, 512>{});
 }
 
 PfFn prefill_wide_fn(int D, int kv_dtype) {

@@ -1,4 +1,4 @@
-// Interface of prefill_wide.hip (the wide-head-dim prefill).
+// Interface of prefill_wide.hip and prefill_narrow.hip.
 #ifndef MOLOT_AMD_CSRC_PREFILL_WIDE_HPP_
 #define MOLOT_AMD_CSRC_PREFILL_WIDE_HPP_
 
@@ -10,7 +10,7 @@
 #include "prefill.hpp"
 
 constexpr int kWideTile = 32;  // keys a tile
-constexpr int kWideTail = 32;  // rows of zeros after a head's pieces (the last tile's overrun)
+constexpr int kWideTail = 64;  // rows of zeros after a head's pieces (two tiles' overrun)
 constexpr int kWideWaves = 8;
 
 // fp16 pieces of a cached value: two for fp32, one for bf16 and Q8 rows.
@@ -19,7 +19,7 @@ constexpr int wide_pieces_v = sizeof(T) == 4 ? 2 : 1;
 inline int wide_pieces(bool f32) { return f32 ? 2 : 1; }
 
 // Query rows of a workgroup.
-constexpr int wide_rows(int D) { return 32 * (kWideWaves / (D / 128)); }
+constexpr int wide_rows(int D) { return D <= 128 ? 128 : 64; }
 
 // Workspace of R attended rows, per K and V and KV head: [pieces][Rp][D] fp16,
 // then the rows' units [Rp] floats (Rp rows: the tail, and heads stay 16-byte
@@ -34,6 +34,9 @@ inline size_t wide_bytes(int nkv, int D, int np, int64_t R) {
   return (size_t)2 * nkv * wide_head_elems(D, np, wide_padded_rows(R)) * sizeof(uint16_t);
 }
 
+// The split of the cached rows, and the attention kernels over the pieces:
+// prefill_narrow.hip (D = 64 and 128), prefill_wide.hip (D = 512).
+PfFn prefill_narrow_fn(int D, int kv_dtype) __attribute__((visibility("hidden")));
 SplitFn prefill_wide_split(int D, int kv_dtype, bool paged) __attribute__((visibility("hidden")));
 PfFn prefill_wide_fn(int D, int kv_dtype) __attribute__((visibility("hidden")));
 
