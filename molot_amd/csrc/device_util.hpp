@@ -346,13 +346,17 @@ typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 // V reads of the other tile buffer), which waited for the next tile's copies
 // halfway through every tile.  The kernel orders the copies itself
 // (wait_vmcnt, then a barrier, before a buffer is read).  m0 takes the LDS
-// address as an input operand (the compiler writes it).  Five wait states
-// (s_nop 4) go before the copy: one after the write of m0, five where a
-// vector instruction (v_readfirstlane) wrote the scalar base, a hazard that
-// the compiler does not resolve inside inline assembly.
+// address as an input operand (the compiler writes it).  The scalar base goes
+// through an s_mov_b64 of the same statement: where a vector instruction
+// (v_readfirstlane) wrote it, a vector memory instruction may read it only
+// five wait states later, a hazard the compiler does not resolve inside inline
+// assembly, while a scalar instruction's read is interlocked and its result
+// has no such hazard.  It is also the wait state between the write of m0 and
+// the copy.
 __device__ __forceinline__ void dma16(const void* base, uint32_t off, uint32_t lds) {
-  asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %0, %1"
-               :
+  const void* b;
+  asm volatile("s_mov_b64 %0, %2\n\tglobal_load_lds_dwordx4 %1, %0"
+               : "=&s"(b)
                : "v"(off), "s"(base), "{m0}"(lds)
                : "memory");
 }
@@ -367,8 +371,9 @@ __device__ __forceinline__ const P* uniform_ptr(const P* p) {
 // dma16 with 4 bytes a lane (global_load_lds_dword): lane l's 4 bytes
 // land at LDS address lds + 4*l.
 __device__ __forceinline__ void dma4(const void* base, uint32_t off, uint32_t lds) {
-  asm volatile("s_nop 4\n\tglobal_load_lds_dword %0, %1"
-               :
+  const void* b;
+  asm volatile("s_mov_b64 %0, %2\n\tglobal_load_lds_dword %1, %0"
+               : "=&s"(b)
                : "v"(off), "s"(base), "{m0}"(lds)
                : "memory");
 }
