@@ -540,7 +540,14 @@ struct AttnArgs {
   // one cache (contiguous, or the prompt's block-table row: max_blocks = 0),
   // t0_b from the window (include/molot/gemm.h:409-446).
   int pf;
-  int nseq;              // chunk_fast: sequences of the launch
+  int nseq;              // chunk_fast, dyn: sequences of the launch
+  // Paged matrix-core launches: the rows a chunk takes follow the sequences'
+  // lengths (paged_chunk), so that about dyn workgroups have work (0: chunk
+  // as given).  chunk then bounds it from above (the LDS layout), nchunks from
+  // the least chunk, and the grid is flat over the (sequence, chunk) pairs.
+  int dyn;
+  int dyn_pairs;         // host side: pairs the grid holds, and the least chunk
+  int dyn_min;
   // In-launch merge (see arrive_and_merge): every chunk of a slot runs on one
   // XCD, and the workgroup that completes a slot merges its chunk partials.
   int fold;              // ROPE: 1 = the step appends the new token (folded into the last
@@ -1877,6 +1884,78 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
 typedef short i16x4_t __attribute__((ext_vector_type(4)));
 
+// ---------------------------------------------------------------------------
+// Chunks of a paged batch on the matrix-core kernel.  The host knows only the
+// longest sequence; a chunk sized from that left a batch of uneven lengths
+// with either a second round of workgroups (two fit a CU) or a few long
+// chunks.  Each wave instead sums the lengths (a load a lane, with the one it
+// needs anyway) and takes the chunk that gives the launch's `target`
+// workgroups, two a CU, in whole rounds of the 4 waves' 32-row tiles.
+// Batches with more than kDynLong rows a chunk then need several rounds and
+// take kDynRound rows (or, of short sequences, one chunk each).
+// us a step, 32q/8kv/d128, chunks from the longest sequence against these: Q8
+// 13 sequences of 1 .. 2999 rows 27.9 against 19.4; 2 of 3000 and 8000 31.4
+// against 16.1; 20 of 31 .. 447 18.7 against 14.1; 64 of 100 .. 1000 32.9
+// against 23.3; bf16 7 of 136 .. 2731 26.1 against 19.0; 2 of 3000 and 8000
+// 49.3 against 19.2; 64 of 100 .. 1000 51.1 against 37.0; 32 of 512 .. 4096
+// 76.0 against 72.3.
+constexpr int kDynUnit = 128, kDynLong = 1024, kDynRound = 768, kDynMax = 2048;
+__host__ __device__ constexpr int dyn_chunk(int rows, int nseq, int heads, int target) {
+  const int den = target - nseq * heads;  // workgroups beyond one a (sequence, head)
+  const int c = den > 0 ? (rows * heads + den - 1) / den : kDynMax;
+  if (den > 0 && c <= kDynLong) return c <= kDynUnit ? kDynUnit : (c + kDynUnit - 1) / kDynUnit * kDynUnit;
+  return rows > kDynLong * nseq ? kDynRound : kDynMax;
+}
+// The least it can give while the longest sequence has `span` rows.
+constexpr int dyn_chunk_min(int span, int nseq, int heads, int target) {
+  const int den = target - nseq * heads;
+  const int c = den > 0 ? (span * heads + den - 1) / den : kDynMax;
+  if (c > kDynLong && span <= kDynLong) return kDynMax;
+  const int r = c <= kDynUnit ? kDynUnit : (c + kDynUnit - 1) / kDynUnit * kDynUnit;
+  return r < kDynRound ? r : kDynRound;
+}
+// A sequence's rows and query position, and the cache rows it attends.
+struct SeqLen {
+  int n = 0, pos = -1;
+};
+__device__ __forceinline__ SeqLen seq_len(const int32_t* seq_lens, const int32_t* pos_arr, int b,
+                                          int nseq) {
+  SeqLen s;
+  if (b < nseq) {
+    s.n = seq_lens[b];
+    s.pos = pos_arr ? pos_arr[b] : s.n - 1;
+  }
+  return s;
+}
+__device__ __forceinline__ int seq_span(SeqLen s, int window, bool fold) {
+  int t0 = (window > 0 && s.pos - window + 1 > 0) ? s.pos - window + 1 : 0;
+  if (t0 > s.n) t0 = s.n;
+  return max((fold ? s.n - 1 : s.n) - t0, 0);
+}
+// Inclusive sum over the lanes up to this one (row shifts, then row
+// broadcasts of the rows before).
+__device__ __forceinline__ int wave_scan(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);
+  return x;
+}
+// The launch's chunk (wave-uniform; every lane of the wave takes part).
+// first: sequence (lane)'s, loaded by the caller.
+__device__ __forceinline__ int paged_chunk(const int32_t* seq_lens, const int32_t* pos_arr,
+                                           SeqLen first, int nseq, int window, bool fold,
+                                           int heads, int target) {
+  const int lane = threadIdx.x & 63;
+  int rows = lane < nseq ? seq_span(first, window, fold) : 0;
+  for (int b = lane + 64; b < nseq; b += 64)
+    rows += seq_span(seq_len(seq_lens, pos_arr, b, nseq), window, fold);
+  rows = __builtin_amdgcn_readlane(wave_scan(rows), 63);
+  return dyn_chunk(rows, nseq, heads, target);
+}
+
 constexpr int kMfmaWaves = 4;                  // waves per workgroup
 constexpr int kMfmaThreads = kMfmaWaves * 64;
 constexpr int kTile = 32;                      // cache rows per wave step
@@ -2014,7 +2093,46 @@ __global__ __launch_bounds__(kMfmaThreads, 2) void attn_mfma_kernel(AttnArgs a) 
   const int G = a.nq / a.nkv;
   const int nsub = G / GH;
   int z, hs, b;
-  if (a.chunk_fast) {  // workgroup id runs on XCD id % 8 (launch_pair)
+  int chunk = a.chunk;
+  int sn = 0, spos = 0;  // dyn: the sequence's length and position
+  if (PAGED && a.dyn) {
+    // flat over the (sequence, chunk) pairs (at least one a sequence), the
+    // sequences in order; Q8: all heads of a pair on one XCD, as below
+    const int HS = a.nkv * nsub;
+    const bool fold = ROPE && a.fold;
+    SeqLen sl = seq_len(a.seq_lens, a.pos_arr, (int)(threadIdx.x & 63), a.nseq);
+    chunk = paged_chunk(a.seq_lens, a.pos_arr, sl, a.nseq, a.window, fold, HS, a.dyn);
+    const int id = (int)blockIdx.x;
+    int pi;
+    if (Q8) {
+      const int k = id >> 3;
+      pi = (k / HS) * 8 + (id & 7);
+      hs = k % HS;
+    } else {
+      pi = id / HS;
+      hs = id % HS;
+    }
+    b = -1;
+    z = 0;
+    for (int b0 = 0; b0 < a.nseq; b0 += 64) {
+      const int bl = b0 + (int)(threadIdx.x & 63);
+      if (b0) sl = seq_len(a.seq_lens, a.pos_arr, bl, a.nseq);
+      const int cnt =
+          bl < a.nseq ? max(1, (seq_span(sl, a.window, fold) + chunk - 1) / chunk) : 0;
+      const int upto = wave_scan(cnt);
+      const uint64_t past = __builtin_amdgcn_ballot_w64(upto > pi);
+      if (past) {  // the first lane whose pairs reach past pi
+        const int l = __builtin_ctzll(past);
+        b = b0 + l;
+        z = pi - (__builtin_amdgcn_readlane(upto, l) - __builtin_amdgcn_readlane(cnt, l));
+        sn = __builtin_amdgcn_readlane(sl.n, l);
+        spos = __builtin_amdgcn_readlane(sl.pos, l);
+        break;
+      }
+      pi -= __builtin_amdgcn_readlane(upto, 63);
+    }
+    if (b < 0) return;  // past the last pair
+  } else if (a.chunk_fast) {  // workgroup id runs on XCD id % 8 (launch_pair)
     const int HS = a.nkv * nsub;
     const int k = (int)(blockIdx.x >> 3);
     // (sequence, chunk) pair pi = (k / HS) * 8 + id % 8, chunk slot slowest;
@@ -2044,8 +2162,8 @@ __global__ __launch_bounds__(kMfmaThreads, 2) void attn_mfma_kernel(AttnArgs a) 
 
   int n = a.n, t0 = a.t0, pos = a.pos;
   if constexpr (PAGED) {
-    n = a.seq_lens[b];
-    pos = a.pos_arr ? a.pos_arr[b] : n - 1;
+    n = a.dyn ? sn : a.seq_lens[b];
+    pos = a.dyn ? spos : a.pos_arr ? a.pos_arr[b] : n - 1;
     t0 = (a.window > 0 && pos - a.window + 1 > 0) ? pos - a.window + 1 : 0;
     if (t0 > n) t0 = n;
   }
@@ -2054,7 +2172,7 @@ __global__ __launch_bounds__(kMfmaThreads, 2) void attn_mfma_kernel(AttnArgs a) 
   int nch = a.nchunks;
   if constexpr (PAGED) {
     const int span = cend - t0;
-    nch = span > 0 ? (span + a.chunk - 1) / a.chunk : (fold ? 1 : 0);
+    nch = span > 0 ? (span + chunk - 1) / chunk : (fold ? 1 : 0);
     if (nch > a.nchunks) nch = a.nchunks;
   }
   if (z >= nch) {
@@ -2065,8 +2183,8 @@ __global__ __launch_bounds__(kMfmaThreads, 2) void attn_mfma_kernel(AttnArgs a) 
     return;
   }
   const int c = nch - 1 - z;  // the new token's chunk first, as in attn_kernel
-  const int tb = t0 + c * a.chunk;
-  const int cntg = max(0, min(a.chunk, cend - tb));
+  const int tb = t0 + c * chunk;
+  const int cntg = max(0, min(chunk, cend - tb));
   const bool is_new = fold && c == nch - 1;
   const bool split = nch > 1;
   const int64_t slot = (int64_t)b * a.nkv * nsub + hs;
@@ -3332,6 +3450,7 @@ struct CombArgs {
   int dh;    // head dim as stored (d: the partials' padded head dim)
   int pf, pos0, n;  // prefill rows (AttnArgs::pf): row b at pos0 + b of a cache of n rows
   int pairs;        // combine_kernel: output pairs per workgroup (16, 32 or 64)
+  int dyn, nseq;    // AttnArgs::dyn: the chunk from the sequences' lengths
 };
 
 // Chunks of sequence b of a per-sequence launch (a paged batch, or prefill
@@ -3348,7 +3467,13 @@ __device__ __forceinline__ int comb_chunks(const CombArgs& a, int b) {
   int t0 = (a.window > 0 && pos - a.window + 1 > 0) ? pos - a.window + 1 : 0;
   if (t0 > n) t0 = n;
   const int span = (a.fold ? n - 1 : n) - t0;
-  const int nch = span > 0 ? (span + a.chunk - 1) / a.chunk : (a.fold ? 1 : 0);
+  int chunk = a.chunk;
+  if (a.dyn) {
+    const SeqLen first = seq_len(a.seq_lens, a.pos_arr, (int)(threadIdx.x & 63), a.nseq);
+    chunk = paged_chunk(a.seq_lens, a.pos_arr, first, a.nseq, a.window, a.fold, a.nkv * a.nsub,
+                        a.dyn);
+  }
+  const int nch = span > 0 ? (span + chunk - 1) / chunk : (a.fold ? 1 : 0);
   return nch > a.nchunks ? a.nchunks : nch;
 }
 
@@ -3877,7 +4002,21 @@ int plan_launch(AttnArgs& a, int d, int span, int gh, int nsubs, int B, int alig
     nch = std::max(1L, std::min({nch, tiles, (long)kMaxChunks}));
     a.nchunks = (int)nch;
     a.chunk = (int)((tiles + nch - 1) / nch * align);
+  } else if (a.dyn && split <= 0 && wpcu <= 0 && span > 0 &&
+             (int64_t)B * span * a.nkv * nsubs < ((int64_t)1 << 30) &&
+             span <= kMaxChunks * dyn_chunk_min(span, B, a.nkv * nsubs, a.dyn)) {
+    const int hs = a.nkv * nsubs;
+    const int cmin = dyn_chunk_min(span, B, hs, a.dyn);
+    a.chunk = kDynMax;
+    a.dyn_min = cmin;
+    a.nchunks = (span + cmin - 1) / cmin;
+    // the pairs' bound: the target's (total / chunk + one a sequence), or of
+    // kDynRound rows a chunk
+    const int64_t rounds = (int64_t)B * ((span + kDynRound - 1) / kDynRound);
+    a.dyn_pairs = (int)std::min<int64_t>((int64_t)B * a.nchunks,
+                                         std::max<int64_t>(a.dyn / hs + 1, rounds));
   } else {
+    a.dyn = 0;
     a.chunk = plan_chunk(span > 0 ? span : 1, rows, align, wpc, split, wpcu);
     a.nchunks = span > 0 ? (span + a.chunk - 1) / a.chunk : 1;
     // bound the chunk count (grid x, and the combine's per-pair loop)
@@ -3962,7 +4101,7 @@ int launch_pair(AttnFn kern, int threads, size_t lds, AttnArgs a, int gh, int d,
   if (lds > kMaxLds) return (int)hipErrorInvalidConfiguration;
   if ((gh * d) % kCombPairs || d % kCombPairs) return MOLOT_ENOTSUP;  // combine tiling
   t_last_nchunks = a.nchunks;
-  t_last_chunk = a.chunk;
+  t_last_chunk = a.dyn ? a.dyn_min : a.chunk;
   a.dynamic = knob(g_dynamic);
   std::lock_guard<std::mutex> plk(g_prof_mu);
   const bool prof = !a.ext_ws && prof_active(stream);
@@ -3986,7 +4125,10 @@ int launch_pair(AttnFn kern, int threads, size_t lds, AttnArgs a, int gh, int d,
   // xmap (in-launch merge, fewer than 8 slots): a 1-D grid of 8 * nchunks
   // workgroups, id running chunk slot id / 8 of slot id % 8, so each slot's
   // chunks share an XCD; ids of absent slots exit at once.
-  const dim3 grid = a.chunk_fast
+  const int64_t dheads = (int64_t)a.nkv * nsubs;
+  const dim3 grid = a.dyn ? dim3((unsigned)((a.chunk_fast ? (a.dyn_pairs + 7) / 8 * 8 : a.dyn_pairs) *
+                                            dheads), 1, 1)
+                    : a.chunk_fast
                         ? dim3((unsigned)(((int64_t)B * a.nchunks + 7) / 8 * 8 * a.nkv * nsubs), 1, 1)
                         : a.xmap ? dim3((unsigned)(8 * a.nchunks), 1, 1)
                                  : dim3(a.nkv * nsubs, B, a.nchunks);
@@ -4026,6 +4168,8 @@ int launch_pair(AttnFn kern, int threads, size_t lds, AttnArgs a, int gh, int d,
   cb.pf = rope ? 0 : a.pf;
   cb.pos0 = a.pos;
   cb.n = a.n;
+  cb.dyn = a.dyn;
+  cb.nseq = a.nseq;
   // At most 8 chunks (batches of sequences: many slots, few chunks): one
   // wave per 64 pairs (combine_wave_kernel<R>, R = 4 or 8 o loads per lane).
   // More chunks: combine_kernel, whose 4 phases per pair keep the loads per
@@ -4099,6 +4243,13 @@ int launch_mfma(AttnArgs a, int span, int nsubs, int B, void* stream) {
   constexpr int kWpc = PAGED ? (Q8 ? 8 : 16) : 1;
   a.chunk_fast = Q8;
   a.nseq = B;
+  // two workgroups fit a CU; the in-launch merge needs a slot's chunks on one XCD
+  // (nor for long sequences that fill the chip whatever their chunks: 64
+  // sequences of 512 .. 8192 rows, bf16: 215.0 against 216.6 us)
+  const int fit = 2 * num_cus();
+  if (PAGED && !a.pf && !a.ext_ws && knob(g_merge) <= 0 &&
+      ((int64_t)B * a.nkv * nsubs < fit || span <= kDynMax))
+    a.dyn = fit;
   int st = plan_launch(a, D, span, GH, nsubs, B, kTile, kWpc, stream, !PAGED);
   if (st) return st;
   // by default the combine kernel: its four waves per workgroup would fold
