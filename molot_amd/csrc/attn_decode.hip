@@ -548,6 +548,7 @@ struct AttnArgs {
   int dyn;
   int dyn_pairs;         // host side: pairs the grid holds, and the least chunk
   int dyn_min;
+  int matrix, brief;     // host side: the matrix-core kernel; a short context (kBriefSpan)
   // In-launch merge (see arrive_and_merge): every chunk of a slot runs on one
   // XCD, and the workgroup that completes a slot merges its chunk partials.
   int fold;              // ROPE: 1 = the step appends the new token (folded into the last
@@ -3985,6 +3986,20 @@ int plan_chunk(int span, int rows_of_wgs, int align, int wpc, int split, int wpc
 // puts slot s on XCD s (xmap).  Other slot counts, token-major Q8 launches
 // (whose grid groups the heads of a chunk on one XCD instead) and slots of
 // more than kMergeMaxChunks chunks use combine_kernel.
+// Short contexts of one sequence: an eager step of two dependent launches
+// costs more than it computes, so up to kOneChunkSpan rows one workgroup a slot
+// takes the context, and up to kBriefSpan at most 16 chunks a slot (the
+// matrix-core kernel past 512 rows: 128, a tile a wave) are merged in the
+// launch, on 4 XCDs or more.  The vector-ALU kernel only to kBriefWork rows *
+// outputs a slot (its merge folds more the longer), and not over Q8, whose
+// heads share an XCD a chunk.  us an eager step at 60 / 300 / 900 / 2040 rows,
+// the combine kernel against these: 32q/8kv/d128 fp32 8.2, 9.1, 9.5, 10.4
+// against 6.8, 8.0, 8.9, (11.0); bf16 9.6, 10.3, 10.8, 10.9 against 7.3, 9.2,
+// 9.2, 9.9; Q8 10.3, 11.2, 11.5, 11.8 against 7.8, 9.8, 9.8, 10.3; 64q/8kv/d128
+// fp32 9.8, 10.6, 11.0, 13.2 against 9.5, 9.8, (12.1), (15.4); 8q/4kv/d256 fp32
+// 7.9, 8.7, 9.5 against 6.4, 8.2, 9.5.
+constexpr int kOneChunkSpan = 64, kBriefSpan = 2048;
+constexpr long kBriefWork = 1 << 19;
 int plan_launch(AttnArgs& a, int d, int span, int gh, int nsubs, int B, int align, int wpc,
                 void* stream, bool cyclic = false) {
   const int rows = a.nkv * nsubs * B;
@@ -3998,6 +4013,15 @@ int plan_launch(AttnArgs& a, int d, int span, int gh, int nsubs, int B, int alig
     } else {
       const long target = (long)(wpcu > 0 ? wpcu : wpc) * num_cus();
       nch = (target + rows - 1) / rows;
+      if (wpcu <= 0 && d <= 256 && span <= kOneChunkSpan) {
+        nch = 1;
+      } else if (wpcu <= 0 && d <= 256 && span <= kBriefSpan && knob(g_merge) < 0 &&
+                 (rows % 8 == 0 || (rows >= 4 && rows < 8)) &&
+                 (a.matrix || (!a.chunk_fast && (long)span * gh * d <= kBriefWork))) {
+        a.brief = 1;
+        if (a.matrix) a.chunk_fast = 0;  // a slot's chunks on one XCD instead
+        nch = std::min(nch, a.matrix && span > 512 ? (span + 127L) / 128 : 16L);
+      }
     }
     nch = std::max(1L, std::min({nch, tiles, (long)kMaxChunks}));
     a.nchunks = (int)nch;
@@ -4066,7 +4090,7 @@ int plan_launch(AttnArgs& a, int d, int span, int gh, int nsubs, int B, int alig
   // keeps the combine kernel (launch_mfma).
   const int mk = knob(g_merge);
   const bool want =
-      mk > 0 || (mk < 0 && rows % 8 == 0 && !a.block_table && span >= kMergeAutoSpan);
+      mk > 0 || (mk < 0 && (a.brief || (rows % 8 == 0 && !a.block_table && span >= kMergeAutoSpan)));
   const bool merge = want && !a.chunk_fast && (rows % 8 == 0 || rows < 8) &&
                      a.nchunks <= kMergeMaxChunks && hipGetDevice(&dev) == hipSuccess &&
                      xcd_ok_cached(dev);
@@ -4242,19 +4266,23 @@ template <int D, int GH, bool PAGED, bool ROPE, bool Q8>
 int launch_mfma(AttnArgs a, int span, int nsubs, int B, void* stream) {
   constexpr int kWpc = PAGED ? (Q8 ? 8 : 16) : 1;
   a.chunk_fast = Q8;
+  a.matrix = 1;
   a.nseq = B;
   // two workgroups fit a CU; the in-launch merge needs a slot's chunks on one XCD
   // (nor for long sequences that fill the chip whatever their chunks: 64
-  // sequences of 512 .. 8192 rows, bf16: 215.0 against 216.6 us)
+  // sequences of 512 .. 8192 rows, bf16: 215.0 against 216.6 us; nor for
+  // batches that fit in one round of single tiles: 7 of 13 .. 192, 64q, bf16:
+  // 10.8 against 11.4)
   const int fit = 2 * num_cus();
-  if (PAGED && !a.pf && !a.ext_ws && knob(g_merge) <= 0 &&
-      ((int64_t)B * a.nkv * nsubs < fit || span <= kDynMax))
+  const int64_t slots = (int64_t)B * a.nkv * nsubs;
+  if (PAGED && !a.pf && !a.ext_ws && knob(g_merge) <= 0 && (slots < fit || span <= kDynMax) &&
+      slots * ((span + kTile - 1) / kTile) > fit)
     a.dyn = fit;
   int st = plan_launch(a, D, span, GH, nsubs, B, kTile, kWpc, stream, !PAGED);
   if (st) return st;
   // by default the combine kernel: its four waves per workgroup would fold
   // the chunks in sequential rounds (c5: 111.7 against 99.5 us per step)
-  if (knob(g_merge) < 0) no_merge(a);
+  if (knob(g_merge) < 0 && !a.brief) no_merge(a);
   if (a.mrg && sizeof(float) * (size_t)LdsM(D, GH, a.chunk, a.page_shift, PAGED, Q8, a.mrg).total >
                    kMaxLds)
     no_merge(a);

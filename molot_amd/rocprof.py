@@ -29,14 +29,19 @@ import sys
 from collections import defaultdict
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
-KERNEL_SOURCE = os.path.join(ROOT, "molot_amd", "csrc", "attn_decode.hip")
+KERNEL_SOURCES = [os.path.join(ROOT, "molot_amd", "csrc", f)
+                  for f in sorted(os.listdir(os.path.join(ROOT, "molot_amd", "csrc")))
+                  if f.endswith((".hip", ".hpp")) and f != "probe.hip"]
 COPY_BYTES = 1 << 30  # bench.py --pmc-run: molot_probe_copy of 1 GiB
 
 
 def source_hash() -> str:
-    """sha256 (first 16 hex digits) of the kernel source a measurement belongs to."""
-    with open(KERNEL_SOURCE, "rb") as f:
-        return hashlib.sha256(f.read()).hexdigest()[:16]
+    """sha256 (first 16 hex digits) of the kernel sources a measurement belongs to."""
+    h = hashlib.sha256()
+    for path in KERNEL_SOURCES:
+        with open(path, "rb") as f:
+            h.update(f.read())
+    return h.hexdigest()[:16]
 
 
 def short_name(name: str, width: int = 110) -> str:
@@ -62,7 +67,7 @@ def _cmd_block(cmds) -> str:
 
 
 def _source_line() -> str:
-    return (f"Kernel source: `molot_amd/csrc/attn_decode.hip`, sha256[:16] `{source_hash()}` "
+    return (f"Kernel sources: `molot_amd/csrc/*.hip, *.hpp`, sha256[:16] `{source_hash()}` "
             "(the tree the summary was written from).\n")
 
 
