@@ -790,7 +790,7 @@ def run_prefill(args, cfg, lib, L, torch, np):
                                       ctypes.byref(nc)), "profile_end")
     k_us = am.value / max(1, na.value) * 1e3
     achieved = flops / (k_us * 1e-6) / 1e12
-    kname = "prefill_mfma16_kernel"
+    kname = "prefill_narrow_kernel" if d <= 128 else "prefill_mfma16_kernel"
     log(args, f"{kname} {k_us:.1f} us/launch -> {achieved:.1f} TFLOP/s")
     out = {
         "metric": "prefill attention TFLOP/s (causal, 4*d flops per head x query x key)",

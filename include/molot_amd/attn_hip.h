@@ -318,7 +318,10 @@ int molot_hip_prob_exp(const float* x, float* y, int64_t n, void* stream);
 /* Split-K chunk size in tokens (0 = automatic). */
 void molot_hip_set_split_chunk(int tokens);
 
-/* Workgroups per CU the split-K plan targets (0 = the plan's own). */
+/* Workgroups per CU the split-K plan targets (0 = the plan's own).  Over a
+ * paged bf16 or Q8 cache of d = 64 or 128 the plan's own follows the
+ * sequences' lengths on the device; molot_hip_last_plan then gives the most
+ * chunks and the least rows a chunk that it can take. */
 void molot_hip_set_tuning(int wgs_per_cu);
 
 /* How a split context's chunk partials are merged.  in_launch = 0: by a
@@ -327,7 +330,10 @@ void molot_hip_set_tuning(int wgs_per_cu);
  * head group) slot, where the device dispatches workgroup i to XCD i % 8
  * (checked once per device) and the launch can keep a slot's chunks on one
  * XCD; other launches use the combine kernel.  in_launch < 0 (default):
- * in the launch for the fp32 vector-ALU kernel when the slots are a
+ * in the launch for one sequence of at most 2048 attended rows on 4 to 7 or a
+ * multiple of 8 slots (the matrix-core kernel; the vector-ALU kernel over
+ * fp32 and bf16 up to 2^19 rows * outputs a slot, head dims up to 256), and
+ * for the fp32 vector-ALU kernel when the slots are a
  * multiple of 8 on a contiguous cache (every XCD busy) and the attended
  * context spans at least 8192 rows, else the combine kernel.  Both give the same result to
  * fp32 rounding.  If a launch ever found a slot's chunks on different XCDs
