@@ -181,7 +181,9 @@ int molot_hip_decode_step_norm(float* q, const float* k_new, const float* v_new,
  * counterpart).  Q/O [B][nq][d] fp32; K/V pages [num_blocks][nkv][page][d];
  * sequence b attends slots [t0_b, seq_lens[b]) through
  * block_table[b*max_blocks + t/page], with pos_cur = pos[b] (seq_lens[b]-1
- * when pos is NULL).  All index arrays are device int32. */
+ * when pos is NULL).  All index arrays are device int32.  max_seq_len: a
+ * bound of every seq_lens[b] (the longest, or a table's capacity); a longer
+ * sequence's rows past it may be left out. */
 int molot_hip_attn_decode_paged(const float* Q, const void* K, const void* V, float* O,
                                 const int32_t* block_table, const int32_t* seq_lens,
                                 const int32_t* pos, int B, int max_blocks, int max_seq_len,

@@ -33,6 +33,7 @@
 
 #include "device_util.hpp"
 #include "molot_amd/attn_hip.h"
+#include "paged_plan.hpp"
 #include "prefill.hpp"
 #include "prefill_wide.hpp"
 
@@ -543,9 +544,10 @@ struct AttnArgs {
   int nseq;              // chunk_fast, dyn: sequences of the launch
   // Paged matrix-core launches: the rows a chunk takes follow the sequences'
   // lengths (paged_chunk), so that about dyn workgroups have work (0: chunk
-  // as given).  chunk then bounds it from above (the LDS layout), nchunks from
-  // the least chunk, and the grid is flat over the (sequence, chunk) pairs.
-  int dyn;
+  // as given).  chunk then bounds it from above (the LDS layout), nchunks the
+  // chunks of a sequence of at most dyn_span rows, and the grid is flat over
+  // the (sequence, chunk) pairs.
+  int dyn, dyn_span;
   int dyn_pairs;         // host side: pairs the grid holds, and the least chunk
   int dyn_min;
   int matrix, brief;     // host side: the matrix-core kernel; a short context (kBriefSpan)
@@ -1886,35 +1888,9 @@ typedef __bf16 bf16x4_t __attribute__((ext_vector_type(4)));
 typedef short i16x4_t __attribute__((ext_vector_type(4)));
 
 // ---------------------------------------------------------------------------
-// Chunks of a paged batch on the matrix-core kernel.  The host knows only the
-// longest sequence; a chunk sized from that left a batch of uneven lengths
-// with either a second round of workgroups (two fit a CU) or a few long
-// chunks.  Each wave instead sums the lengths (a load a lane, with the one it
-// needs anyway) and takes the chunk that gives the launch's `target`
-// workgroups, two a CU, in whole rounds of the 4 waves' 32-row tiles.
-// Batches with more than kDynLong rows a chunk then need several rounds and
-// take kDynRound rows (or, of short sequences, one chunk each).
-// us a step, 32q/8kv/d128, chunks from the longest sequence against these: Q8
-// 13 sequences of 1 .. 2999 rows 27.9 against 19.4; 2 of 3000 and 8000 31.4
-// against 16.1; 20 of 31 .. 447 18.7 against 14.1; 64 of 100 .. 1000 32.9
-// against 23.3; bf16 7 of 136 .. 2731 26.1 against 19.0; 2 of 3000 and 8000
-// 49.3 against 19.2; 64 of 100 .. 1000 51.1 against 37.0; 32 of 512 .. 4096
-// 76.0 against 72.3.
-constexpr int kDynUnit = 128, kDynLong = 1024, kDynRound = 768, kDynMax = 2048;
-__host__ __device__ constexpr int dyn_chunk(int rows, int nseq, int heads, int target) {
-  const int den = target - nseq * heads;  // workgroups beyond one a (sequence, head)
-  const int c = den > 0 ? (rows * heads + den - 1) / den : kDynMax;
-  if (den > 0 && c <= kDynLong) return c <= kDynUnit ? kDynUnit : (c + kDynUnit - 1) / kDynUnit * kDynUnit;
-  return rows > kDynLong * nseq ? kDynRound : kDynMax;
-}
-// The least it can give while the longest sequence has `span` rows.
-constexpr int dyn_chunk_min(int span, int nseq, int heads, int target) {
-  const int den = target - nseq * heads;
-  const int c = den > 0 ? (span * heads + den - 1) / den : kDynMax;
-  if (c > kDynLong && span <= kDynLong) return kDynMax;
-  const int r = c <= kDynUnit ? kDynUnit : (c + kDynUnit - 1) / kDynUnit * kDynUnit;
-  return r < kDynRound ? r : kDynRound;
-}
+// Chunks of a paged batch on the matrix-core kernel, from the sequences'
+// lengths (paged_plan.hpp).
+
 // A sequence's rows and query position, and the cache rows it attends.
 struct SeqLen {
   int n = 0, pos = -1;
@@ -1928,10 +1904,12 @@ __device__ __forceinline__ SeqLen seq_len(const int32_t* seq_lens, const int32_t
   }
   return s;
 }
-__device__ __forceinline__ int seq_span(SeqLen s, int window, bool fold) {
+// (limit: the host's bound of the rows.  A longer sequence would take pairs
+// and partials that the launch does not have.)
+__device__ __forceinline__ int seq_span(SeqLen s, int window, bool fold, int limit) {
   int t0 = (window > 0 && s.pos - window + 1 > 0) ? s.pos - window + 1 : 0;
   if (t0 > s.n) t0 = s.n;
-  return max((fold ? s.n - 1 : s.n) - t0, 0);
+  return min(max((fold ? s.n - 1 : s.n) - t0, 0), limit);
 }
 // Inclusive sum over the lanes up to this one (row shifts, then row
 // broadcasts of the rows before).
@@ -1948,11 +1926,11 @@ __device__ __forceinline__ int wave_scan(int x) {
 // first: sequence (lane)'s, loaded by the caller.
 __device__ __forceinline__ int paged_chunk(const int32_t* seq_lens, const int32_t* pos_arr,
                                            SeqLen first, int nseq, int window, bool fold,
-                                           int heads, int target) {
+                                           int limit, int heads, int target) {
   const int lane = threadIdx.x & 63;
-  int rows = lane < nseq ? seq_span(first, window, fold) : 0;
+  int rows = lane < nseq ? seq_span(first, window, fold, limit) : 0;
   for (int b = lane + 64; b < nseq; b += 64)
-    rows += seq_span(seq_len(seq_lens, pos_arr, b, nseq), window, fold);
+    rows += seq_span(seq_len(seq_lens, pos_arr, b, nseq), window, fold, limit);
   rows = __builtin_amdgcn_readlane(wave_scan(rows), 63);
   return dyn_chunk(rows, nseq, heads, target);
 }
@@ -2095,14 +2073,15 @@ __global__ __launch_bounds__(kMfmaThreads, 2) void attn_mfma_kernel(AttnArgs a) 
   const int nsub = G / GH;
   int z, hs, b;
   int chunk = a.chunk;
-  int sn = 0, spos = 0;  // dyn: the sequence's length and position
+  int sn = 0, spos = 0, scnt = 0;  // dyn: the sequence's length, position and chunks
   if (PAGED && a.dyn) {
     // flat over the (sequence, chunk) pairs (at least one a sequence), the
     // sequences in order; Q8: all heads of a pair on one XCD, as below
     const int HS = a.nkv * nsub;
     const bool fold = ROPE && a.fold;
     SeqLen sl = seq_len(a.seq_lens, a.pos_arr, (int)(threadIdx.x & 63), a.nseq);
-    chunk = paged_chunk(a.seq_lens, a.pos_arr, sl, a.nseq, a.window, fold, HS, a.dyn);
+    chunk = paged_chunk(a.seq_lens, a.pos_arr, sl, a.nseq, a.window, fold,
+                        a.dyn_span, HS, a.dyn);
     const int id = (int)blockIdx.x;
     int pi;
     if (Q8) {
@@ -2119,13 +2098,14 @@ __global__ __launch_bounds__(kMfmaThreads, 2) void attn_mfma_kernel(AttnArgs a) 
       const int bl = b0 + (int)(threadIdx.x & 63);
       if (b0) sl = seq_len(a.seq_lens, a.pos_arr, bl, a.nseq);
       const int cnt =
-          bl < a.nseq ? max(1, (seq_span(sl, a.window, fold) + chunk - 1) / chunk) : 0;
+          bl < a.nseq ? max(1, dyn_chunks(seq_span(sl, a.window, fold, a.dyn_span), chunk)) : 0;
       const int upto = wave_scan(cnt);
       const uint64_t past = __builtin_amdgcn_ballot_w64(upto > pi);
       if (past) {  // the first lane whose pairs reach past pi
         const int l = __builtin_ctzll(past);
         b = b0 + l;
-        z = pi - (__builtin_amdgcn_readlane(upto, l) - __builtin_amdgcn_readlane(cnt, l));
+        scnt = __builtin_amdgcn_readlane(cnt, l);
+        z = pi - (__builtin_amdgcn_readlane(upto, l) - scnt);
         sn = __builtin_amdgcn_readlane(sl.n, l);
         spos = __builtin_amdgcn_readlane(sl.pos, l);
         break;
@@ -2173,8 +2153,12 @@ __global__ __launch_bounds__(kMfmaThreads, 2) void attn_mfma_kernel(AttnArgs a) 
   int nch = a.nchunks;
   if constexpr (PAGED) {
     const int span = cend - t0;
-    nch = span > 0 ? (span + chunk - 1) / chunk : (fold ? 1 : 0);
-    if (nch > a.nchunks) nch = a.nchunks;
+    if (a.dyn) {
+      nch = span > 0 || fold ? scnt : 0;
+    } else {
+      nch = span > 0 ? (span + chunk - 1) / chunk : (fold ? 1 : 0);
+      if (nch > a.nchunks) nch = a.nchunks;
+    }
   }
   if (z >= nch) {
     if (z == 0) {  // empty attended range: o = 0, and q normed and rotated (empty_range_q)
@@ -3451,7 +3435,7 @@ struct CombArgs {
   int dh;    // head dim as stored (d: the partials' padded head dim)
   int pf, pos0, n;  // prefill rows (AttnArgs::pf): row b at pos0 + b of a cache of n rows
   int pairs;        // combine_kernel: output pairs per workgroup (16, 32 or 64)
-  int dyn, nseq;    // AttnArgs::dyn: the chunk from the sequences' lengths
+  int dyn, dyn_span, nseq;  // AttnArgs::dyn: the chunk from the sequences' lengths
 };
 
 // Chunks of sequence b of a per-sequence launch (a paged batch, or prefill
@@ -3467,12 +3451,13 @@ __device__ __forceinline__ int comb_chunks(const CombArgs& a, int b) {
   }
   int t0 = (a.window > 0 && pos - a.window + 1 > 0) ? pos - a.window + 1 : 0;
   if (t0 > n) t0 = n;
-  const int span = (a.fold ? n - 1 : n) - t0;
+  int span = (a.fold ? n - 1 : n) - t0;
   int chunk = a.chunk;
   if (a.dyn) {
+    span = min(span, a.dyn_span);
     const SeqLen first = seq_len(a.seq_lens, a.pos_arr, (int)(threadIdx.x & 63), a.nseq);
-    chunk = paged_chunk(a.seq_lens, a.pos_arr, first, a.nseq, a.window, a.fold, a.nkv * a.nsub,
-                        a.dyn);
+    chunk = paged_chunk(a.seq_lens, a.pos_arr, first, a.nseq, a.window, a.fold, a.dyn_span,
+                        a.nkv * a.nsub, a.dyn);
   }
   const int nch = span > 0 ? (span + chunk - 1) / chunk : (a.fold ? 1 : 0);
   return nch > a.nchunks ? a.nchunks : nch;
@@ -4028,17 +4013,13 @@ int plan_launch(AttnArgs& a, int d, int span, int gh, int nsubs, int B, int alig
     a.chunk = (int)((tiles + nch - 1) / nch * align);
   } else if (a.dyn && split <= 0 && wpcu <= 0 && span > 0 &&
              (int64_t)B * span * a.nkv * nsubs < ((int64_t)1 << 30) &&
-             span <= kMaxChunks * dyn_chunk_min(span, B, a.nkv * nsubs, a.dyn)) {
-    const int hs = a.nkv * nsubs;
-    const int cmin = dyn_chunk_min(span, B, hs, a.dyn);
+             dyn_plan(span, B, a.nkv * nsubs, a.dyn).nchunks <= kMaxChunks) {
+    const DynPlan p = dyn_plan(span, B, a.nkv * nsubs, a.dyn);
     a.chunk = kDynMax;
-    a.dyn_min = cmin;
-    a.nchunks = (span + cmin - 1) / cmin;
-    // the pairs' bound: the target's (total / chunk + one a sequence), or of
-    // kDynRound rows a chunk
-    const int64_t rounds = (int64_t)B * ((span + kDynRound - 1) / kDynRound);
-    a.dyn_pairs = (int)std::min<int64_t>((int64_t)B * a.nchunks,
-                                         std::max<int64_t>(a.dyn / hs + 1, rounds));
+    a.nchunks = p.nchunks;
+    a.dyn_span = span;
+    a.dyn_pairs = p.pairs;
+    a.dyn_min = p.min_chunk;
   } else {
     a.dyn = 0;
     a.chunk = plan_chunk(span > 0 ? span : 1, rows, align, wpc, split, wpcu);
@@ -4193,6 +4174,7 @@ int launch_pair(AttnFn kern, int threads, size_t lds, AttnArgs a, int gh, int d,
   cb.pos0 = a.pos;
   cb.n = a.n;
   cb.dyn = a.dyn;
+  cb.dyn_span = a.dyn_span;
   cb.nseq = a.nseq;
   // At most 8 chunks (batches of sequences: many slots, few chunks): one
   // wave per 64 pairs (combine_wave_kernel<R>, R = 4 or 8 o loads per lane).

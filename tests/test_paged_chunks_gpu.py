@@ -4,6 +4,7 @@ dyn_chunk, more sequences than a wave has lanes, single rows beside long
 contexts, windows, explicit positions, empty sequences; against the oracle, and
 against the same launch with chunks forced from the host.
 """
+import ctypes
 import math
 
 import numpy as np
@@ -14,6 +15,7 @@ import oracle
 from conftest import normwise_err
 from gpu_util import dev, dev_bf16, host, make_paged, oracle_paged
 from molot_amd import attn
+from molot_amd import lib as _lib
 from molot_amd.synth import Stream, f32_to_bf16
 
 pytestmark = pytest.mark.gpu
@@ -52,6 +54,13 @@ CASES = [
     ("130 sequences", [1 + (37 * i) % 400 for i in range(130)], 16, 4, 64, 0),
     ("window", [3000, 10, 1025, 1024, 5000], 64, 8, 128, 1024),
     ("G = 1, many heads", [900, 20, 333], 40, 40, 64, 0),
+    # one row either side of where a chunk grows by 128 rows: the step attends
+    # one cached row less than its longest sequence counts
+    ("one of 8065", [8065], 32, 8, 128, 0),
+    ("one of 16129", [16129], 32, 8, 64, 0),
+    ("one of 1511, 40 heads", [1511], 40, 40, 64, 0),
+    ("one long of four", [7681, 1, 1, 1], 32, 8, 128, 0),
+    ("one long of 13", [6529] + 12 * [1], 32, 8, 128, 0),
 ]
 
 
@@ -74,6 +83,34 @@ def test_paged_step_vs_oracle(gpu, case):
     Kh, Vh = (host(x.view(torch.int16)).view(np.uint16) for x in (K, V))
     R = oracle.attn_decode_paged(host(q), Kh, Vh, P["bt"], P["n"], None, B, P["max_blocks"], nq,
                                  nkv, d, PAGE, s, window)
+    for b in range(B):
+        assert normwise_err(host(O[b]), R[b]) < TOL, (b, lens[b])
+
+
+@pytest.mark.parametrize("lens", [[4097], [8064], [6570, 200, 300, 107], [33, 700, 5]])
+@pytest.mark.parametrize("bound", ["5/4", "table"])
+def test_paged_step_loose_max_seq_len(gpu, lens, bound):
+    """max_seq_len as a bound above the longest sequence (a captured graph's, a
+    table's capacity) gives the result of the exact one."""
+    print(f"[case] paged chunks, loose bound: {lens} {bound}", flush=True)
+    nq, nkv, d = 32, 8, 128
+    P = batch(lens, nq, nkv, d, 500 + len(lens))
+    B, width = len(lens), 2048  # 32768 rows a sequence
+    table = np.zeros((B, width), np.int32)
+    table[:, :P["max_blocks"]] = P["bt"]
+    inv, s = oracle.rope_inv_freq(500000.0, d), 1 / math.sqrt(d)
+    q, K, V = dev(P["q"]), dev_bf16(P["Kp"]), dev_bf16(P["Vp"])
+    kn, vn, bt, n, iv = (dev(x) for x in (P["k_new"], P["v_new"], table, P["n"], inv))
+    O = torch.full((B, nq, d), float("nan"), device="cuda")
+    p = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    most = width * PAGE if bound == "table" else max(lens) * 5 // 4
+    status = _lib.load().molot_hip_decode_step_paged(
+        p(q), p(kn), p(vn), p(K), p(V), p(O), p(bt), p(n), None, B, width, most, nq, nkv, d, PAGE,
+        p(iv), s, 0, attn.KV_BF16, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert status == 0
+    Kh, Vh = (host(x.view(torch.int16)).view(np.uint16) for x in (K, V))
+    R = oracle.attn_decode_paged(host(q), Kh, Vh, table, P["n"], None, B, width, nq, nkv, d, PAGE,
+                                 s, 0)
     for b in range(B):
         assert normwise_err(host(O[b]), R[b]) < TOL, (b, lens[b])
 
