@@ -287,11 +287,14 @@ __device__ __forceinline__ void split3x2(float a, float b, uint32_t& hi, uint32_
 // holds y to 2^-22 of |y| while |y| >= 2^-3 (lo a normal fp16), and to
 // 2^-25 absolute below (2^-38 of the row's largest |y|); the scaling is
 // exact.  y's unit is 2^(ex-14) (f16_row_unit), the factor that takes a
-// dot product of such pieces back.  Non-finite values make NaN pieces.
+// dot product of such pieces back: a normal float, so that a masked score's
+// -inf stays one over a row of subnormal values (their bits, multiples of
+// 2^-149, are whole numbers of y's 2^-24 at the shift of 126 too).
+// Non-finite values make NaN pieces.
 __device__ __forceinline__ int f16_row_shift(float amax) {
   int ex = 0;
   (void)frexpf(amax, &ex);
-  return 14 - ex;
+  return min(14 - ex, 126);
 }
 __device__ __forceinline__ float f16_row_unit(int shift) { return ldexpf(1.f, -shift); }
 __device__ __forceinline__ uint32_t f16_pair(float a, float b) {
