@@ -124,7 +124,8 @@ struct RowState {
   float m = -1e30f;  // no key yet
   float l = 0.f;     // this lane's keys
   int wsh = 1 << 20;
-  float sc = 0.f;    // 2^wsh
+  float sc = 0.f;      // 2^wsh
+  float lim = 1e-45f;  // 2^(14-wsh), the bound of z; no V unit yet: any z > 0 needs one
 };
 
 // y = z * sc as two fp16 pieces, hi = fp16(y) and lo = fp16(y - hi) of the
@@ -179,8 +180,7 @@ __device__ __forceinline__ float softmax_tile(float (&s)[NK], const float (&ku)[
   };
   probs(st.m);
   float fac = 1.f;
-  // (no V unit yet, sc = 0: any y to come is out of range)
-  const bool fine = ps < 512.f && zt * (st.sc == 0.f ? 3e38f : st.sc) < 16384.f;
+  const bool fine = ps < 512.f && zt < st.lim;
   if (__builtin_amdgcn_ballot_w64(!fine) != 0) {
     float tm = s[0];
 #pragma unroll
@@ -199,6 +199,7 @@ __device__ __forceinline__ float softmax_tile(float (&s)[NK], const float (&ku)[
     st.m = mn;
     st.wsh = ns;
     st.sc = ns == kNoShift ? 0.f : ldexpf(1.f, ns);
+    if (ns != kNoShift) st.lim = ldexpf(1.f, 14 - ns);
   }
   st.l += ps;
 #pragma unroll

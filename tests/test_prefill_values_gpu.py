@@ -1,6 +1,6 @@
 """The 32-row prefill kernels (prefill_narrow.hip, prefill_wide.hip; MI355X only)
-over values at the ends of the number range: subnormal query rows;
-against the oracle at the prefill's 1e-5
+over values at the ends of the number range: subnormal query rows, keys without
+a V value yet before tiny ones; against the oracle at the prefill's 1e-5
 normwise bar.  Every shape has the work from which the library takes these
 kernels.
 """
@@ -16,6 +16,7 @@ from gpu_util import dev, host
 from molot_amd import attn
 from molot_amd.synth import Stream
 from test_d512_gpu import caches, on_dev
+from test_prefill_narrow_gpu import to_cache
 
 pytestmark = pytest.mark.gpu
 
@@ -51,3 +52,20 @@ def test_subnormal_query_rows(gpu, shape, kind):
     assert np.isfinite(O).all()
     assert normwise_err(O, R) < TOL
     assert normwise_err(O[::4], R[::4]) < TOL
+
+
+@pytest.mark.parametrize("kind", ["f32", "bf16", "q8"])
+@pytest.mark.parametrize("shape", [NARROW, WIDE], ids=["narrow", "wide"])
+def test_tiny_values_after_zero_ones(gpu, shape, kind):
+    """V zero over the first tiles and of magnitude 1e-32 after them: the first
+    V unit a row meets is taken however small it is."""
+    nq, nkv, d, M, N = shape
+    print(f"[case] tiny V after zeros {shape} {kind}", flush=True)
+    st = Stream(711 + d)
+    Q, K, V = st.normal((M, nq, d)), st.normal((N, nkv * d)), st.normal((N, nkv * d))
+    V[:200] = 0
+    V[200:] *= np.float32(1e-32)
+    K, V = to_cache(kind, K, V, nkv, d)
+    O, R = run(Q, K, V, nq, nkv, d)
+    assert np.abs(R).max() > 1e-34
+    assert normwise_err(O, R) < TOL
