@@ -342,27 +342,27 @@ void molot_hip_set_tuning(int wgs_per_cu);
  * its merged output would be NaN rather than a stale merge. */
 void molot_hip_set_merge(int in_launch);
 
-/* How the prefill entries feed the matrix cores.  Prompts with enough work
- * (rows * query heads * attended keys * d from 1.2e9 on up to d = 128; from
- * 400000 (query head, key) pairs above 256; any cache type, whatever this
- * switch says): the attended keys of every KV head are split into fp16 pieces
- * once per launch, two of an fp32 row, one of a bf16 or Q8 row, each row
- * scaled by a power of two, into a per-stream workspace of 4 (bf16, Q8) or 8
- * (fp32) bytes * nkv * (N - t0) * d (at most 1 GiB; it grows outside stream
- * capture only, and the buffers it outgrows stay allocated, under 1 GiB in
- * all).  Smaller prompts over fp32 and Q8 caches take K and V as two such
- * pieces too.
- * on = 1 (default): at d = 256, and where one step appends all the keys it
- * attends, made once per launch (12 bytes * nkv * (N - t0) * d of the same
- * workspace), else by the attention kernel from each staged tile.  on = 0: always from
- * the staged tiles.  Both give the same bits.  When the workspace is
- * unavailable every prompt runs as a smaller one does, which agrees to fp32
- * rounding.  A Q8 cache at d = 256 always takes the pieces (its matrix-core
- * kernel has no per-tile split); without them it runs on the vector-ALU
- * kernel, each query row a sequence of its own (the path of smaller prompts
- * at head dims above 256, at those that are not multiples of 8, and of Q8
- * caches at head dims other than 64, 128 and 256), which agrees to fp32
- * rounding. */
+/* How the prefill entries feed the matrix cores.
+ * on = 1 (default): prompts with enough work (rows * query heads * attended
+ * keys * d from 1.2e9 on up to d = 128; from 400000 (query head, key) pairs
+ * above 256; any cache type) have the attended keys of every KV head split
+ * into fp16 pieces once per launch, two of an fp32 row, one of a bf16 or Q8
+ * row, each row scaled by a power of two, into a per-stream workspace of 4
+ * (bf16, Q8) or 8 (fp32) bytes * nkv * (N - t0) * d (at most 1 GiB; it grows
+ * outside stream capture only, and the buffers it outgrows stay allocated,
+ * under 1 GiB in all).  Smaller prompts over fp32 and Q8 caches take K and V
+ * as two such pieces too: at d = 256, and where one step appends all the keys
+ * it attends, made once per launch (12 bytes * nkv * (N - t0) * d of the same
+ * workspace), else by the attention kernel from each staged tile, with the
+ * same bits.
+ * on = 0: no workspace; every prompt runs as a smaller one does, from the
+ * staged tiles, which agrees to fp32 rounding.  So it is when the workspace
+ * is unavailable.  A Q8 cache at d = 256 takes the pieces whatever this says
+ * (its matrix-core kernel has no per-tile split); without them it runs on the
+ * vector-ALU kernel, each query row a sequence of its own (the path of
+ * smaller prompts at head dims above 256, at those that are not multiples of
+ * 8, and of Q8 caches at head dims other than 64, 128 and 256), which agrees
+ * to fp32 rounding. */
 void molot_hip_set_prefill_presplit(int on);
 
 /* Order in which the waves of a workgroup take their chunk's row blocks.

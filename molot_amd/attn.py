@@ -485,9 +485,9 @@ def set_merge(in_launch) -> None:
 
 
 def set_prefill_presplit(on: bool) -> None:
-    """Prefill over fp32/Q8 caches from keys split into pieces once per
-    launch (True, the default) or split per staged tile (False); see
-    molot_hip_set_prefill_presplit.  Both give the same bits."""
+    """Prefill from keys split into pieces once per launch where that pays
+    (True, the default) or without a workspace, split per staged tile (False);
+    see molot_hip_set_prefill_presplit.  Both agree to fp32 rounding."""
     _lib.load().molot_hip_set_prefill_presplit(1 if on else 0)
 
 

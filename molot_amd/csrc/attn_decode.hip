@@ -4977,11 +4977,11 @@ static int rope_append_paged_impl(float* q, const float* k_new, const float* v_n
 // past it, or under a capture that would grow them, such a prefill runs as
 // prefill rows).
 static int prefill_pieces(int nkv, int N, int d, int pos0, int window, int kv_dtype, void* stream,
-                          void** ws, int* T0, int64_t* R, bool only = false) {
+                          int presplit, void** ws, int* T0, int64_t* R, bool only = false) {
   *ws = nullptr;
   *T0 = window > 0 && pos0 - window + 1 > 0 ? std::min(pos0 - window + 1, N) : 0;
   *R = (int64_t)N - *T0;
-  if (!only && (kv_dtype == MOLOT_KV_BF16 || !g_presplit.load(std::memory_order_relaxed))) return 0;
+  if (!only && (kv_dtype == MOLOT_KV_BF16 || !presplit)) return 0;
   const size_t need = (size_t)2 * nkv * 3 * *R * d * sizeof(uint16_t);
   void* p = nullptr;
   const int st =
@@ -5152,11 +5152,13 @@ static int prefill_D(int d) { return d <= 64 ? 64 : d <= 128 ? 128 : d <= 256 ? 
 // against 70 / - / 62; (512, 0) 39 / 35 / 40 against 38 / 36 / 37; (200, 500)
 // 44 / 35 / 45 against 48 / 45 / 46; (512, 16384) 497 / 414 / 485 against 432
 // / 299 / 294.
-static bool prefill_takes_pieces(int d, int M, int N, int nq, int window) {
+// (molot_hip_set_prefill_presplit(0) keeps every prompt off them, and so out
+// of their workspace.)
+static bool prefill_takes_pieces(int d, int M, int N, int nq, int window, int presplit) {
   constexpr int64_t kWideWork = 400000, kPairFlops = 1200000000;
   const int64_t span = window > 0 && window < N ? window : N;
   const int64_t pairs = (int64_t)M * nq * span;
-  if (M > 65535 || (d > 128 && d <= 256)) return false;
+  if (!presplit || M > 65535 || (d > 128 && d <= 256)) return false;
   return d > 256 ? pairs >= kWideWork : pairs * prefill_D(d) >= kPairFlops;
 }
 
@@ -5234,12 +5236,14 @@ static int prefill_on_pieces(const float* Qm, const void* K, const void* V, floa
                         nqb * nkv * a.nsplit, 64 * kWideWaves, a, D, stream);
 }
 
-// split_rows: rows of [T0, N) pf_split_kernel still has to split (the
+// presplit: the setting, read once a call (an appending step's RoPE/append
+// has written pieces in the layout that it selects).
+// split_rows: rows of [T0, N) the split kernel still has to split (the
 // appending step wrote the pieces of the others; -1: all of them)
 static int attn_prefill_impl(const float* Qm, const void* K, const void* V, float* Om, int nq,
                              int nkv, int M, int N, int d, float scale, int pos0, int window,
                              int kv_dtype, const int32_t* block_row, int page, void* stream,
-                             int split_rows = -1) {
+                             int presplit, int split_rows = -1) {
   int st = check_common(nq, nkv, d, kv_dtype);
   if (st) return st;
   // The prefill kernels are built for D = 64, 128, 256.  Any other head dim
@@ -5262,7 +5266,7 @@ static int attn_prefill_impl(const float* Qm, const void* K, const void* V, floa
   if (N == 0) return zero_out(Om, (int64_t)M * nq * d, (hipStream_t)stream);
   if (!K || !V || !aligned16(K) || !aligned16(V) || !aligned16(Qm) || !aligned16(Om))
     return MOLOT_EINVAL;
-  if (prefill_takes_pieces(d, M, N, nq, window)) {
+  if (prefill_takes_pieces(d, M, N, nq, window, presplit)) {
     st = prefill_on_pieces(Qm, K, V, Om, nq, nkv, M, N, d, scale, pos0, window, kv_dtype, block_row,
                            page, stream, split_rows);
     if (st != MOLOT_ENOWS) return st;
@@ -5338,7 +5342,7 @@ static int attn_prefill_impl(const float* Qm, const void* K, const void* V, floa
     void* ws = nullptr;
     int T0 = 0;
     int64_t R = 0;
-    st = prefill_pieces(nkv, N, D, pos0, window, kv_dtype, stream, &ws, &T0, &R, pieces_only);
+    st = prefill_pieces(nkv, N, D, pos0, window, kv_dtype, stream, presplit, &ws, &T0, &R, pieces_only);
     if (st) return st;
     if (!ws && pieces_only) {
       if (R == 0) return zero_out(Om, (int64_t)M * nq * d, (hipStream_t)stream);  // no key attended
@@ -5371,7 +5375,7 @@ int molot_hip_attn_prefill_gqa(const float* Qm, const void* K, const void* V, fl
                                int nkv, int M, int N, int d, float scale, int pos0, int window,
                                int kv_dtype, void* stream) {
   return attn_prefill_impl(Qm, K, V, Om, nq, nkv, M, N, d, scale, pos0, window, kv_dtype,
-                           nullptr, 0, stream);
+                           nullptr, 0, stream, g_presplit.load(std::memory_order_relaxed));
 }
 
 static int prefill_step_impl(float* q, const float* k_new, const float* v_new, void* K, void* V,
@@ -5431,7 +5435,8 @@ static int prefill_step_impl(float* q, const float* k_new, const float* v_new, v
   void* pws = nullptr;
   int T0 = 0;
   int split_rows = -1;
-  if (prefill_takes_pieces(d, M, slot0 + M, nq, window)) {
+  const int presplit = g_presplit.load(std::memory_order_relaxed);
+  if (prefill_takes_pieces(d, M, slot0 + M, nq, window, presplit)) {
     // at d = 512 the split of all rows is as fast (8q/2kv, 1999 tokens: 29 + 7
     // us against 49 for a RoPE/append that leaves the pieces)
     if (d == 64 || d == 128) {
@@ -5445,7 +5450,7 @@ static int prefill_step_impl(float* q, const float* k_new, const float* v_new, v
     }
   } else if (supported_d(d)) {
     int64_t R = 0;
-    st = prefill_pieces(nkv, slot0 + M, d, pos0, window, kv_dtype, stream, &pws, &T0, &R,
+    st = prefill_pieces(nkv, slot0 + M, d, pos0, window, kv_dtype, stream, presplit, &pws, &T0, &R,
                         pieces_only);
     if (st) return st;
     r.pc_R = (int)R;
@@ -5459,7 +5464,7 @@ static int prefill_step_impl(float* q, const float* k_new, const float* v_new, v
   st = launch_rope_tok(r, M, stream);
   if (st) return st;
   return attn_prefill_impl(q, K, V, O, nq, nkv, M, slot0 + M, d, scale, pos0, window, kv_dtype,
-                           block_row, page, stream, split_rows);
+                           block_row, page, stream, presplit, split_rows);
 }
 
 int molot_hip_prefill_step(float* q, const float* k_new, const float* v_new, void* K, void* V,
@@ -5576,7 +5581,7 @@ int molot_hip_attn_prefill_paged(const float* Qm, const void* K, const void* V, 
   if (!block_row || max_blocks <= 0 || N < 0 || (int64_t)N > (int64_t)max_blocks * page)
     return MOLOT_EINVAL;
   return attn_prefill_impl(Qm, K, V, Om, nq, nkv, M, N, d, scale, pos0, window, kv_dtype,
-                           block_row, page, stream);
+                           block_row, page, stream, g_presplit.load(std::memory_order_relaxed));
 }
 
 int molot_hip_vexp(const float* x, float* y, int64_t n, void* stream) {

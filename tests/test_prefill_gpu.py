@@ -225,7 +225,7 @@ def _prefill_both(run):
 
 
 @pytest.mark.parametrize("nq,nkv,d,M,N,pos0,window,kv", [
-    (32, 8, 128, 300, 1300, 1000, 0, "f32"),    # 8 waves, two tile buffers
+    (32, 8, 128, 300, 900, 600, 0, "f32"),      # 8 waves, two tile buffers
     (8, 4, 256, 70, 3070, 3000, 1024, "f32"),   # fp32 d256: two K buffers and one V, window
     (32, 2, 64, 40, 90, 50, 0, "f32"),          # d64
     (8, 2, 128, 5, 40, 35, 0, "f32"),           # few rows: the 4-wave grid
@@ -301,6 +301,34 @@ def test_prefill_presplit_paged(gpu, d, q8):
     o1, o0 = _prefill_both(run)
     assert np.isfinite(o1).all()
     assert np.array_equal(o1, o0)
+
+
+def test_prefill_presplit_off_takes_no_workspace(gpu):
+    """With the switch off a prompt with work enough for the 32-row kernels keeps
+    off their workspace (136 MB here, on a stream of its own), and agrees."""
+    announce("presplit off: no workspace")
+    nq, nkv, d, M, N = 32, 8, 128, 64, 32768
+    st = Stream(333)
+    Q = dev(st.normal((M, nq, d)))
+    K, V = (torch.randn(N, nkv * d, device="cuda").to(torch.bfloat16) for _ in range(2))
+    O = [torch.empty((M, nq, d), device="cuda") for _ in range(2)]
+    s = 1 / math.sqrt(d)
+    taken = []
+    stream = torch.cuda.Stream()
+    stream.wait_stream(torch.cuda.current_stream())
+    try:
+        with torch.cuda.stream(stream):
+            for on in (False, True):
+                attn.set_prefill_presplit(on)
+                torch.cuda.synchronize()
+                free = torch.cuda.mem_get_info()[0]
+                attn.attn_prefill_gqa(Q, K, V, O[on], nq, nkv, M, N, d, s, N - M, 0)
+                torch.cuda.synchronize()
+                taken.append(free - torch.cuda.mem_get_info()[0])
+    finally:
+        attn.set_prefill_presplit(True)
+    assert taken[0] < 100e6 < taken[1]
+    assert normwise_err(host(O[0]), host(O[1])) < TOL
 
 
 def _key_splits(M, N, nq, nkv, pos0, cus):
