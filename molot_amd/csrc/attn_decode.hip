@@ -5134,6 +5134,13 @@ static int pieces_splits(int64_t nqb, int nkv, int M, int N, int G, int qb, int 
   return ns_best;
 }
 
+// Head dims whose smaller prompts run as prefill rows: those the 16-row
+// matrix-core prefill does not tile, and Q8 caches at padded ones (it reads
+// whole 16-code chunks of the built dims only).
+static bool prefill_by_rows(int d, int kv_dtype) {
+  return d > 256 || d % 8 != 0 || (!supported_d(d) && kv_dtype == MOLOT_KV_Q8);
+}
+
 // The head dim a prefill of head dim d is padded to.
 static int prefill_D(int d) { return d <= 64 ? 64 : d <= 128 ? 128 : d <= 256 ? 256 : 512; }
 
@@ -5195,6 +5202,8 @@ static int prefill_on_pieces(const float* Qm, const void* K, const void* V, floa
   a.pos0 = pos0;
   a.window = window;
   a.scale = scale;
+  a.own = prefill_by_rows(d, kv_dtype);
+  a.kv_dtype = kv_dtype;
   if (block_row) {
     if (page <= 0 || (page & (page - 1)) || !q8_pages_ok(nkv, page, kv_dtype))
       return MOLOT_EINVAL;
@@ -5232,7 +5241,7 @@ static int prefill_on_pieces(const float* Qm, const void* K, const void* V, floa
     st = (int)hipGetLastError();
     if (st) return st;
   }
-  return launch_prefill(D <= 128 ? prefill_narrow_fn(D, kv_dtype) : prefill_wide_fn(D, kv_dtype),
+  return launch_prefill(D <= 128 ? prefill_narrow_fn(D, kv_dtype, a.own) : prefill_wide_fn(D, kv_dtype),
                         nqb * nkv * a.nsplit, 64 * kWideWaves, a, D, stream);
 }
 
@@ -5256,9 +5265,7 @@ static int attn_prefill_impl(const float* Qm, const void* K, const void* V, floa
   // (prefill_rows).  Prompts with enough work, at any head dim, take the
   // 32-row kernels instead (prefill_on_pieces).
   const bool padded = !supported_d(d);
-  // Q8 caches at padded dims too (the matrix-core prefill reads whole
-  // 16-code chunks of the built dims only)
-  const bool rows_path = d > 256 || d % 8 != 0 || (padded && kv_dtype == MOLOT_KV_Q8);
+  const bool rows_path = prefill_by_rows(d, kv_dtype);
   const bool pieces_only = kv_dtype == MOLOT_KV_Q8 && d == 256;
   const int D = padded ? (d <= 64 ? 64 : d <= 128 ? 128 : 256) : d;
   if (M < 0 || N < 0 || pos0 < 0 || (M > 0 && (!Qm || !Om))) return MOLOT_EINVAL;

@@ -14,6 +14,9 @@ struct PfArgs {
   int dh;  // head dim as stored (< D: the launch runs padded to D, through the pieces)
   int page_shift;
   float scale;
+  // 32-row kernels: a query row's output depends on the keys it attends alone
+  // (own_rows below); the cache type then says how to read them
+  int own, kv_dtype;
   // the attended keys [T0, T0 + R) of every KV head split into 16-bit pieces
   // once for the launch (pf_split_kernel): [K, V][nkv][3 pieces][R][D]; NULL:
   // the kernel splits each staged tile itself

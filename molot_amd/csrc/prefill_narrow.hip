@@ -39,7 +39,8 @@
 
 namespace {
 
-template <int D, int NP>
+// OWN: PfArgs::own (prefill_tile.hpp).
+template <int D, int NP, bool OWN>
 __global__ __launch_bounds__(512) void prefill_narrow_kernel(PfArgs a) {
   static_assert(D == 64 || D == 128, "head dims up to 128");
   constexpr int KT = kWideTile;
@@ -199,6 +200,7 @@ __global__ __launch_bounds__(512) void prefill_narrow_kernel(PfArgs a) {
   f32x16 s;               // a tile's scores: keys 8*(i/4) + 4*hh + i%4
   uint32_t yh[8], yl[8];  // its y pieces, pairs of the same keys
   float fac = 1.f;
+  [[maybe_unused]] float mark = 0.f;  // OWN: NaN once this lane's units held one
 
   // Scores of this wave's tile of interval it; `copies`: a part of the
   // interval's staging between the products.
@@ -252,6 +254,10 @@ __global__ __launch_bounds__(512) void prefill_narrow_kernel(PfArgs a) {
         vu[4 * i + e] = z[e];
       }
     }
+    if constexpr (OWN)
+      mark = fmaf(reinterpret_cast<const float*>(unit_buf(0, it & 1, kg))[c32] +
+                      reinterpret_cast<const float*>(unit_buf(1, it & 1, kg))[c32],
+                  0.f, mark);
     const bool full = __builtin_amdgcn_ballot_w64(tk < rt0 || tk + KT > rnn) == 0;
     fac = softmax_tile<16>(
         x, ku, vu, qunit, rs, full, [](float v) { return max_xor32(v); },
@@ -333,6 +339,8 @@ __global__ __launch_bounds__(512) void prefill_narrow_kernel(PfArgs a) {
   }
   if (kg == 1 && nint > 0) pv(nint - 1);
   rs.l = sum_xor32(rs.l);
+  float redo = 0.f;  // this key group met a marked row
+  if constexpr (OWN) redo = __builtin_amdgcn_ballot_w64(mark != 0.f) != 0 ? 1.f : 0.f;
 
   // merge of the key groups: group 1's o and (l, m, wsh) through LDS
   lds_barrier();  // every wave is past its tiles
@@ -345,11 +353,18 @@ __global__ __launch_bounds__(512) void prefill_narrow_kernel(PfArgs a) {
       for (int i = 0; i < 4; ++i)
         *reinterpret_cast<f32x4*>(mo + ((b * 4 + i) * 64 + lane) * 4) =
             f32x4{o[b][4 * i], o[b][4 * i + 1], o[b][4 * i + 2], o[b][4 * i + 3]};
-    if (hh == 0) ml[c32] = f32x4{rs.l, rs.m, (float)rs.wsh, 0.f};
+    if (hh == 0) ml[c32] = f32x4{rs.l, rs.m, (float)rs.wsh, redo};
   }
   lds_barrier();
-  if (kg == 1 || !rv) return;
+  if (kg == 1) return;
   const f32x4 st = ml[c32];
+  if constexpr (OWN) {
+    if (redo + st[3] != 0.f) {  // wave-uniform
+      own_rows<D>(own_args(), h, r0 + 32 * rg, 32, kt_s, kt_s + ntile * KT, sp);
+      return;
+    }
+  }
+  if (!rv) return;
   // both in units of the larger max: factors 2^(m_g - M - wsh_g)
   const float M = fmaxf(rs.m, st[1]);
   const int d0 = (int)fmaxf(rs.m - M, -1e6f), d1 = (int)fmaxf(st[1] - M, -1e6f);
@@ -385,8 +400,12 @@ __global__ __launch_bounds__(512) void prefill_narrow_kernel(PfArgs a) {
 
 }  // namespace
 
-PfFn prefill_narrow_fn(int D, int kv_dtype) {
+PfFn prefill_narrow_fn(int D, int kv_dtype, bool own) {
   const bool f32 = kv_dtype == MOLOT_KV_F32;
-  if (D == 64) return f32 ? prefill_narrow_kernel<64, 2> : prefill_narrow_kernel<64, 1>;
-  return f32 ? prefill_narrow_kernel<128, 2> : prefill_narrow_kernel<128, 1>;
+  if (D == 64) {
+    if (own) return f32 ? prefill_narrow_kernel<64, 2, true> : prefill_narrow_kernel<64, 1, true>;
+    return f32 ? prefill_narrow_kernel<64, 2, false> : prefill_narrow_kernel<64, 1, false>;
+  }
+  if (own) return f32 ? prefill_narrow_kernel<128, 2, true> : prefill_narrow_kernel<128, 1, true>;
+  return f32 ? prefill_narrow_kernel<128, 2, false> : prefill_narrow_kernel<128, 1, false>;
 }

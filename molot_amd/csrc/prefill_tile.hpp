@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include "device_util.hpp"
+#include "molot_amd/attn_hip.h"
 #include "prefill.hpp"
 #include "prefill_wide.hpp"
 
@@ -116,6 +117,133 @@ __device__ __forceinline__ float wide_load8(const PfArgs& a, int kv, int h, int 
     }
   }
   return 1.f;
+}
+
+// Rows that the pieces cannot hold for every query row alike.  A product over a
+// tile takes each of its keys for all its query rows, a masked one times zero:
+// a non-finite V row reaches rows that do not attend it, and a K row's infinity
+// leaves no score of its sign.  Where each query row used to read its own keys
+// alone (head dims above 256 and those that are not multiples of 8, Q8 at any
+// padded one: PfArgs::own) the split marks such rows, and those out of the
+// units' range, by a NaN unit, and a workgroup that met one forms its rows'
+// results again from the cache (own_rows).
+constexpr float kOwnMaxK = 3.0e23f;   // 2^78: past it a raw score times its unit may overflow
+constexpr float kOwnMinV = 7.9e-31f;  // 2^-100: below it a V row's unit keeps fewer bits
+__device__ __forceinline__ float own_mark(float xmax, float nonfinite, int kv) {
+  const bool out = kv ? xmax > 0.f && xmax < kOwnMinV : xmax > kOwnMaxK;
+  return out ? NAN : nonfinite;  // 0, or NaN
+}
+
+// Element e of the row at off (wide_row_off's unit), not yet times a Q8 scale.
+__device__ __forceinline__ float own_elem(const PfArgs& a, const char* base, int64_t off, int e) {
+  if (a.kv_dtype == MOLOT_KV_Q8) return (float)reinterpret_cast<const int8_t*>(base)[off + e];
+  if (a.kv_dtype == MOLOT_KV_BF16)
+    return __uint_as_float((uint32_t)reinterpret_cast<const uint16_t*>(base)[off + e] << 16);
+  return reinterpret_cast<const float*>(base)[off + e];
+}
+__device__ __forceinline__ int64_t own_row_off(const PfArgs& a, int h, int t, int64_t& soff) {
+  const bool q8 = a.kv_dtype == MOLOT_KV_Q8;
+  if (a.block_table)
+    return q8 ? wide_row_off<q8_t, true>(a, h, t, soff) : wide_row_off<float, true>(a, h, t, soff);
+  return q8 ? wide_row_off<q8_t, false>(a, h, t, soff) : wide_row_off<float, false>(a, h, t, soff);
+}
+
+// The address of the kernel's arguments (a PfArgs, its only parameter), to be
+// taken in the kernel itself: a called function has no such pointer (the
+// builtin gives null there), so it and own_rows are inlined.
+__device__ __forceinline__ uint64_t own_args() {
+  uint64_t args = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(args));
+  return args;
+}
+
+// Query rows [row0, row0 + n) of KV head h over their own keys of [k_lo, k_hi),
+// a row at a time (every lane of the wave takes part), for the launch's split
+// sp.  Meant for caches that hold non-finite values; two keys in flight.  The
+// arguments are read again from args (own_args), where the compiler cannot move
+// the loads ahead: kept in registers through the kernel's loop they would
+// spill.
+template <int D>
+__device__ __forceinline__ void own_rows(uint64_t args, int h, int row0, int n, int k_lo, int k_hi,
+                                         int sp) {
+  const auto* ka = (const __attribute__((address_space(4))) PfArgs*)args;
+  PfArgs a{};
+  a.q = ka->q, a.k = ka->k, a.v = ka->v, a.o = ka->o, a.block_table = ka->block_table;
+  a.nq = ka->nq, a.nkv = ka->nkv, a.M = ka->M, a.N = ka->N, a.pos0 = ka->pos0;
+  a.window = ka->window, a.dh = ka->dh, a.page_shift = ka->page_shift, a.scale = ka->scale;
+  a.kv_dtype = ka->kv_dtype, a.nsplit = ka->nsplit, a.part_o = ka->part_o, a.part_ml = ka->part_ml;
+  constexpr int EPL = D / 64;  // elements lane + 64*i of a lane
+  const int lane = threadIdx.x & 63;
+  const int G = a.nq / a.nkv;
+  const bool q8 = a.kv_dtype == MOLOT_KV_Q8;
+  const char* kb = reinterpret_cast<const char*>(a.k);
+  const char* vb = reinterpret_cast<const char*>(a.v);
+  for (int row = row0; row < min(row0 + n, a.M * G); ++row) {
+    const int m = row / G, pos = a.pos0 + m;
+    const int64_t slot = (int64_t)m * a.nq + h * G + (row - m * G);
+    int lo = (a.window > 0 && pos - a.window + 1 > 0) ? pos - a.window + 1 : 0;
+    lo = max(lo, k_lo);
+    const int hi = min(min(pos + 1, a.N), k_hi);
+    float q[EPL], o[EPL];
+#pragma unroll
+    for (int i = 0; i < EPL; ++i) {
+      const int e = lane + 64 * i;
+      q[i] = e < a.dh ? a.q[slot * a.dh + e] : 0.f;
+      o[i] = 0.f;
+    }
+    const float qsc = a.scale * kLog2e;
+    float mx = -INFINITY, l = 0.f;
+    for (int t0 = lo; t0 < hi; t0 += 2) {
+      float s[2], v[2][EPL];
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        int64_t soff = 0;
+        const int64_t off = own_row_off(a, h, min(t0 + u, hi - 1), soff);
+        const float ks = q8 ? *reinterpret_cast<const float*>(kb + soff) : 1.f;
+        const float vs = q8 ? *reinterpret_cast<const float*>(vb + soff) : 1.f;
+        float acc = 0.f;
+#pragma unroll
+        for (int i = 0; i < EPL; ++i) {
+          const int e = lane + 64 * i;
+          const bool in = e < a.dh;
+          if (in) acc = fmaf(q[i], own_elem(a, kb, off, e), acc);
+          v[u][i] = in ? own_elem(a, vb, off, e) * vs : 0.f;
+        }
+        s[u] = t0 + u < hi ? wave_reduce<false>(acc) * (ks * qsc) : -INFINITY;
+      }
+      const float mn = fmaxf(mx, fmaxf(s[0], s[1]));
+      if (mn > mx) {
+        const float f = exp2_hw(mx - mn);
+        l *= f;
+#pragma unroll
+        for (int i = 0; i < EPL; ++i) o[i] *= f;
+        mx = mn;
+      }
+#pragma unroll
+      for (int u = 0; u < 2; ++u) {
+        if (t0 + u >= hi) break;
+        const float p = s[u] == -INFINITY ? 0.f : exp2_hw(s[u] - mx);
+        l += p;
+#pragma unroll
+        for (int i = 0; i < EPL; ++i) o[i] = fmaf(p, v[u][i], o[i]);
+      }
+    }
+    const bool part = a.nsplit > 1;
+    const int64_t ps = slot * a.nsplit + sp;
+    const float inv = part ? 1.f : l == 0.f ? 0.f : 1.f / l;  // no key: O = 0 (gemm.h:438)
+#pragma unroll
+    for (int i = 0; i < EPL; ++i) {
+      const int e = lane + 64 * i;
+      if (part)
+        a.part_o[ps * D + e] = o[i];
+      else if (e < a.dh)
+        a.o[slot * a.dh + e] = o[i] * inv;
+    }
+    if (part && lane == 0) {
+      a.part_ml[2 * ps] = l == 0.f ? -INFINITY : mx * kLn2;
+      a.part_ml[2 * ps + 1] = l;
+    }
+  }
 }
 
 // The softmax state of a query row.  o and l are held times 2^-m, and o

@@ -68,6 +68,12 @@ __global__ __launch_bounds__(256) void wide_split_kernel(PfArgs a, uint16_t* out
 #pragma unroll
   for (int e = 0; e < 8; ++e) xm = fmaxf(xm, fabsf(x[e]));
   xm = group_max<UPR>(xm);
+  float mark = 0.f;
+  if (a.own) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) mark = fmaf(x[e] * s, 0.f, mark);
+    mark = own_mark(xm * s, group_sum<UPR>(mark), kv);
+  }
   const int shift = kv ? f16_vrow_shift(xm) : f16_row_shift(xm);
   uint32_t pc[2][4];
 #pragma unroll
@@ -79,7 +85,7 @@ __global__ __launch_bounds__(256) void wide_split_kernel(PfArgs a, uint16_t* out
         u32x4{pc[p][0], pc[p][1], pc[p][2], pc[p][3]};
   if (j == 0)
     reinterpret_cast<float*>(head + NP * Rp * D)[r] =
-        (kv ? f16_vrow_unit(xm, shift) : f16_row_unit(shift)) * s;
+        (kv ? f16_vrow_unit(xm, shift) : f16_row_unit(shift)) * s + mark;
 }
 
 template <int D, int NP>
@@ -266,6 +272,7 @@ __global__ __launch_bounds__(512) void prefill_wide_kernel(PfArgs a) {
     }
   };
   float nku[KPL], nvu[KPL];
+  float mark = 0.f;  // NaN once a tile's units held one (a row's 8 lanes hold all its keys)
   if (ntile > 0) load_units(kt_s);
   wait_vmcnt<0>();
   __syncthreads();
@@ -362,6 +369,8 @@ __global__ __launch_bounds__(512) void prefill_wide_kernel(PfArgs a) {
       const int k0 = tk + KPL * oc;
       const bool full = __builtin_amdgcn_ballot_w64(tk < rt0 || tk + KT > rnn) == 0;
       next_k(1);
+#pragma unroll
+      for (int e = 0; e < KPL; ++e) mark = fmaf(ku[e] + vu[e], 0.f, mark);
       uint32_t yh[KPL / 2], yl[KPL / 2];
       const float fac = softmax_tile<KPL>(
           sv, ku, vu, qunit, rs, full, [](float x) { return group_max<LPR>(x); },
@@ -448,6 +457,11 @@ __global__ __launch_bounds__(512) void prefill_wide_kernel(PfArgs a) {
     lds_barrier();    // C: V, P and the shares may be overwritten
   }
 
+  // (every wave met the same units: the workgroup decides alike)
+  if (__builtin_amdgcn_ballot_w64(mark != 0.f) != 0) {
+    own_rows<D>(own_args(), h, r0 + (QB / 8) * w, QB / 8, kt_s, kt_s + ntile * KT, sp);
+    return;
+  }
   // the rows' (l, m, wsh) from their owners to the waves that hold their o
   rs.l = group_sum<LPR>(rs.l);
   if (oc == 0)

@@ -36,7 +36,7 @@ inline size_t wide_bytes(int nkv, int D, int np, int64_t R) {
 
 // The split of the cached rows, and the attention kernels over the pieces:
 // prefill_narrow.hip (D = 64 and 128), prefill_wide.hip (D = 512).
-PfFn prefill_narrow_fn(int D, int kv_dtype) __attribute__((visibility("hidden")));
+PfFn prefill_narrow_fn(int D, int kv_dtype, bool own) __attribute__((visibility("hidden")));
 SplitFn prefill_wide_split(int D, int kv_dtype, bool paged) __attribute__((visibility("hidden")));
 PfFn prefill_wide_fn(int D, int kv_dtype) __attribute__((visibility("hidden")));
 
