@@ -22,6 +22,12 @@
 // Products and pieces as prefill_wide.hip: q and p two fp16 pieces, K and V
 // NP = 2 for fp32 values, 1 for bf16 and Q8 rows.
 //
+// Error: the scores take the products with a low piece before the others, and
+// the first running maximum of a row is its own (softmax_tile).  Against 64
+// bits (2-norm, 32q/8kv/d128 fp32), before, now and prefill_mfma16_kernel: 300
+// tokens after 900 3.0e-7, 2.6e-7 and 2.7e-7; 2048 tokens 2.6e-7, 2.2e-7 and
+// 2.6e-7; 512 after 16384 7.9e-7, 7.7e-7 and 1.1e-6 (bf16 6.3, 6.3 and 10).
+//
 // What bounds it (32q/8kv/d128, stamped, cycles an interval; products alone
 // take a SIMD 3072 over fp32, 2048 over bf16): 5700 over fp32 and 4100 over
 // bf16, the longer key group's PV 1870 / 1280, scores 2600 / 1330 and softmax
@@ -210,15 +216,18 @@ __global__ __launch_bounds__(512) void prefill_narrow_kernel(PfArgs a) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) s[i] = 0.f;
     // a step's operands are read while the last step's products run (the
-    // compiler would sink the reads to their use)
-    f16x8_t kk[2][2][NP];
+    // compiler would sink the reads to their use).  The products with a low
+    // piece first: they are small beside the others, whose sums alone then
+    // round at the scores' size.
+    f16x8_t kh[QS], kl[2][2];
     auto read_k = [&](int s0) {
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int p = 0; p < NP; ++p)
-          kk[(s0 >> 1) & 1][j][p] =
-              *reinterpret_cast<const f16x8_t*>(kr + p * PB + (kx ^ (32 * (s0 + j))));
+      for (int j = 0; j < 2; ++j) {
+        kh[s0 + j] = *reinterpret_cast<const f16x8_t*>(kr + (kx ^ (32 * (s0 + j))));
+        if constexpr (NP == 2)
+          kl[(s0 >> 1) & 1][j] =
+              *reinterpret_cast<const f16x8_t*>(kr + PB + (kx ^ (32 * (s0 + j))));
+      }
     };
     read_k(0);
 #pragma unroll
@@ -226,17 +235,17 @@ __global__ __launch_bounds__(512) void prefill_narrow_kernel(PfArgs a) {
       if (s0 + 2 < QS) read_k(s0 + 2);
       copies(s0 / 2);
       __builtin_amdgcn_sched_barrier(0);
-      auto& kc = kk[(s0 >> 1) & 1];
       if constexpr (NP == 2) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) s = mfma32_f16(kc[j][1], qh[s0 + j], s);
+        for (int j = 0; j < 2; ++j) s = mfma32_f16(kl[(s0 >> 1) & 1][j], qh[s0 + j], s);
       }
 #pragma unroll
-      for (int j = 0; j < 2; ++j) s = mfma32_f16(kc[j][0], ql[s0 + j], s);
-#pragma unroll
-      for (int j = 0; j < 2; ++j) s = mfma32_f16(kc[j][0], qh[s0 + j], s);
+      for (int j = 0; j < 2; ++j) s = mfma32_f16(kh[s0 + j], ql[s0 + j], s);
       __builtin_amdgcn_sched_barrier(0);
     }
+#pragma unroll
+    for (int i = 0; i < QS; ++i) s = mfma32_f16(kh[i], qh[i], s);
+    __builtin_amdgcn_sched_barrier(0);
   };
   auto soft = [&](int it) {
     const int tk = kt_s + (2 * it + kg) * KT;
@@ -365,13 +374,13 @@ __global__ __launch_bounds__(512) void prefill_narrow_kernel(PfArgs a) {
     }
   }
   if (!rv) return;
-  // both in units of the larger max: factors 2^(m_g - M - wsh_g)
+  // both in units of the larger max: factors 2^(m_g - M), times 2^-wsh_g for o
   const float M = fmaxf(rs.m, st[1]);
-  const int d0 = (int)fmaxf(rs.m - M, -1e6f), d1 = (int)fmaxf(st[1] - M, -1e6f);
-  const int e0 = d0 - rs.wsh, e1 = d1 - (int)st[2];
-  const float l = ldexpf(rs.l, d0) + ldexpf(st[0], d1);
+  const float f0 = exp2_hw(rs.m - M), f1 = exp2_hw(st[1] - M);
+  const int e0 = -rs.wsh, e1 = -(int)st[2];
+  const float l = fmaf(rs.l, f0, st[0] * f1);
   const bool part = a.nsplit > 1;
-  const float inv = part ? 1.f : (l > 0.f ? 1.f / l : 0.f);  // no key: O = 0 (gemm.h:438)
+  const float inv = l > 0.f ? 1.f / l : 0.f;  // no key: O = 0 (gemm.h:438)
   const int64_t ps = slot * a.nsplit + sp;
   float* po = part ? a.part_o + ps * D : a.o + slot * a.dh;
   const int dh = part ? D : a.dh;
@@ -384,7 +393,10 @@ __global__ __launch_bounds__(512) void prefill_narrow_kernel(PfArgs a) {
       const int e = 32 * b + 8 * i + 4 * hh;
       f32x4 y;
 #pragma unroll
-      for (int x = 0; x < 4; ++x) y[x] = (ldexpf(o[b][4 * i + x], e0) + ldexpf(z[x], e1)) * inv;
+      for (int x = 0; x < 4; ++x) {
+        y[x] = fmaf(ldexpf(o[b][4 * i + x], e0), f0, ldexpf(z[x], e1) * f1);
+        if (!part) y[x] = div_by(y[x], l, inv);
+      }
       if (v4) {
         if (e < dh) *reinterpret_cast<f32x4*>(po + e) = y;
       } else {

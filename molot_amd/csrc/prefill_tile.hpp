@@ -247,7 +247,8 @@ __device__ __forceinline__ void own_rows(uint64_t args, int h, int row0, int n, 
 }
 
 // The softmax state of a query row.  o and l are held times 2^-m, and o
-// times 2^wsh more; m is an integer, so every rescale is by a power of two.
+// times 2^wsh more; m moves by whole numbers, so every rescale is by a power
+// of two.
 struct RowState {
   float m = -1e30f;  // no key yet
   float l = 0.f;     // this lane's keys
@@ -268,6 +269,12 @@ __device__ __forceinline__ void mix_split(float z0, float z1, float sc, uint32_t
       : "v"(z1), "v"(sc), "v"(hi));
 }
 
+// o / l from o * (1 / l) and its remainder, rounded once but for ties nearby.
+__device__ __forceinline__ float div_by(float o, float l, float inv) {
+  const float q = o * inv;
+  return fmaf(fmaf(-q, l, o), inv, q);
+}
+
 // One tile of NK keys a lane: s[e] the scores over the row units (K's ku, the
 // q row's qunit: powers of two, Q8 ku times the row's scale), vu the keys' V
 // row units.  Leaves y = p * vu * 2^wsh as two fp16 pieces, y < 2^14, and
@@ -277,7 +284,7 @@ __device__ __forceinline__ void mix_split(float z0, float z1, float sc, uint32_t
 //
 // A tile whose probabilities and y stay in range (the usual one) takes no row
 // maximum: p from the m so far, and two checks.  Otherwise, in any row of the
-// wave, m moves where a score passes it by 4, to the integer above; wsh
+// wave, m moves where a score passes it by 4, by a whole number past it; wsh
 // follows o down with it, and is lowered where y would pass 2^14, by kRoom
 // bits more than needed, so that the next records of 32 rows do not each
 // rescale o.
@@ -314,8 +321,15 @@ __device__ __forceinline__ float softmax_tile(float (&s)[NK], const float (&ku)[
 #pragma unroll
     for (int e = 1; e < NK; ++e) tm = fmaxf(tm, s[e]);
     tm = gmax(tm) * qunit;
-    const float mn = tm > st.m + 4.f ? ceilf(tm) : st.m;
-    const int gsh = (int)fminf(mn - st.m, 1e6f);
+    // a first m within 2^-15 of the maximum (a row of one key then has p = 1 but
+    // for that, and loses nothing to the dropped product of the low pieces);
+    // multiples of 2^-14, so that steps by whole numbers are exact
+    float mn = st.m;
+    if (tm > st.m + 4.f)
+      mn = st.m != -1e30f       ? st.m + ceilf(tm - st.m)
+           : fabsf(tm) < 512.f ? rintf(tm * 16384.f) * (1.f / 16384.f)
+                               : ceilf(tm);
+    const int gsh = (int)rintf(fminf(mn - st.m, 1e6f));
     probs(mn);
     zt = gmax(zt);
     const int grown = min(st.wsh + gsh, kNoShift);

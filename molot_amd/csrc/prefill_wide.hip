@@ -28,6 +28,13 @@
 // values (8 bits; codes of 7) one piece holds exactly down to 2^-28 of the
 // row's largest (two products).  A Q8 row's fp32 scale goes into its unit.
 //
+// Error: PV sums a tile on its own and adds it to o once.  With every product
+// added to o, whose roundings then are six a tile of o's size, the error
+// against 64 bits (2-norm, 8q/2kv/d512 fp32) was larger than the vector-ALU
+// kernel's: 1999 tokens 2.2e-7 against 1.9e-7, now 1.8e-7; 300 after 9000
+// 4.9e-7 against 3.5e-7, now 2.8e-7 (bf16 4.0, 3.5 and 2.6; Q8 3.9, 3.0 and
+// 2.6).  It costs 1.3 % of the step.
+//
 // What bounds it (D = 512, fp32, 8q/2kv, a fresh 1999-token prompt; cycles a
 // tile, stamped): the three phases' latencies, 7400 against the 3072 its 192
 // products of 32 cycles a SIMD take.  Scores 3000 and PV 2300 (each 1536 of
@@ -271,7 +278,6 @@ __global__ __launch_bounds__(512) void prefill_wide_kernel(PfArgs a) {
       }
     }
   };
-  float nku[KPL], nvu[KPL];
   float mark = 0.f;  // NaN once a tile's units held one (a row's 8 lanes hold all its keys)
   if (ntile > 0) load_units(kt_s);
   wait_vmcnt<0>();
@@ -329,19 +335,6 @@ __global__ __launch_bounds__(512) void prefill_wide_kernel(PfArgs a) {
       }
     }
     lds_barrier();  // A: the shares are in LDS, K's buffer is free
-    if (more) {
-      // the next tile's units (waited for where the copies are, below)
-#pragma unroll
-      for (int q = 0; q < KPL; q += 4) {
-        const f32x4_u x = *reinterpret_cast<const f32x4_u*>(kun + tk + KT + q);
-        const f32x4_u y = *reinterpret_cast<const f32x4_u*>(vun + tk + KT + q);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          nku[q + e] = x[e];
-          nvu[q + e] = y[e];
-        }
-      }
-    }
     // K's copies of the next tile between the softmax's steps
     auto next_k = [&](int t) {
       if constexpr (!DB) {
@@ -397,6 +390,8 @@ __global__ __launch_bounds__(512) void prefill_wide_kernel(PfArgs a) {
     }
     lds_barrier();  // B: P is in LDS
     {  // 3. O^T += V^T . P^T of this slice
+      if (more) load_units(tk + KT);  // waited for where the copies are, below
+      __builtin_amdgcn_sched_barrier(0);
       const float fac = (*reinterpret_cast<const f32x4*>(region(my_ow) + 2048 + 16 * my_rr))[0];
       f16x8_t yh[2], yl[2];
 #pragma unroll
@@ -404,55 +399,57 @@ __global__ __launch_bounds__(512) void prefill_wide_kernel(PfArgs a) {
         yh[j] = *reinterpret_cast<const f16x8_t*>(p_ld + (2 * j + hh) * 256);
         yl[j] = *reinterpret_cast<const f16x8_t*>(p_ld + 1024 + (2 * j + hh) * 256);
       }
-      if (__builtin_amdgcn_ballot_w64(fac != 1.f) != 0) {
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
-#pragma unroll
-          for (int i = 0; i < 16; ++i) o[b][i] *= fac;
-      }
       // transposed reads: 16-lane group (2*h + x) reads keys 16j + 8h + 4u ..
       // +3 (lane/4 of it) of the block's 16 columns 16x .. +15
       const int l16 = lane & 15;
       const char* vr = vb + (8 * hh + (l16 >> 2)) * RB + 256 * sl + 32 * ((lane >> 4) & 1) +
                        16 * ((l16 & 3) >> 1) + 8 * (l16 & 1);
       const int vx = 64 * (l16 >> 2);  // the rows' swizzle (64-byte steps)
+      // a tile's sum on its own (the small products first), then one addition to
+      // o, under the next block's products: o takes a rounding a tile instead of
+      // one a product (error: the kernel's head)
+      f32x16 t[2];
 #pragma unroll
-      for (int j = 0; j < 2; ++j) {
+      for (int b = 0; b < 4; ++b) {
+        f16x8_t av[2][NP];
 #pragma unroll
-        for (int b0 = 0; b0 < 4; b0 += 2) {
-          f16x8_t av[2][NP];
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
-          for (int b = 0; b < 2; ++b)
+          for (int p = 0; p < NP; ++p) {
+            i16x4_t t2[2];
 #pragma unroll
-            for (int p = 0; p < NP; ++p) {
-              i16x4_t t2[2];
-#pragma unroll
-              for (int u = 0; u < 2; ++u)
-                t2[u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                    (__attribute__((address_space(3))) i16x4_t*)(
-                        vr + p * KT * RB + (16 * j + 4 * u) * RB + ((64 * (b0 + b)) ^ vx)));
-              av[b][p] = __builtin_bit_cast(
-                  f16x8_t, __builtin_shufflevector(t2[0], t2[1], 0, 1, 2, 3, 4, 5, 6, 7));
-            }
-          if constexpr (NP == 2) {
-#pragma unroll
-            for (int b = 0; b < 2; ++b) o[b0 + b] = mfma32_f16(av[b][1], yh[j], o[b0 + b]);
+            for (int u = 0; u < 2; ++u)
+              t2[u] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                  (__attribute__((address_space(3))) i16x4_t*)(
+                      vr + p * KT * RB + (16 * j + 4 * u) * RB + ((64 * b) ^ vx)));
+            av[j][p] = __builtin_bit_cast(
+                f16x8_t, __builtin_shufflevector(t2[0], t2[1], 0, 1, 2, 3, 4, 5, 6, 7));
           }
+        f32x16 x;
 #pragma unroll
-          for (int b = 0; b < 2; ++b) o[b0 + b] = mfma32_f16(av[b][0], yl[j], o[b0 + b]);
+        for (int i = 0; i < 16; ++i) x[i] = 0.f;
+        if constexpr (NP == 2) {
 #pragma unroll
-          for (int b = 0; b < 2; ++b) o[b0 + b] = mfma32_f16(av[b][0], yh[j], o[b0 + b]);
+          for (int j = 0; j < 2; ++j) x = mfma32_f16(av[j][1], yh[j], x);
         }
-      }
-    }
-    if (more) {
 #pragma unroll
-      for (int e = 0; e < KPL; ++e) {
-        ku[e] = nku[e];
-        vu[e] = nvu[e];
-        asm volatile("" : "+v"(ku[e]), "+v"(vu[e]));  // the units' wait falls here
+        for (int j = 0; j < 2; ++j) x = mfma32_f16(av[j][0], yl[j], x);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) x = mfma32_f16(av[j][0], yh[j], x);
+        t[b & 1] = x;
+        if (b > 0) {
+#pragma unroll
+          for (int i = 0; i < 16; ++i) o[b - 1][i] = fmaf(o[b - 1][i], fac, t[(b - 1) & 1][i]);
+          asm volatile("" : "+v"(o[b - 1]));  // (else all of them sink to the loop's end)
+        }
+        __builtin_amdgcn_sched_barrier(0);
       }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) o[3][i] = fmaf(o[3][i], fac, t[1][i]);
     }
+#pragma unroll
+    for (int e = 0; e < KPL; ++e)
+      asm volatile("" : "+v"(ku[e]), "+v"(vu[e]));  // the units' wait falls here
     wait_vmcnt<0>();  // the next tile's copies (one buffer: K's) are in LDS
     lds_barrier();    // C: V, P and the shares may be overwritten
   }
@@ -500,7 +497,7 @@ __global__ __launch_bounds__(512) void prefill_wide_kernel(PfArgs a) {
         const int e0 = 128 * sl + 32 * b + 8 * i + 4 * hh;
         f32x4 y;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) y[e] = ldexpf(o[b][4 * i + e], sh) * inv;
+        for (int e = 0; e < 4; ++e) y[e] = div_by(ldexpf(o[b][4 * i + e], sh), st[0], inv);
         if (v4) {
           if (e0 < a.dh) *reinterpret_cast<f32x4*>(po + e0) = y;
         } else {
