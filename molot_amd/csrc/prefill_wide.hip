@@ -3,9 +3,8 @@
 //
 // Query rows of one KV head are r = m*G + g (token m at pos0 + m, q head g of
 // the group), as in prefill_mfma16_kernel.  A workgroup of 8 waves owns
-// 32 * RG of them: wave (rg, sl) takes row group rg and the SL = 128
-// elements sl*128 .. of the head dim, for the scores and for the output.
-// (D = 512: 2 row groups x 4 slices, 64 rows).
+// 64 of them: wave (rg, sl) takes row group rg (of two) and the 128 elements
+// sl*128 .. of the head dim, for the scores and for the output.
 // Per tile of 32 keys:
 //   1. every wave forms its slice's share of S^T = K . Q^T on
 //      v_mfma_f32_32x32x16_f16 (A = K from LDS, B = its q pieces in
@@ -103,14 +102,14 @@ __global__ __launch_bounds__(512) void prefill_wide_kernel(PfArgs a) {
   constexpr int QB = 32 * RG;        // query rows a workgroup
   constexpr int RPO = 32 / NSL;      // rows of its group a wave owns in the softmax
   constexpr int LPR = 64 / RPO;      // lanes of an owned row
-  constexpr int KPL = KT / LPR;      // keys a lane of it holds (4 or 8)
+  constexpr int KPL = KT / LPR;      // keys a lane of it holds
   constexpr int RB = 2 * D;          // bytes of a staged row of one piece
   constexpr int TB = NP * KT * RB;   // bytes of a staged tile (K or V)
   constexpr int SXB = 8 * 4096;      // score shares, then P (8 owner regions)
   constexpr bool DB = 4 * TB + SXB <= 160 * 1024;  // two buffers of K and of V
   constexpr int NB = DB ? 2 : 1;
   constexpr int NL = TB / 1024 / 8;  // 1 KB copies a wave issues per K or V tile
-  static_assert(KPL == 4 || KPL == 8, "4 or 8 keys a lane");
+  static_assert(NSL == 4 && KPL == 4, "the layout of the shares and of P");
   static_assert(2 * NB * TB + SXB <= 160 * 1024, "LDS");
   __shared__ __attribute__((aligned(16))) char kbuf[NB][TB];
   __shared__ __attribute__((aligned(16))) char vbuf[NB][TB];
@@ -252,30 +251,25 @@ __global__ __launch_bounds__(512) void prefill_wide_kernel(PfArgs a) {
   // hit distinct units; then, read by its owner alone, overwritten with P:
   // [piece][key octet][row] 16 bytes, and the rows' (alpha, dsh).
   auto region = [&](int ow) { return sx + (rg * NSL + ow) * 4096; };
-  auto swz = [](int rr) {
-    return NSL == 4 ? rr & 7 : ((rr >> 1) & 1) | ((rr & 1) << 1) | (rr & 4);
-  };
+  auto swz = [](int rr) { return rr & 7; };
   const int my_ow = c32 / RPO, my_rr = c32 % RPO;  // this lane's MFMA column
   char* s_st = region(my_ow) + sl * (RPO * 128) + my_rr * 128;
   const int s_sw = 16 * (hh ^ swz(my_rr));
   const char* s_ld = region(sl) + orr * 128;
   const int o_sw = 16 * swz(orr);
-  const char* p_ld = region(my_ow) + (NSL == 4 ? (my_ow & 1) * 128 : 0) + my_rr * 16;
-  char* p_st = region(sl) + (NSL == 4 ? (sl & 1) * 128 : 0) + orr * 16;
+  const char* p_ld = region(my_ow) + (my_ow & 1) * 128 + my_rr * 16;
+  char* p_st = region(sl) + (sl & 1) * 128 + orr * 16;
 
   const float* kun = reinterpret_cast<const float*>(khead + NP * Rp * D) - a.T0 + KPL * oc;
   const float* vun = reinterpret_cast<const float*>(vhead + NP * Rp * D) - a.T0 + KPL * oc;
   float ku[KPL], vu[KPL];
   auto load_units = [&](int tk) {
+    const f32x4_u x = *reinterpret_cast<const f32x4_u*>(kun + tk);
+    const f32x4_u y = *reinterpret_cast<const f32x4_u*>(vun + tk);
 #pragma unroll
-    for (int q = 0; q < KPL; q += 4) {
-      const f32x4_u x = *reinterpret_cast<const f32x4_u*>(kun + tk + q);
-      const f32x4_u y = *reinterpret_cast<const f32x4_u*>(vun + tk + q);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        ku[q + e] = x[e];
-        vu[q + e] = y[e];
-      }
+    for (int e = 0; e < 4; ++e) {
+      ku[e] = x[e];
+      vu[e] = y[e];
     }
   };
   float mark = 0.f;  // NaN once a tile's units held one (a row's 8 lanes hold all its keys)
@@ -346,18 +340,16 @@ __global__ __launch_bounds__(512) void prefill_wide_kernel(PfArgs a) {
     };
     {  // 2. softmax of the owned rows
       float sv[KPL];
-#pragma unroll
-      for (int q = 0; q < KPL; q += 4) {
-        const int un = 16 * ((KPL / 4) * oc + q / 4);
+      {
         f32x4 t = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int s = 0; s < NSL; ++s) {
-          const f32x4 y = *reinterpret_cast<const f32x4*>(s_ld + s * (RPO * 128) + (un ^ o_sw));
+          const f32x4 y = *reinterpret_cast<const f32x4*>(s_ld + s * (RPO * 128) + (16 * oc ^ o_sw));
           t = s ? t + y : y;
         }
-        if (q == 0) next_k(0);
+        next_k(0);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) sv[q + e] = t[e];
+        for (int e = 0; e < 4; ++e) sv[e] = t[e];
       }
       const int k0 = tk + KPL * oc;
       const bool full = __builtin_amdgcn_ballot_w64(tk < rt0 || tk + KT > rnn) == 0;
@@ -370,15 +362,9 @@ __global__ __launch_bounds__(512) void prefill_wide_kernel(PfArgs a) {
           [&](int e) { return k0 + e < rt0 || k0 + e >= rnn; }, yh, yl);
       next_k(2);
       next_k(3);
-      if constexpr (KPL == 4) {
-        char* d = p_st + (oc >> 1) * 256 + (oc & 1) * 8;
-        *reinterpret_cast<u32x2*>(d) = u32x2{yh[0], yh[1]};
-        *reinterpret_cast<u32x2*>(d + 1024) = u32x2{yl[0], yl[1]};
-      } else {
-        char* d = p_st + oc * 256;
-        *reinterpret_cast<u32x4*>(d) = u32x4{yh[0], yh[1], yh[KPL / 2 - 2], yh[KPL / 2 - 1]};
-        *reinterpret_cast<u32x4*>(d + 1024) = u32x4{yl[0], yl[1], yl[KPL / 2 - 2], yl[KPL / 2 - 1]};
-      }
+      char* d = p_st + (oc >> 1) * 256 + (oc & 1) * 8;
+      *reinterpret_cast<u32x2*>(d) = u32x2{yh[0], yh[1]};
+      *reinterpret_cast<u32x2*>(d + 1024) = u32x2{yl[0], yl[1]};
       if (oc == 0)
         *reinterpret_cast<f32x4*>(region(sl) + 2048 + 16 * orr) = f32x4{fac, 0.f, 0.f, 0.f};
     }
