@@ -545,11 +545,10 @@ struct AttnArgs {
   // Paged matrix-core launches: the rows a chunk takes follow the sequences'
   // lengths (paged_chunk), so that about dyn workgroups have work (0: chunk
   // as given).  chunk then bounds it from above (the LDS layout), nchunks the
-  // chunks of a sequence of at most dyn_span rows, and the grid is flat over
-  // the (sequence, chunk) pairs.
+  // chunks of a sequence of at most dyn_span rows (dyn = 0: no limit), and the
+  // grid is flat over the (sequence, chunk) pairs.
   int dyn, dyn_span;
-  int dyn_pairs;         // host side: pairs the grid holds, and the least chunk
-  int dyn_min;
+  int dyn_min;           // host side: the least chunk (and dyn_pairs, below)
   int matrix, brief;     // host side: the matrix-core kernel; a short context (kBriefSpan)
   // In-launch merge (see arrive_and_merge): every chunk of a slot runs on one
   // XCD, and the workgroup that completes a slot merges its chunk partials.
@@ -571,6 +570,7 @@ struct AttnArgs {
   // (token-major) or the block (paged), and the byte stride between heads'
   // scales; a paged block's scales step 4 bytes per slot
   int64_t sc_off, sc_head;
+  int dyn_pairs;         // host side: (sequence, chunk) pairs the grid holds
 };
 
 // Work mapping of one kernel instance.
@@ -2073,7 +2073,7 @@ __global__ __launch_bounds__(kMfmaThreads, 2) void attn_mfma_kernel(AttnArgs a) 
   const int nsub = G / GH;
   int z, hs, b;
   int chunk = a.chunk;
-  int sn = 0, spos = 0, scnt = 0;  // dyn: the sequence's length, position and chunks
+  int sn = 0, spos = 0;  // dyn: the sequence's length and position
   if (PAGED && a.dyn) {
     // flat over the (sequence, chunk) pairs (at least one a sequence), the
     // sequences in order; Q8: all heads of a pair on one XCD, as below
@@ -2104,8 +2104,7 @@ __global__ __launch_bounds__(kMfmaThreads, 2) void attn_mfma_kernel(AttnArgs a) 
       if (past) {  // the first lane whose pairs reach past pi
         const int l = __builtin_ctzll(past);
         b = b0 + l;
-        scnt = __builtin_amdgcn_readlane(cnt, l);
-        z = pi - (__builtin_amdgcn_readlane(upto, l) - scnt);
+        z = pi - (__builtin_amdgcn_readlane(upto, l) - __builtin_amdgcn_readlane(cnt, l));
         sn = __builtin_amdgcn_readlane(sl.n, l);
         spos = __builtin_amdgcn_readlane(sl.pos, l);
         break;
@@ -2152,13 +2151,9 @@ __global__ __launch_bounds__(kMfmaThreads, 2) void attn_mfma_kernel(AttnArgs a) 
   const int cend = fold ? n - 1 : n;
   int nch = a.nchunks;
   if constexpr (PAGED) {
-    const int span = cend - t0;
-    if (a.dyn) {
-      nch = span > 0 || fold ? scnt : 0;
-    } else {
-      nch = span > 0 ? (span + chunk - 1) / chunk : (fold ? 1 : 0);
-      if (nch > a.nchunks) nch = a.nchunks;
-    }
+    const int span = min(cend - t0, a.dyn_span);
+    nch = span > 0 ? dyn_chunks(span, chunk) : (fold ? 1 : 0);
+    if (nch > a.nchunks) nch = a.nchunks;
   }
   if (z >= nch) {
     if (z == 0) {  // empty attended range: o = 0, and q normed and rotated (empty_range_q)
@@ -3433,10 +3428,14 @@ struct CombArgs {
   int nq, nkv, gh, nsub, d, nchunks, chunk, window, rope, paged;
   int fold;  // the attention launch folded in a new token (its chunks tile n - 1 rows)
   int dh;    // head dim as stored (d: the partials' padded head dim)
-  int pf, pos0, n;  // prefill rows (AttnArgs::pf): row b at pos0 + b of a cache of n rows
+  // prefill rows (AttnArgs::pf): row b at pos0 + b of a cache of n rows; dyn: n
+  // is AttnArgs::dyn_span (one field, so that the arguments stay within two
+  // 64-byte lines: the first loads wait for each, 0.14 us a step of 13 sequences)
+  int pf, pos0, n;
   int pairs;        // combine_kernel: output pairs per workgroup (16, 32 or 64)
-  int dyn, dyn_span, nseq;  // AttnArgs::dyn: the chunk from the sequences' lengths
+  int dyn, nseq;    // AttnArgs::dyn: the chunk from the sequences' lengths
 };
+static_assert(sizeof(CombArgs) <= 128, "two lines");
 
 // Chunks of sequence b of a per-sequence launch (a paged batch, or prefill
 // rows), as the attention kernel derives them.
@@ -3454,9 +3453,9 @@ __device__ __forceinline__ int comb_chunks(const CombArgs& a, int b) {
   int span = (a.fold ? n - 1 : n) - t0;
   int chunk = a.chunk;
   if (a.dyn) {
-    span = min(span, a.dyn_span);
+    span = min(span, a.n);
     const SeqLen first = seq_len(a.seq_lens, a.pos_arr, (int)(threadIdx.x & 63), a.nseq);
-    chunk = paged_chunk(a.seq_lens, a.pos_arr, first, a.nseq, a.window, a.fold, a.dyn_span,
+    chunk = paged_chunk(a.seq_lens, a.pos_arr, first, a.nseq, a.window, a.fold, a.n,
                         a.nkv * a.nsub, a.dyn);
   }
   const int nch = span > 0 ? (span + chunk - 1) / chunk : (a.fold ? 1 : 0);
@@ -3989,6 +3988,8 @@ int plan_launch(AttnArgs& a, int d, int span, int gh, int nsubs, int B, int alig
                 void* stream, bool cyclic = false) {
   const int rows = a.nkv * nsubs * B;
   const int split = knob(g_split_chunk), wpcu = knob(g_wgs_per_cu);
+  DynPlan p{};
+  a.dyn_span = 0x7FFFFFFF;
   if (cyclic) {
     const long tiles = span > 0 ? ((long)span + align - 1) / align : 1;
     long nch;
@@ -4013,8 +4014,7 @@ int plan_launch(AttnArgs& a, int d, int span, int gh, int nsubs, int B, int alig
     a.chunk = (int)((tiles + nch - 1) / nch * align);
   } else if (a.dyn && split <= 0 && wpcu <= 0 && span > 0 &&
              (int64_t)B * span * a.nkv * nsubs < ((int64_t)1 << 30) &&
-             dyn_plan(span, B, a.nkv * nsubs, a.dyn).nchunks <= kMaxChunks) {
-    const DynPlan p = dyn_plan(span, B, a.nkv * nsubs, a.dyn);
+             (p = dyn_plan(span, B, a.nkv * nsubs, a.dyn)).nchunks <= kMaxChunks) {
     a.chunk = kDynMax;
     a.nchunks = p.nchunks;
     a.dyn_span = span;
@@ -4172,9 +4172,8 @@ int launch_pair(AttnFn kern, int threads, size_t lds, AttnArgs a, int gh, int d,
   cb.fold = rope && a.fold ? 1 : 0;
   cb.pf = rope ? 0 : a.pf;
   cb.pos0 = a.pos;
-  cb.n = a.n;
+  cb.n = a.dyn ? a.dyn_span : a.n;
   cb.dyn = a.dyn;
-  cb.dyn_span = a.dyn_span;
   cb.nseq = a.nseq;
   // At most 8 chunks (batches of sequences: many slots, few chunks): one
   // wave per 64 pairs (combine_wave_kernel<R>, R = 4 or 8 o loads per lane).
