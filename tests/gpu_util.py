@@ -120,3 +120,21 @@ def oracle_paged(P, inv, scale, window=0, pos=None):
     O = oracle.attn_decode_paged(q, Kp, Vp, P["bt"], P["n"], pos, B, P["max_blocks"], nq, nkv, d,
                                  page, scale, window)
     return q, Kp, Vp, O
+
+
+def pages(X, row, blocks, nkv, d, page, kind):
+    """A pool of `blocks` pages holding the token-major cache X at page ids row."""
+    if kind == "q8":
+        P = np.zeros((blocks, oracle.q8_block_bytes(nkv, d, page)), np.uint8)
+        codes = P[:, :nkv * page * d].reshape(blocks, nkv, page, d)
+        scales = P[:, nkv * page * d:].reshape(blocks, -1, 4)
+        for t in range(X.shape[0]):
+            codes[row[t // page], :, t % page] = X[t, :nkv * d].reshape(nkv, d)
+            sc = X[t, nkv * d:nkv * d + 4 * nkv].reshape(nkv, 4)
+            for h in range(nkv):
+                scales[row[t // page], h * page + t % page] = sc[h]
+    else:
+        P = np.zeros((blocks, nkv, page, d), X.dtype)
+        for t in range(X.shape[0]):
+            P[row[t // page], :, t % page] = X[t].reshape(nkv, d)
+    return P.reshape(blocks, -1)

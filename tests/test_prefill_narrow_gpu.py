@@ -13,7 +13,7 @@ import torch
 
 import oracle
 from conftest import normwise_err
-from gpu_util import dev, host
+from gpu_util import dev, host, pages
 from molot_amd import attn
 from molot_amd.synth import Stream
 from test_d512_gpu import caches, on_dev
@@ -121,3 +121,57 @@ def test_prefill_narrow_step_pieces(gpu, d, kind, n0):
     attn.attn_prefill_gqa(q, Kd, Vd, O2, nq, nkv, M, n0 + M, d, s, n0, 0)
     assert np.isfinite(host(O1)).all()
     assert np.array_equal(host(O1), host(O2))
+
+
+@pytest.mark.parametrize("nq,nkv,d,M,N", [(32, 8, 128, 300, 1300), (64, 8, 64, 300, 1100)])
+@pytest.mark.parametrize("kind", ["f32", "bf16", "q8"])
+def test_prefill_narrow_paged_matches_contiguous(gpu, nq, nkv, d, M, N, kind):
+    """Shuffled pages give the bits of the token-major cache: the same pieces
+    and the same products."""
+    print(f"[case] narrow prefill paged d={d} {kind}", flush=True)
+    assert M * nq * N * d >= 1200000000
+    page = 16
+    st = Stream(281 + d)
+    Q = dev(st.normal((M, nq, d)))
+    K, V = caches(st, N, nkv, d, kind)
+    nb = (N + page - 1) // page
+    row = st.permutation(nb + 3)[:nb].astype(np.int32)
+    Kp, Vp = (on_dev(pages(X, row, nb + 3, nkv, d, page, kind)) for X in (K, V))
+    s = 1 / math.sqrt(d)
+    Oc, Op = (torch.full((M, nq, d), float("nan"), device="cuda") for _ in range(2))
+    attn.attn_prefill_gqa(Q, on_dev(K), on_dev(V), Oc, nq, nkv, M, N, d, s, N - M, 0)
+    attn.attn_prefill_paged(Q, Kp, Vp, Op, dev(row), nb, page, nq, nkv, M, N, d, s, N - M, 0)
+    assert np.isfinite(host(Oc)).all()
+    assert np.array_equal(host(Oc), host(Op))
+
+
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("kind", ["f32", "bf16", "q8"])
+def test_prefill_narrow_step_paged_matches_contiguous(gpu, d, kind):
+    """The step into a sequence's pages behind 131 cached rows (a page begun): the
+    RoPE/append's pieces beside the split of the cached page rows, the bits of
+    the step into a token-major cache, and the same rows stored."""
+    print(f"[case] narrow prefill step, paged d={d} {kind}", flush=True)
+    nq, nkv, M, n0, page = 32, 8, 1017 if d == 64 else 601, 131, 16
+    N = n0 + M
+    assert M * nq * N * d >= 1200000000
+    st = Stream(291 + d)
+    K, V = caches(st, N, nkv, d, kind)
+    q, k, v = (st.normal(x) for x in ((M, nq, d), (M, nkv, d), (M, nkv, d)))
+    nb = (N + page - 1) // page
+    row = st.permutation(nb + 3)[:nb].astype(np.int32)
+    Kc, Vc = on_dev(K), on_dev(V)
+    Kp, Vp = (on_dev(pages(X, row, nb + 3, nkv, d, page, kind)) for X in (K, V))
+    inv, s = dev(oracle.rope_inv_freq(500000.0, d)), 1 / math.sqrt(d)
+    qc, qp = dev(q), dev(q)
+    Oc, Op = (torch.full((M, nq, d), float("nan"), device="cuda") for _ in range(2))
+    attn.prefill_step(qc, dev(k), dev(v), Kc, Vc, Oc, nq, nkv, d, M, n0, n0, inv, s, 0)
+    attn.prefill_step_paged(qp, dev(k), dev(v), Kp, Vp, Op, dev(row), nb, page, nq, nkv, d, M, n0,
+                            n0, inv, s, 0)
+    assert np.isfinite(host(Oc)).all()
+    assert np.array_equal(host(Oc), host(Op)) and np.array_equal(host(qc), host(qp))
+    bits = lambda t: host(t.view(torch.int16) if kind == "bf16" else t)  # noqa: E731
+    for c, p in ((Kc, Kp), (Vc, Vp)):
+        want = pages(bits(c), row, nb + 3, nkv, d, page, kind)
+        got = bits(p).reshape(want.shape)
+        assert np.array_equal(got[row], want[row])

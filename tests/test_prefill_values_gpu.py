@@ -12,7 +12,7 @@ import torch
 
 import oracle
 from conftest import normwise_err
-from gpu_util import dev, host
+from gpu_util import dev, host, pages
 from molot_amd import attn
 from molot_amd.synth import Stream
 from test_d512_gpu import caches, on_dev
@@ -69,24 +69,6 @@ def test_tiny_values_after_zero_ones(gpu, shape, kind):
     O, R = run(Q, K, V, nq, nkv, d)
     assert np.abs(R).max() > 1e-34
     assert normwise_err(O, R) < TOL
-
-
-def pages(X, row, blocks, nkv, d, page, kind):
-    """A pool of `blocks` pages holding the token-major cache X at page ids row."""
-    if kind == "q8":
-        P = np.zeros((blocks, oracle.q8_block_bytes(nkv, d, page)), np.uint8)
-        codes = P[:, :nkv * page * d].reshape(blocks, nkv, page, d)
-        scales = P[:, nkv * page * d:].reshape(blocks, -1, 4)
-        for t in range(X.shape[0]):
-            codes[row[t // page], :, t % page] = X[t, :nkv * d].reshape(nkv, d)
-            sc = X[t, nkv * d:nkv * d + 4 * nkv].reshape(nkv, 4)
-            for h in range(nkv):
-                scales[row[t // page], h * page + t % page] = sc[h]
-    else:
-        P = np.zeros((blocks, nkv, page, d), X.dtype)
-        for t in range(X.shape[0]):
-            P[row[t // page], :, t % page] = X[t].reshape(nkv, d)
-    return P.reshape(blocks, -1)
 
 
 OWN = [
