@@ -351,10 +351,10 @@ void molot_hip_set_merge(int in_launch);
  * (bf16, Q8) or 8 (fp32) bytes * nkv * (N - t0) * d (at most 1 GiB; it grows
  * outside stream capture only, and the buffers it outgrows stay allocated,
  * under 1 GiB in all).  Smaller prompts over fp32 and Q8 caches take K and V
- * as two such pieces too: at d = 256, and where one step appends all the keys
- * it attends, made once per launch (12 bytes * nkv * (N - t0) * d of the same
- * workspace), else by the attention kernel from each staged tile, with the
- * same bits.
+ * as two such pieces too: at d = 256, where one step appends all the keys it
+ * attends, and at d <= 128 where that is faster, made once per launch (12 bytes
+ * * nkv * (N - t0) * d of the same workspace), else by the attention kernel from
+ * each staged tile, with the same bits.
  * on = 0: no workspace; every prompt runs as a smaller one does, from the
  * staged tiles, which agrees to fp32 rounding.  So it is when the workspace
  * is unavailable.  A Q8 cache at d = 256 takes the pieces whatever this says

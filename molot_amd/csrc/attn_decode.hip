@@ -4462,11 +4462,16 @@ PfFn pf_kernel_pre(int d, int pw) {
                  : prefill_mfma16_kernel<256, float, false, 4, true>;
 }
 
-// The split of cached rows for it (d = 256: below, a step's rows leave their
-// pieces themselves or no pieces are made).
-SplitFn pf_split(int kv_dtype, bool paged) {
+// The split of cached rows for it.
+SplitFn pf_split(int d, int kv_dtype, bool paged) {
+  if (kv_dtype == MOLOT_KV_Q8 && d == 64)
+    return paged ? pf_split_kernel<64, q8_t, true> : pf_split_kernel<64, q8_t, false>;
+  if (kv_dtype == MOLOT_KV_Q8 && d == 128)
+    return paged ? pf_split_kernel<128, q8_t, true> : pf_split_kernel<128, q8_t, false>;
   if (kv_dtype == MOLOT_KV_Q8)
     return paged ? pf_split_kernel<256, q8_t, true> : pf_split_kernel<256, q8_t, false>;
+  if (d == 64) return paged ? pf_split_kernel<64, float, true> : pf_split_kernel<64, float, false>;
+  if (d == 128) return paged ? pf_split_kernel<128, float, true> : pf_split_kernel<128, float, false>;
   return paged ? pf_split_kernel<256, float, true> : pf_split_kernel<256, float, false>;
 }
 
@@ -5140,6 +5145,32 @@ static bool prefill_by_rows(int d, int kv_dtype) {
   return d > 256 || d % 8 != 0 || (!supported_d(d) && kv_dtype == MOLOT_KV_Q8);
 }
 
+// Whether a small prompt's launch (head dims up to 128) takes its keys' pieces
+// from one split of them, and not of every staged tile in every query block.
+// The split is a launch of its own: it pays where the tiles of one workgroup
+// follow each other (4 to 7 of them, fp32 at D = 128; from 8 on the keys are
+// split over workgroups), and with 7.5e8 (query head, key, element) products
+// of two row blocks of 128 or more over 512 keys or more (not Q8 at D = 128, nor
+// where each query head has its own KV head: the split itself then takes as
+// much).  Both sides, us a call of the attention alone over fp32 / Q8, per tile
+// against pieces, (rows, cached) of 32q/8kv/d128: (40, 150) 20.6 / 17.3 against
+// 17.0 / 17.0; (150, 0) 17.7 / 15.1 against 15.1 / 15.1; (77, 0) 12.4 / 10.8
+// against 12.2 / 12.3; (77, 150) 19.5 / 19.0 against 20.5 / 20.3; (16, 5000) 35 /
+// 33 against 42 / 39; (16, 16000) 89 / 80 against 107 / 97; (150, 1500) 51.5 /
+// 48.0 against 49.4 / 50.2; 64q (77, 1500) 56.3 / 52.8 against 49.9 / 51.7; 64q
+// (300, 40) 35.6 / 35.3 against 37.2 / 37.3; 32q/8kv/d64 (40, 150) 13.2 / 13.8
+// against 13.1 / 13.1; (300, 1500) 46.2 / 50.4 against 43.0 / 43.0;
+// 16q/16kv/d128 (500, 500) 37.7 / 35.7 against 35.7 / 36.9 (the step 42.7 / 43.1
+// against 45.0 / 46.1).
+static bool prefill_split_pays(int M, int N, int nq, int nkv, int D, int kv_dtype, int window) {
+  const int64_t span = window > 0 && window < N ? window : N;
+  const int64_t tiles = (span + 31) / 32;
+  if (kv_dtype == MOLOT_KV_F32 && D == 128 && tiles >= 4 && tiles < 8) return true;
+  return (kv_dtype == MOLOT_KV_F32 || D == 64) && nq >= 2 * nkv &&
+         (int64_t)M * (nq / nkv) >= 256 && span >= 512 &&
+         (int64_t)M * nq * span * D >= 750000000;
+}
+
 // The head dim a prefill of head dim d is padded to.
 static int prefill_D(int d) { return d <= 64 ? 64 : d <= 128 ? 128 : d <= 256 ? 256 : 512; }
 
@@ -5341,10 +5372,9 @@ static int attn_prefill_impl(const float* Qm, const void* K, const void* V, floa
   // attention kernel copies into LDS, where a fresh prompt's step wrote them
   // (split_rows = 0), and at d = 256, split here.  Not under stream capture
   // when the workspace would have to grow, nor past kMaxPiecesBytes, nor at
-  // d <= 128 after cached rows (a prompt too small for prefill_on_pieces:
-  // 16 rows after 2000 of 32q/8kv/d128 fp32 take 36 us with the split, 29
-  // without): the kernel then splits each staged tile itself.
-  if (D == 256 || split_rows == 0) {
+  // d <= 128 where prefill_split_pays says no: the kernel then splits each
+  // staged tile itself.
+  if (D == 256 || split_rows == 0 || prefill_split_pays(M, N, nq, nkv, D, kv_dtype, window)) {
     void* ws = nullptr;
     int T0 = 0;
     int64_t R = 0;
@@ -5364,7 +5394,7 @@ static int attn_prefill_impl(const float* Qm, const void* K, const void* V, floa
       a.Rsplit = split_rows < 0 ? (int)R : (int)std::min<int64_t>(split_rows, R);
       if (a.Rsplit > 0) {
         const int64_t units = (int64_t)a.Rsplit * (D / 8);
-        hipLaunchKernelGGL(pf_split(kv_dtype, block_row != nullptr),
+        hipLaunchKernelGGL(pf_split(D, kv_dtype, block_row != nullptr),
                            dim3((unsigned)((units + 255) / 256), nkv, 2), dim3(256), 0,
                            (hipStream_t)stream, a, reinterpret_cast<uint16_t*>(ws));
         st = (int)hipGetLastError();
@@ -5460,7 +5490,9 @@ static int prefill_step_impl(float* q, const float* k_new, const float* v_new, v
                         pieces_only);
     if (st) return st;
     r.pc_R = (int)R;
-    if (d <= 128 && slot0 > T0) pws = nullptr;  // cached rows attended: split per tile
+    // cached rows attended: split per tile where that is faster
+    if (d <= 128 && slot0 > T0 && !prefill_split_pays(M, slot0 + M, nq, nkv, d, kv_dtype, window))
+      pws = nullptr;
   }
   if (pws) {
     r.pieces = reinterpret_cast<uint16_t*>(pws);

@@ -25,6 +25,7 @@ from conftest import normwise_err
 from gpu_util import dev, dev_bf16, host, make_decode, make_paged, oracle_decode, oracle_paged
 from molot_amd import attn
 from molot_amd.synth import Stream, bf16_to_f32, f32_to_bf16
+from test_prefill_gpu import presplits
 
 pytestmark = pytest.mark.gpu
 
@@ -299,12 +300,13 @@ def test_prefill_step_paged_head_dims(gpu, d, bf16):
 
 
 @pytest.mark.parametrize("nq,nkv,d,M,N,pos0,window", [
-    (16, 4, 96, 70, 1070, 1000, 0), (8, 4, 200, 40, 540, 500, 100), (8, 2, 56, 33, 33, 0, 0)])
+    (16, 4, 96, 70, 170, 100, 0), (8, 4, 200, 40, 540, 500, 100), (64, 8, 56, 300, 700, 400, 0)])
 def test_prefill_head_dims_per_tile_split(gpu, nq, nkv, d, M, N, pos0, window):
     """An fp32 cache at a padded head dim: the keys split once per launch and
     split per staged tile (the path under stream capture and past the pieces
     workspace's limit) give the same bits, and the oracle's result."""
     announce(f"prefill per-tile split {nq}/{nkv}/d{d} M={M} N={N} win={window}")
+    assert presplits(nq, nkv, d, M, N, window, "f32")
     st = Stream(300 + d)
     Q = st.normal((M, nq, d))
     K, V = prefill_cache(st, N, nkv, d, False)

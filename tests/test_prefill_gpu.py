@@ -224,14 +224,29 @@ def _prefill_both(run):
     return o1, o0
 
 
+def presplits(nq, nkv, d, M, N, window, kv):
+    """Whether the attention entry splits these keys once per launch (a small
+    prompt at d <= 128: prefill_split_pays; above, fp32 and Q8 always do), with
+    too little work for the 32-row kernels."""
+    D = 64 if d <= 64 else 128 if d <= 128 else 256
+    span = min(window, N) if window else N
+    if D == 256:
+        return True
+    work = M * nq * span * D
+    return work < 1200000000 and (
+        (kv == "f32" and D == 128 and 4 <= -(-span // 32) < 8)
+        or ((kv == "f32" or D == 64) and nq >= 2 * nkv and M * (nq // nkv) >= 256 and span >= 512
+            and work >= 750000000))
+
+
 @pytest.mark.parametrize("nq,nkv,d,M,N,pos0,window,kv", [
     (32, 8, 128, 300, 900, 600, 0, "f32"),      # 8 waves, two tile buffers
     (8, 4, 256, 70, 3070, 3000, 1024, "f32"),   # fp32 d256: two K buffers and one V, window
-    (32, 2, 64, 40, 90, 50, 0, "f32"),          # d64
-    (8, 2, 128, 5, 40, 35, 0, "f32"),           # few rows: the 4-wave grid
+    (64, 8, 64, 300, 700, 400, 0, "f32"),       # d64
+    (8, 2, 128, 5, 140, 135, 0, "f32"),         # few rows: the 4-wave grid
     (8, 4, 256, 33, 233, 200, 37, "f32"),       # window cutting inside a tile
-    (32, 8, 128, 77, 1077, 1000, 0, "q8"),
-    (8, 2, 64, 50, 3050, 3000, 1024, "q8"),
+    (64, 8, 64, 250, 850, 600, 0, "q8"),
+    (64, 8, 64, 220, 1220, 1000, 1024, "q8"),
 ])
 def test_prefill_presplit_matches_per_tile(gpu, nq, nkv, d, M, N, pos0, window, kv):
     """fp32 and Q8 caches: the keys split into bf16 pieces once per launch
@@ -239,6 +254,7 @@ def test_prefill_presplit_matches_per_tile(gpu, nq, nkv, d, M, N, pos0, window, 
     the per-tile split (the same pieces, the same products), and the
     oracle's result."""
     announce(f"presplit {nq}/{nkv}/{d} M={M} N={N} pos0={pos0} win={window} {kv}")
+    assert presplits(nq, nkv, d, M, N, window, kv)
     st = Stream(M + N + 3 * d + nq)
     Q = st.normal((M, nq, d))
     if kv == "q8":
@@ -263,14 +279,39 @@ def test_prefill_presplit_matches_per_tile(gpu, nq, nkv, d, M, N, pos0, window, 
     assert err < TOL
 
 
+@pytest.mark.parametrize("nq,nkv,d,M,kv", [(32, 8, 128, 500, "q8"), (32, 8, 128, 333, "f32"),
+                                           (16, 8, 64, 700, "q8"), (16, 8, 64, 61, "f32"),
+                                           (8, 4, 256, 300, "f32")])
+def test_prefill_presplit_step_matches_per_tile(gpu, nq, nkv, d, M, kv):
+    """A fresh prompt's step leaves its rows' pieces from the RoPE/append: the
+    bits of the step that splits every staged tile."""
+    announce(f"presplit step {nq}/{nkv}/{d} M={M} {kv}")
+    assert M * nq * M * d < 1200000000
+    st = Stream(777 + M + d)
+    q, k, v = (st.normal(x) for x in ((M, nq, d), (M, nkv, d), (M, nkv, d)))
+    inv, s = dev(oracle.rope_inv_freq(500000.0, d)), 1 / math.sqrt(d)
+
+    def run():
+        K, V = (torch.zeros(M, attn.q8_row_bytes(nkv, d) if kv == "q8" else nkv * d, device="cuda",
+                            dtype=torch.uint8 if kv == "q8" else torch.float32) for _ in range(2))
+        O = torch.full((M, nq, d), float("nan"), device="cuda")
+        attn.prefill_step(dev(q), dev(k), dev(v), K, V, O, nq, nkv, d, M, 0, 0, inv, s, 0)
+        return host(O)
+
+    o1, o0 = _prefill_both(run)
+    assert np.isfinite(o1).all()
+    assert np.array_equal(o1, o0)
+
+
 @pytest.mark.parametrize("d,q8", [(128, False), (256, False), (64, True)])
 def test_prefill_presplit_paged(gpu, d, q8):
     """The paged prefill over shuffled pages: pieces gathered through the
     block table once per launch, the same bits as the per-tile split."""
     announce(f"presplit paged d={d} q8={q8}")
     st = Stream(300 + d + q8)
-    nq, nkv, M, n0, page, spare = 16, 4, 60, 400, 16, 3
+    nq, nkv, M, n0, page, spare = 64, 8, 250 if d == 64 else 150, 600, 16, 3
     N = n0 + M
+    assert presplits(nq, nkv, d, M, N, 0, "q8" if q8 else "f32")
     nb = (N + page - 1) // page
     nblk = nb + spare
     row = st.permutation(nblk)[:nb].astype(np.int32)
@@ -378,13 +419,16 @@ def test_prefill_row_scales(gpu, kv, presplit):
     largest scores stay near 5 and the softmax mixes rows of every scale,
     on both splits of the keys, against the oracle."""
     announce(f"prefill row scales kv={kv} presplit={presplit}")
-    nq, nkv, d, M, N, pos0 = 16, 4, 128, 64, 1064, 1000
+    nq, nkv, pos0 = 64, 8, 1000
+    d, M = (64, 180) if kv == "q8" else (128, 96)
+    N = pos0 + M
+    assert presplits(nq, nkv, d, M, N, 0, kv)
     st = Stream(950 + (kv == "q8") + 2 * presplit)
     e = np.random.default_rng(951).integers(-30, 31, size=N)
     K = (st.normal((N, nkv * d)) * np.exp2(e)[:, None]).astype(np.float32)
     V = st.normal((N, nkv * d))
     Q = st.normal((M, nq, d))
-    Q[:, :, [5, 40, 99]] *= 1000.0
+    Q[:, :, [5, 40, d - 29]] *= 1000.0
     Q = (Q * 2.0 ** -30 / 30).astype(np.float32)
     if kv == "q8":
         K, V = oracle.q8_cache(K, nkv, d), oracle.q8_cache(V, nkv, d)
@@ -415,7 +459,10 @@ def test_prefill_v_row_scales(gpu, kv, presplit):
     times K channel 0 adds -e ln 2), so that every scale contributes to O
     alike and a band dropped or misweighted shows; against the oracle."""
     announce(f"prefill V row scales kv={kv} presplit={presplit}")
-    nq, nkv, d, M, N, pos0 = 16, 4, 128, 64, 1064, 1000
+    nq, nkv, pos0 = 64, 8, 1000
+    d, M = (64, 180) if kv == "q8" else (128, 96)
+    N = pos0 + M
+    assert presplits(nq, nkv, d, M, N, 0, kv)
     st = Stream(960 + (kv == "q8") + 2 * presplit)
     e = np.random.default_rng(961).integers(-20, 21, size=N)
     s = 1 / math.sqrt(d)
@@ -455,7 +502,10 @@ def test_prefill_ramp_scales(gpu, kv, presplit):
     at the early keys' scale would hold the late keys' terms to 2^-40 of
     it).  Prompt rows see the whole ramp; against the oracle."""
     announce(f"prefill ramp scales kv={kv} presplit={presplit}")
-    nq, nkv, d, M, N, pos0 = 16, 4, 128, 64, 1064, 1000
+    nq, nkv, pos0 = 64, 8, 1000
+    d, M = (64, 180) if kv == "q8" else (128, 96)
+    N = pos0 + M
+    assert presplits(nq, nkv, d, M, N, 0, kv)
     st = Stream(970 + (kv == "q8") + 2 * presplit)
     e = np.round(np.arange(N) * 40.0 / N) - 20.0
     s = 1 / math.sqrt(d)
