@@ -4971,6 +4971,14 @@ static int rope_append_paged_impl(float* q, const float* k_new, const float* v_n
   return (int)hipGetLastError();
 }
 
+// A workspace that the device has no memory for is one that is unavailable:
+// the path without it runs instead.
+static int without_memory(int st) {
+  if (st != (int)hipErrorOutOfMemory) return st;
+  (void)hipGetLastError();
+  return MOLOT_ENOWS;
+}
+
 // The attended keys of a prefill: [T0, N) with T0 the window start of its
 // first query (pos0), split into 16-bit pieces once per launch for fp32 and
 // Q8 caches when the pieces fit (kMaxPiecesBytes) and the workspace need not
@@ -4989,7 +4997,8 @@ static int prefill_pieces(int nkv, int N, int d, int pos0, int window, int kv_dt
   const size_t need = (size_t)2 * nkv * 3 * *R * d * sizeof(uint16_t);
   void* p = nullptr;
   const int st =
-      *R > 0 && need <= kMaxPiecesBytes ? pieces_workspace(stream, need, &p) : MOLOT_ENOWS;
+      *R > 0 && need <= kMaxPiecesBytes ? without_memory(pieces_workspace(stream, need, &p))
+                                        : MOLOT_ENOWS;
   if (st && st != MOLOT_ENOWS) return st;
   if (!st) *ws = p;
   return 0;
@@ -5206,14 +5215,14 @@ static int pieces32_workspace(int nkv, int N, int d, int pos0, int window, int k
   *R = N - *T0;
   const size_t need = wide_bytes(nkv, prefill_D(d), wide_pieces(kv_dtype == MOLOT_KV_F32), *R);
   if (need > kMaxPiecesBytes) return MOLOT_ENOWS;
-  return pieces_workspace(stream, need, ws);
+  return without_memory(pieces_workspace(stream, need, ws));
 }
 
 // The prefill on the 32-row kernels (prefill_narrow.hip, prefill_wide.hip):
 // the attended keys' pieces first (split_rows of them; the appending step
 // wrote the others), then the attention over them.  MOLOT_ENOWS: a capture
-// that would have to grow the workspace, or keys past its cap (the caller
-// takes the other path).
+// that would have to grow the workspace, no memory for it, or keys past its
+// cap (the caller takes the other path).
 static int prefill_on_pieces(const float* Qm, const void* K, const void* V, float* Om, int nq,
                              int nkv, int M, int N, int d, float scale, int pos0, int window,
                              int kv_dtype, const int32_t* block_row, int page, void* stream,
@@ -5252,10 +5261,11 @@ static int prefill_on_pieces(const float* Qm, const void* K, const void* V, floa
   if (a.nsplit > 1) {
     unsigned long long* ctr = nullptr;
     void* ws = nullptr;
-    st = workspace(stream, sizeof(float) * (size_t)M * nq * a.nsplit * (D + 2), &ctr, &ws);
+    st = without_memory(
+        workspace(stream, sizeof(float) * (size_t)M * nq * a.nsplit * (D + 2), &ctr, &ws));
     if (st && st != MOLOT_ENOWS) return st;
     if (st) {
-      a.nsplit = 1;  // under capture the workspace cannot grow
+      a.nsplit = 1;  // under capture, or without memory, the workspace cannot grow
     } else {
       a.part_o = reinterpret_cast<float*>(ws);
       a.part_ml = a.part_o + (size_t)M * nq * a.nsplit * D;

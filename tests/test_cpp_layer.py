@@ -8,6 +8,7 @@ import pytest
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 BIN = os.path.join(HERE, "cpp", "test_attn_cpp")
+BIN_NO_MEMORY = os.path.join(HERE, "cpp", "prefill_no_memory")
 BIN_PAGED = os.path.join(HERE, "cpp", "test_paged_kv")
 
 
@@ -48,3 +49,15 @@ def test_paged_kv_binary_links():
     out = subprocess.run(["ldd", BIN_PAGED], capture_output=True, text=True).stdout
     assert "not found" not in out, out
     assert "libmolot_amd.so" in out and "liboracle.so" in out
+
+
+@pytest.mark.gpu
+def test_prefill_without_memory_for_its_workspace(gpu):
+    """A prompt whose pieces workspace the device has no memory for (the program
+    refuses the allocation itself) runs without it, with the same result."""
+    if not os.path.exists(BIN_NO_MEMORY):
+        pytest.fail(f"{BIN_NO_MEMORY} not built (run __graft_entry__.build())")
+    r = subprocess.run([BIN_NO_MEMORY], capture_output=True, text=True, timeout=120)
+    print(r.stdout)
+    assert r.returncode == 0, r.stdout + r.stderr
+    assert "PASSED" in r.stdout
