@@ -4981,8 +4981,8 @@ static int without_memory(int st) {
 
 // The attended keys of a prefill: [T0, N) with T0 the window start of its
 // first query (pos0), split into 16-bit pieces once per launch for fp32 and
-// Q8 caches when the pieces fit (kMaxPiecesBytes) and the workspace need not
-// grow under capture.  Returns the pieces buffer (NULL: the attention kernel
+// Q8 caches when the pieces fit (kMaxPiecesBytes), there is memory for them and
+// the workspace need not grow under capture.  Returns the pieces buffer (NULL: the attention kernel
 // splits each staged tile itself) and sets T0 and R.
 // only: the launch has no per-tile kernel (a Q8 cache at d = 256): the
 // pieces are made whatever the presplit switch says (within the same cap;
@@ -5159,7 +5159,7 @@ static bool prefill_by_rows(int d, int kv_dtype) {
 // The split is a launch of its own: it pays where the tiles of one workgroup
 // follow each other (4 to 7 of them, fp32 at D = 128; from 8 on the keys are
 // split over workgroups), and with 7.5e8 (query head, key, element) products
-// of two row blocks of 128 or more over 512 keys or more (not Q8 at D = 128, nor
+// of three row blocks of 128 or more over 512 keys or more (not Q8 at D = 128, nor
 // where each query head has its own KV head: the split itself then takes as
 // much).  Both sides, us a call of the attention alone over fp32 / Q8, per tile
 // against pieces, (rows, cached) of 32q/8kv/d128: (40, 150) 20.6 / 17.3 against
@@ -5176,7 +5176,7 @@ static bool prefill_split_pays(int M, int N, int nq, int nkv, int D, int kv_dtyp
   const int64_t tiles = (span + 31) / 32;
   if (kv_dtype == MOLOT_KV_F32 && D == 128 && tiles >= 4 && tiles < 8) return true;
   return (kv_dtype == MOLOT_KV_F32 || D == 64) && nq >= 2 * nkv &&
-         (int64_t)M * (nq / nkv) >= 256 && span >= 512 &&
+         (int64_t)M * (nq / nkv) > 256 && span >= 512 &&
          (int64_t)M * nq * span * D >= 750000000;
 }
 
@@ -5188,24 +5188,44 @@ static int prefill_D(int d) { return d <= 64 ? 64 : d <= 128 ? 128 : d <= 256 ? 
 // enough work.  Not at 129 to 256: prefill_wide_kernel built for D = 256 took
 // 103 / 117 / 118 us a step (2048 tokens, 8q/4kv/d256, window 1024; fp32 / bf16
 // / Q8) against 102 / 90 / 105 on prefill_mfma16_kernel.
-// Above 256 the other path is prefill_rows.  Both sides, 8q/2kv/d512, us a
-// step over fp32 / bf16 / Q8 caches: (rows, cached) = (64, 500) prefill rows
-// 40 / 40 / 37, matrix cores 44 / 38 / 38; (8, 4000) 43 / 38 / 37 against 47 /
-// 38 / 41; (24, 4000) 123 / 117 / 96 against 53 / 44 / 46; (8, 16384) 118 / 94
-// / 77 against 92 / 64 / 61; (2, 16384) 63 / 41 / 36 against 89 / 60 / 58.
+// Above 256 the other path is prefill_rows, which streams the keys once a row
+// and four query heads; below 8 such passes it is the faster one however long
+// the cache.  Both sides, 8q/2kv/d512, us a step over fp32 / bf16 / Q8 caches:
+// (rows, cached) = (64, 500) prefill rows 40 / 40 / 37, matrix cores 44 / 38 /
+// 38; (8, 4000) 43 / 38 / 37 against 47 / 38 / 41; (24, 4000) 123 / 117 / 96
+// against 53 / 44 / 46; (8, 16384) 118 / 94 / 77 against 92 / 64 / 61; (2, 65536),
+// the attention, 162 / 92 / 70 against 350 / 177 / 199; (4, 32768) 164 / 96 / 69
+// against 177 / 94 / 86.
 // Up to 128 it is prefill_mfma16_kernel.  32q/8kv/d128, fp32 / bf16 / Q8:
 // (77, 4000) 80 / 64 / 78 against 75 / 64 / 65; (200, 2000) 76 / - / 77
 // against 70 / - / 62; (512, 0) 39 / 35 / 40 against 38 / 36 / 37; (200, 500)
-// 44 / 35 / 45 against 48 / 45 / 46; (512, 16384) 497 / 414 / 485 against 432
-// / 299 / 294.
+// 44 / 35 / 45 against 48 / 45 / 46; (512, 16384) 497 / 414 / 485 against 438
+// / 301 / 298.
+// At D = 128 that kernel keeps the prompts whose row blocks its key splits (up
+// to 16) multiply to the CUs evenly, while there are too few of them to pay for
+// the split of the cached rows: the attention, (rows a KV head, cached), other
+// against 32 rows, 16q/16kv (128, 16384) fp32 107 against 175, bf16 66 against
+// 101, Q8 89 against 92; 32q/8kv (256, 16384) 104 / 69 / 86 against 113 / 73 /
+// 72; (512, 4000) 55 / 38 / 51 against 55 / 42 / 42; (512, 16384) 170 / 111 / 152
+// against 156 / 102 / 102; (1024, 1500) 47 / 33 / 43 against 44 / 36 / 37.
 // (molot_hip_set_prefill_presplit(0) keeps every prompt off them, and so out
 // of their workspace.)
-static bool prefill_takes_pieces(int d, int M, int N, int nq, int window, int presplit) {
+static bool prefill_takes_pieces(int d, int M, int N, int nq, int nkv, int kv_dtype, int window,
+                                 int presplit) {
   constexpr int64_t kWideWork = 400000, kPairFlops = 1200000000;
   const int64_t span = window > 0 && window < N ? window : N;
   const int64_t pairs = (int64_t)M * nq * span;
+  const int G = nq / nkv;
   if (!presplit || M > 65535 || (d > 128 && d <= 256)) return false;
-  return d > 256 ? pairs >= kWideWork : pairs * prefill_D(d) >= kPairFlops;
+  if (d > 256) return pairs >= kWideWork && (int64_t)M * ((G + 3) / 4) >= 8;
+  if (pairs * prefill_D(d) < kPairFlops) return false;
+  const int64_t nqb = ((int64_t)M * G + 127) / 128, wgs = nqb * nkv;
+  const int cus = num_cus();
+  if (prefill_D(d) == 128 && !prefill_by_rows(d, kv_dtype) && 16 * wgs >= cus && cus % wgs == 0) {
+    if (nqb <= (kv_dtype == MOLOT_KV_Q8 ? 1 : 2)) return false;
+    if (kv_dtype == MOLOT_KV_BF16 && (nqb - 3) * span * nkv < 75000) return false;
+  }
+  return true;
 }
 
 // Their workspace for the attended keys [T0, N).
@@ -5313,7 +5333,7 @@ static int attn_prefill_impl(const float* Qm, const void* K, const void* V, floa
   if (N == 0) return zero_out(Om, (int64_t)M * nq * d, (hipStream_t)stream);
   if (!K || !V || !aligned16(K) || !aligned16(V) || !aligned16(Qm) || !aligned16(Om))
     return MOLOT_EINVAL;
-  if (prefill_takes_pieces(d, M, N, nq, window, presplit)) {
+  if (prefill_takes_pieces(d, M, N, nq, nkv, kv_dtype, window, presplit)) {
     st = prefill_on_pieces(Qm, K, V, Om, nq, nkv, M, N, d, scale, pos0, window, kv_dtype, block_row,
                            page, stream, split_rows);
     if (st != MOLOT_ENOWS) return st;
@@ -5482,7 +5502,7 @@ static int prefill_step_impl(float* q, const float* k_new, const float* v_new, v
   int T0 = 0;
   int split_rows = -1;
   const int presplit = g_presplit.load(std::memory_order_relaxed);
-  if (prefill_takes_pieces(d, M, slot0 + M, nq, window, presplit)) {
+  if (prefill_takes_pieces(d, M, slot0 + M, nq, nkv, kv_dtype, window, presplit)) {
     // at d = 512 the split of all rows is as fast (8q/2kv, 1999 tokens: 29 + 7
     // us against 49 for a RoPE/append that leaves the pieces)
     if (d == 64 || d == 128) {

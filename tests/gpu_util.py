@@ -138,3 +138,23 @@ def pages(X, row, blocks, nkv, d, page, kind):
         for t in range(X.shape[0]):
             P[row[t // page], :, t % page] = X[t].reshape(nkv, d)
     return P.reshape(blocks, -1)
+
+
+def on_32_rows(nq, nkv, d, M, N, window, kind):
+    """Whether a prompt runs on the 32-row prefill kernels (the library's
+    prefill_takes_pieces)."""
+    span, G = min(window, N) if window else N, nq // nkv
+    if d > 256:
+        return M * nq * span >= 400000 and M * -(-G // 4) >= 8
+    D = 64 if d <= 64 else 128
+    if d > 128 or M * nq * span * D < 1200000000:
+        return False
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    nqb = -(-M * G // 128)
+    by_rows = d % 8 != 0 or (kind == "q8" and d not in (64, 128))
+    if D == 128 and not by_rows and 16 * nqb * nkv >= cus and cus % (nqb * nkv) == 0:
+        if nqb <= (1 if kind == "q8" else 2):
+            return False
+        if kind == "bf16" and (nqb - 3) * span * nkv < 75000:
+            return False
+    return True

@@ -235,7 +235,7 @@ def presplits(nq, nkv, d, M, N, window, kv):
     work = M * nq * span * D
     return work < 1200000000 and (
         (kv == "f32" and D == 128 and 4 <= -(-span // 32) < 8)
-        or ((kv == "f32" or D == 64) and nq >= 2 * nkv and M * (nq // nkv) >= 256 and span >= 512
+        or ((kv == "f32" or D == 64) and nq >= 2 * nkv and M * (nq // nkv) > 256 and span >= 512
             and work >= 750000000))
 
 
@@ -348,7 +348,7 @@ def test_prefill_presplit_off_takes_no_workspace(gpu):
     """With the switch off a prompt with work enough for the 32-row kernels keeps
     off their workspace (136 MB here, on a stream of its own), and agrees."""
     announce("presplit off: no workspace")
-    nq, nkv, d, M, N = 32, 8, 128, 64, 32768
+    nq, nkv, d, M, N = 32, 8, 128, 96, 32768
     st = Stream(333)
     Q = dev(st.normal((M, nq, d)))
     K, V = (torch.randn(N, nkv * d, device="cuda").to(torch.bfloat16) for _ in range(2))

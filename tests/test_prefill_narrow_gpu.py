@@ -2,8 +2,8 @@
 (prefill_narrow.hip; MI355X only): shapes at the edges of its row blocks (128
 query rows), key tiles (32, two an interval: odd counts leave one key group a
 masked tile), key splits and padding, over every cache type, against the
-oracle at the prefill's 1e-5 normwise bar.  Every shape has the 1.2e9 (query
-head, key, element) products from which the library takes this path.
+oracle at the prefill's 1e-5 normwise bar.  Every shape is one that the library
+sends here (on_32_rows).
 """
 import math
 
@@ -13,8 +13,9 @@ import torch
 
 import oracle
 from conftest import normwise_err
-from gpu_util import dev, host, pages
+from gpu_util import dev, host, on_32_rows, pages
 from molot_amd import attn
+from molot_amd import lib as _lib
 from molot_amd.synth import Stream
 from test_d512_gpu import caches, on_dev
 
@@ -55,8 +56,7 @@ def to_cache(kind, K, V, nkv, d):
 def test_prefill_narrow_vs_oracle(gpu, shape):
     nq, nkv, d, M, N, pos0, window, kind = shape
     print(f"[case] narrow prefill {shape}", flush=True)
-    D = 64 if d <= 64 else 128
-    assert M * nq * (min(window, N) if window else N) * D >= 1200000000
+    assert on_32_rows(nq, nkv, d, M, N, window, kind)
     st = Stream(M + N + d + nq + 13)
     Q = st.normal((M, nq, d))
     K, V = caches(st, N, nkv, d, kind)
@@ -107,7 +107,7 @@ def test_prefill_narrow_step_pieces(gpu, d, kind, n0):
     K0, V0 = caches(st, n0 + M, nkv, d, kind)
     q = dev(st.normal((M, nq, d)))
     k, v = (dev(st.normal((M, nkv, d))) for _ in range(2))
-    assert M * nq * (n0 + M) * d >= 1200000000
+    assert on_32_rows(nq, nkv, d, M, n0 + M, 0, kind)
     M2, N2 = M + 300, n0 + M + 900
     Kb, Vb = caches(st, N2, nkv, d, kind, sigma=50.0)
     big = torch.empty((M2, nq, d), device="cuda")
@@ -129,7 +129,7 @@ def test_prefill_narrow_paged_matches_contiguous(gpu, nq, nkv, d, M, N, kind):
     """Shuffled pages give the bits of the token-major cache: the same pieces
     and the same products."""
     print(f"[case] narrow prefill paged d={d} {kind}", flush=True)
-    assert M * nq * N * d >= 1200000000
+    assert on_32_rows(nq, nkv, d, M, N, 0, kind)
     page = 16
     st = Stream(281 + d)
     Q = dev(st.normal((M, nq, d)))
@@ -154,7 +154,7 @@ def test_prefill_narrow_step_paged_matches_contiguous(gpu, d, kind):
     print(f"[case] narrow prefill step, paged d={d} {kind}", flush=True)
     nq, nkv, M, n0, page = 32, 8, 1017 if d == 64 else 601, 131, 16
     N = n0 + M
-    assert M * nq * N * d >= 1200000000
+    assert on_32_rows(nq, nkv, d, M, N, 0, kind)
     st = Stream(291 + d)
     K, V = caches(st, N, nkv, d, kind)
     q, k, v = (st.normal(x) for x in ((M, nq, d), (M, nkv, d), (M, nkv, d)))
@@ -175,3 +175,35 @@ def test_prefill_narrow_step_paged_matches_contiguous(gpu, d, kind):
         want = pages(bits(c), row, nb + 3, nkv, d, page, kind)
         got = bits(p).reshape(want.shape)
         assert np.array_equal(got[row], want[row])
+
+
+@pytest.mark.parametrize("nq,nkv,d,M,N,kind", [
+    (16, 16, 128, 100, 7000, "bf16"),  # one row block a head, which 16 key splits multiply to the CUs
+    (16, 16, 128, 100, 7000, "q8"),
+    (32, 8, 128, 64, 8000, "f32"),     # two
+    (32, 8, 128, 128, 4100, "bf16"),   # four, over too few keys
+    (8, 2, 512, 2, 30000, "q8"),       # a few rows over a long cache
+    (8, 2, 512, 7, 8000, "f32"),
+])
+def test_prompts_that_keep_the_smaller_ones_path(gpu, nq, nkv, d, M, N, kind):
+    """Work enough for the 32-row kernels, but too few rows to pay for the split of
+    the cached rows: the bits of the path without a workspace."""
+    print(f"[case] few rows {nq}/{nkv}/{d} M={M} N={N} {kind}", flush=True)
+    assert M * nq * N >= 400000 if d > 256 else M * nq * N * d >= 1200000000
+    assert not on_32_rows(nq, nkv, d, M, N, 0, kind)
+    st = Stream(311 + M)
+    Q = dev(st.normal((M, nq, d)))
+    K, V = (on_dev(x) for x in caches(st, N, nkv, d, kind))
+    out = []
+    _lib.load().molot_hip_set_block_order(0)  # the vector-ALU kernel: the same sums every time
+    try:
+        for on in (True, False):
+            attn.set_prefill_presplit(on)
+            O = torch.full((M, nq, d), float("nan"), device="cuda")
+            attn.attn_prefill_gqa(Q, K, V, O, nq, nkv, M, N, d, 1 / math.sqrt(d), N - M, 0)
+            out.append(host(O))
+    finally:
+        attn.set_prefill_presplit(True)
+        _lib.load().molot_hip_set_block_order(1)
+    assert np.isfinite(out[0]).all()
+    assert np.array_equal(out[0], out[1])

@@ -12,7 +12,7 @@ import torch
 
 import oracle
 from conftest import normwise_err
-from gpu_util import dev, host, pages
+from gpu_util import dev, host, on_32_rows, pages
 from molot_amd import attn
 from molot_amd.synth import Stream
 from test_d512_gpu import caches, on_dev
@@ -30,7 +30,8 @@ WIDE = (8, 2, 512, 150, 700)
 def run(Q, K, V, nq, nkv, d, window=0):
     """(kernel, oracle) outputs of a prompt at the end of its cache."""
     M, N, s = Q.shape[0], K.shape[0], 1 / math.sqrt(d)
-    assert M * nq * N >= 400000 if d > 256 else M * nq * N * (64 if d <= 64 else 128) >= 1.2e9
+    kind = {np.dtype(np.uint8): "q8", np.dtype(np.uint16): "bf16"}.get(K.dtype, "f32")
+    assert on_32_rows(nq, nkv, d, M, N, window, kind)
     O = torch.full((M, nq, d), -77.0, device="cuda")
     attn.attn_prefill_gqa(dev(Q), on_dev(K), on_dev(V), O, nq, nkv, M, N, d, s, N - M, window)
     return host(O), oracle.attn_prefill(Q, K, V, nq, nkv, M, N, d, s, N - M, window)

@@ -1,8 +1,8 @@
 """The prefill at head dims above 256 on the matrix cores (prefill_wide.hip;
 MI355X only): shapes at the edges of its row blocks (64 query rows), key tiles
 (32), key splits and padding to D = 512, over every cache type, against the
-oracle at the prefill's 1e-5 normwise bar.  Every shape has at least the
-400000 (query head, key) pairs from which the library takes this path.
+oracle at the prefill's 1e-5 normwise bar.  Every shape is one that the library
+sends here (on_32_rows).
 """
 import math
 
@@ -12,7 +12,7 @@ import torch
 
 import oracle
 from conftest import normwise_err
-from gpu_util import dev, host
+from gpu_util import dev, host, on_32_rows
 from molot_amd import attn
 from molot_amd.synth import Stream
 from test_d512_gpu import caches, on_dev
@@ -43,7 +43,7 @@ SHAPES = [
 def test_prefill_wide_vs_oracle(gpu, shape):
     nq, nkv, d, M, N, pos0, window, kind = shape
     print(f"[case] wide prefill {shape}", flush=True)
-    assert M * nq * (min(window, N) if window else N) >= 400000
+    assert on_32_rows(nq, nkv, d, M, N, window, kind)
     st = Stream(M + N + d + nq + 11)
     Q = st.normal((M, nq, d))
     K, V = caches(st, N, nkv, d, kind)
