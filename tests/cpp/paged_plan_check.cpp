@@ -1,5 +1,5 @@
-// Host check of molot_amd/csrc/paged_plan.hpp: over every length of a lone
-// sequence and over random batches, with the host's bound of the longest
+// Host check of molot_amd/csrc/paged_plan.hpp, bf16 and Q8: over every length of
+// a lone sequence and over random batches, with the host's bound of the longest
 // sequence exact (a fused step attends one row less than it counts) or loose,
 // the chunks the device takes stay within the chunks, pairs and least rows that
 // the host planned for.  Prints the first failures; exit status 0 if none.
@@ -16,22 +16,29 @@ namespace {
 constexpr int kTarget = 512;  // two workgroups on each of 256 CUs
 long g_bad = 0;
 
-void check(const std::vector<int>& lens, int span, int heads) {
+void check(const std::vector<int>& lens, int span, int heads, bool q8) {
   const int B = (int)lens.size();
-  const DynPlan p = dyn_plan(span, B, heads, kTarget);
+  const DynPlan p = dyn_plan(span, B, heads, kTarget, q8);
   long rows = 0, pairs = 0;
   for (int n : lens) rows += n;
-  const int chunk = dyn_chunk((int)rows, B, heads, kTarget);
+  const int chunk = dyn_chunk((int)rows, B, heads, kTarget, q8);
   int most = 0;
   for (int n : lens) {
     most = std::max(most, dyn_chunks(n, chunk));
     pairs += std::max(1, dyn_chunks(n, chunk));
   }
-  if (most <= p.nchunks && pairs <= p.pairs && chunk >= p.min_chunk && chunk <= kDynMax) return;
+  if (most <= p.nchunks && pairs <= p.pairs && chunk >= p.min_chunk && chunk <= kDynMax &&
+      p.likely >= 1 && p.likely <= p.nchunks)
+    return;
   if (g_bad++ < 20)
-    std::printf("%d sequences, %d heads, bound %d, %ld rows: chunk %d (planned >= %d), "
-                "%d chunks of %d, %ld pairs of %d\n",
-                B, heads, span, rows, chunk, p.min_chunk, most, p.nchunks, pairs, p.pairs);
+    std::printf("%s, %d sequences, %d heads, bound %d, %ld rows: chunk %d (planned >= %d), "
+                "%d chunks of %d (likely %d), %ld pairs of %d\n",
+                q8 ? "Q8" : "bf16", B, heads, span, rows, chunk, p.min_chunk, most, p.nchunks, p.likely, pairs, p.pairs);
+}
+
+void check(const std::vector<int>& lens, int span, int heads) {
+  check(lens, span, heads, false);
+  check(lens, span, heads, true);
 }
 
 }  // namespace

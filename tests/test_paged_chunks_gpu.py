@@ -115,6 +115,57 @@ def test_paged_step_loose_max_seq_len(gpu, lens, bound):
         assert normwise_err(host(O[b]), R[b]) < TOL, (b, lens[b])
 
 
+def pools(P, nkv, d, kind, seed):
+    """P's K and V pools on the device, or Q8 ones of as many blocks."""
+    if kind == "bf16":
+        return dev_bf16(P["Kp"]), dev_bf16(P["Vp"])
+    st = Stream(seed)
+    nblk, out = P["Kp"].shape[0], []
+    for _ in range(2):
+        X = np.zeros((nblk, oracle.q8_block_bytes(nkv, d, PAGE)), np.uint8)
+        cut = nkv * PAGE * d
+        codes = np.clip(np.rint(st.normal((nblk, cut)) * 32), -127, 127).astype(np.int8)
+        X[:, :cut] = codes.view(np.uint8)
+        sc = (np.abs(st.normal((nblk, nkv * PAGE))) * 0.03 + 0.01).astype(np.float32)
+        X[:, cut:cut + 4 * nkv * PAGE] = sc.view(np.uint8)
+        out.append(dev(X))
+    return out
+
+
+@pytest.mark.parametrize("kind", ["bf16", "q8"])
+@pytest.mark.parametrize("lens, nq, nkv, d", [
+    # the others leave the chunks short: the long ones may have more of them than a
+    # batch of long ones would (dyn_plan's likely), in the combine's first round
+    # of loads (9 to 32, 33 to 64, 65 to 128 chunks) and past it
+    ([1100] + 40 * [10], 16, 2, 128),
+    ([6000] + 40 * [10], 16, 2, 128),
+    ([12000, 9000] + 20 * [10], 16, 2, 128),
+    ([14000] + 40 * [10], 8, 1, 64),
+    # several rounds: 768 rows a chunk, Q8 768, 1024 or 1536
+    ([1025, 1024, 4097, 4096] + 60 * [1030], 32, 8, 64),
+    ([2049, 2048, 1, 4000] + 60 * [2060], 32, 8, 64),
+    ([4097, 4096, 4200, 6145] + 60 * [4110], 32, 8, 64),
+], ids=lambda x: f"{len(x)}x{max(x)}" if isinstance(x, list) else None)
+def test_more_chunks_than_likely(gpu, kind, lens, nq, nkv, d):
+    print(f"[case] paged chunks past the likely ones: {kind} {len(lens)}x{max(lens)}", flush=True)
+    P = batch(lens, nq, nkv, d, 611)
+    B = len(lens)
+    K, V = pools(P, nkv, d, kind, 612)
+    Q, bt, n = dev(P["q"]), dev(P["bt"].reshape(-1)), dev(P["n"])
+    outs = []
+    try:
+        for forced in (0, 96):
+            attn.set_split_chunk(forced)
+            O = torch.full((B, nq, d), float("nan"), device="cuda")
+            attn.attn_decode_paged(Q, K, V, O, bt, n, None, B, P["max_blocks"], nq, nkv, d, PAGE,
+                                   1 / math.sqrt(d), 0)
+            outs.append(host(O))
+    finally:
+        attn.set_split_chunk(0)
+    for b in range(B):
+        assert normwise_err(outs[0][b], outs[1][b]) < TOL, (b, lens[b])
+
+
 @pytest.mark.parametrize("kind", ["bf16", "q8"])
 @pytest.mark.parametrize("positions", [False, True])
 def test_paged_attention_matches_forced_chunks(gpu, kind, positions):
@@ -126,21 +177,7 @@ def test_paged_attention_matches_forced_chunks(gpu, kind, positions):
     nq, nkv, d, window = 32, 8, 128, 200 if positions else 0
     P = batch(lens, nq, nkv, d, 411)
     B = len(lens)
-    if kind == "q8":
-        st = Stream(412)
-        nblk = P["Kp"].shape[0]
-        pools = []
-        for _ in range(2):
-            X = np.zeros((nblk, oracle.q8_block_bytes(nkv, d, PAGE)), np.uint8)
-            cut = nkv * PAGE * d
-            codes = np.clip(np.rint(st.normal((nblk, cut)) * 32), -127, 127).astype(np.int8)
-            X[:, :cut] = codes.view(np.uint8)
-            sc = (np.abs(st.normal((nblk, nkv * PAGE))) * 0.03 + 0.01).astype(np.float32)
-            X[:, cut:cut + 4 * nkv * PAGE] = sc.view(np.uint8)
-            pools.append(dev(X))
-        K, V = pools
-    else:
-        K, V = dev_bf16(P["Kp"]), dev_bf16(P["Vp"])
+    K, V = pools(P, nkv, d, kind, 412)
     pos = dev(np.asarray([max(0, n - 1 - 7 * b) for b, n in enumerate(lens)], np.int32)) \
         if positions else None
     Q, bt, n = dev(P["q"]), dev(P["bt"].reshape(-1)), dev(P["n"])
