@@ -33,8 +33,8 @@
 // bf16, the longer key group's PV 1870 / 1280, scores 2600 / 1330 and softmax
 // 870 / 900 one after the other; without the copies 5100.  Against
 // prefill_mfma16_kernel (16 rows a wave; three bf16 products over bf16 and
-// Q8 values): 2048-token prompt fp32 step 154 -> 137 us, 512 tokens after
-// 16384 bf16 414 -> 302, Q8 485 -> 294, fp32 497 -> 432 us.
+// Q8 values): 2048-token prompt fp32 step 154 -> 136 us, 512 tokens after
+// 16384 bf16 414 -> 301, Q8 485 -> 298, fp32 497 -> 438 us.
 #include <hip/hip_runtime.h>
 
 #include "device_util.hpp"

@@ -35,13 +35,15 @@
 // 2.6).  It costs 1.3 % of the step.
 //
 // What bounds it (D = 512, fp32, 8q/2kv, a fresh 1999-token prompt; cycles a
-// tile, stamped): the three phases' latencies, 7400 against the 3072 its 192
-// products of 32 cycles a SIMD take.  Scores 3000 and PV 2300 (each 1536 of
-// products, then the barrier, the first LDS reads and the stores of the
-// shares), the softmax with the next K copies 1950.  The copies go out between
-// products and softmax steps: in a row they held each wave ~500 cycles.
-// The step: 1468 us with each query row streamed by the vector-ALU kernel
-// (prefill_rows), 230 us here, of which this kernel ~140.
+// tile, stamped before PV's sums were a tile's own): the three phases'
+// latencies, 7200 against the 3072 its 192 products of 32 cycles a SIMD take.
+// Scores 3000 and PV 2300 (each 1536 of products, then the barrier, the first
+// LDS reads and the stores of the shares), the softmax with the next K copies
+// 1900.  The copies go out between products and softmax steps: in a row they
+// held each wave ~500 cycles.  The step: 1468 us with each query row streamed by
+// the vector-ALU kernel (prefill_rows), 196 us here; of the kernel trace's 215
+// this kernel 159, the RoPE/append 33, the merge of the key splits 16, the
+// split 7.
 #include <hip/hip_runtime.h>
 
 #include "device_util.hpp"
